@@ -4,7 +4,7 @@
 //                  block per (64-position chunk, KV head, token): all of K streams in parallel.
 //   k_attn_av      softmax over the scores (e = exp(s - max) in f64, stored f32; p = f32(e * (1/sum e))), then
 //                  out_i = sum_t p_t V_t,i accumulated in f32 in position order, one block per (32-dim slice, query
-//                  head, token); the head output is also quantised for the output projection.
+//                  head, token, chunk of 2048 positions); the head output is also quantised for the output projection.
 // Scores live in a [token][head][ctx] f32 buffer between the two. The weighted sum keeps the reference's f32 rounding
 // after every position: a random-weight network turns a 1e-7 change there into a visible logit difference.
 #include "zl_kernels.h"
@@ -420,40 +420,145 @@ __global__ __launch_bounds__(NWV * 64) void k_attn_scores_mm(const AttnArgs a, i
 size_t attention_mm_lds(int hd) { return (size_t)MM_PT * (hd + 2) * 8; }
 
 
-// One block per (32-dim slice, query head, token). The slice's V rows (dimension-major in the cache) are staged
-// through LDS in chunks of ROWB bytes per dimension (1024: 512 f16 or 256 f32 positions, at long contexts where the
-// softmax row leaves room; else 512), double buffered, the first chunk during the softmax; fewer chunks, fewer barriers in the
-// chain. The
-// chain runs on lanes 0-31 of wave 0, one output dimension each, reading 16 bytes of consecutive positions at a time.
+constexpr double LN2_HI = 2977044472.0 / 4294967296.0;     // ln 2 to 32 fractional bits (n LN2_HI is exact)
+constexpr double LN2_LO = -4.2009150726810846e-11;          // ln 2 - LN2_HI
+
+// exp of x <= 0 in f64 (NaN and -inf included): x = n ln 2 + r with |r| <= ln 2 / 2 (ln 2 in two parts, n exact), the
+// Taylor polynomial of degree 13 in Horner form (remainder r^14 / 14! < 5e-18), scaled by 2^n. Within an ulp of the
+// exact value. 21 VALU instructions where the device library's exp, which serves every argument, takes about 45: the
+// softmax of a 12K-position prefill row is bound by them.
+__device__ __forceinline__ double exp_neg(double x) {
+  const double y = x < -1000.0 ? -1000.0 : x;  // (2^n underflows to 0 long before; a NaN stays one)
+  const double n = rint(y * 1.4426950408889634);
+  double r = fma(n, -LN2_HI, y);
+  r = fma(n, -LN2_LO, r);
+  double p = 1.0 / 6227020800.0;
+  p = fma(p, r, 1.0 / 479001600.0);
+  p = fma(p, r, 1.0 / 39916800.0);
+  p = fma(p, r, 1.0 / 3628800.0);
+  p = fma(p, r, 1.0 / 362880.0);
+  p = fma(p, r, 1.0 / 40320.0);
+  p = fma(p, r, 1.0 / 5040.0);
+  p = fma(p, r, 1.0 / 720.0);
+  p = fma(p, r, 1.0 / 120.0);
+  p = fma(p, r, 1.0 / 24.0);
+  p = fma(p, r, 1.0 / 6.0);
+  p = fma(p, r, 0.5);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return ldexp(p, (int)n);
+}
+
+// ---- chunks of a row. A row of positions 0 .. pos is cut into chunks of ATTN_CHUNK positions. Each chunk is a softmax
+// and a weighted sum of its own, with the reference's arithmetic (src/compute/ref-kernels.js:313-320,
+// src/model/forward.js:131-134): m_c = the chunk's largest score, e_t = exp(s_t - m_c) (f64), l_c = their sum,
+// p_t = f32(f32(e_t) * (1 / l_c)), o_c = the f32 chain of p_t V_t over the chunk's positions in order. A row of one
+// chunk is the reference's row bit for bit. A longer row's chunks are joined in f64 in chunk order,
+//   out = f32(sum_c w_c o_c / sum_c w_c),  w_c = exp(m_c - max m) l_c,
+// so its chains run side by side instead of one dependent step per position over the whole row: a 16K-position head
+// took 16,384 steps of ~4 ns on one wave. Chunks start at multiples of ATTN_CHUNK, so the order is a function of the
+// position alone and a token gets the same bits in a pass of any size. Against float64 the joined chunks are closer than
+// the single f32 chain, whose rounding errors grow with its length.
+//
+// A chunk of a longer row leaves a record [m_c, l_c (lane chains), o_c of 32 dimensions] in a.rec ([token][head][32-dimension slice]
+// [chunk]); the block that arrives last at the counter of its (token, head, slice) or row block joins them. The hand-off
+// is that of the GEMV's K parts: device-coherent stores, complete (vmcnt(0)) before the relaxed arrival, device-coherent
+// loads by the last.
+constexpr int REC_D = ATTN_REC_DOUBLES;
+__device__ __forceinline__ double *chunk_rec(const AttnArgs &a, int b, int h, int slice, int c) {
+  return a.rec + ((((long)b * a.nHead + h) * (a.hd >> 5) + slice) * a.nchunk + c) * REC_D;
+}
+// o of dimension `lane` on 32 consecutive lanes, m and l the same on all of them
+__device__ __forceinline__ void chunk_store(double *r, int lane, double m, double l, float o) {
+  __hip_atomic_store((float *)(r + 2) + lane, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (lane < 2) __hip_atomic_store(r + lane, lane == 0 ? m : l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The joined outputs of dimension `lane` (32 consecutive lanes) of NS neighbouring slices of n chunks' records at r
+// (slices lds apart); ml(c) gives chunk c's (m, l). A chunk whose scores are all -inf counts for nothing beside one that
+// has a finite score (the reference's e of such a position is 0).
+template <int NS, typename ML>
+__device__ __forceinline__ void chunk_join(const double *r, long lds, int n, int lane, const ML &ml, float (&out)[NS]) {
+  constexpr int NJ = NS > 1 ? 4 : 8;  // chunks whose loads are issued together
+  float M = -INFINITY;
+  for (int c = lane; c < n; c += 32) M = fmaxf(M, (float)ml(c).x);
+  M = group_fmax(M, 32);
+  double L = 0.0, O[NS];
+  #pragma unroll
+  for (int i = 0; i < NS; i++) O[i] = 0.0;
+  for (int c0 = 0; c0 < n; c0 += 32) {
+    const int nc = min(32, n - c0);
+    const double2 v = ml(min(c0 + lane, n - 1));
+    const double w = v.x == -INFINITY && M != -INFINITY ? 0.0 : exp(v.x - (double)M) * v.y;
+    for (int j0 = 0; j0 < nc; j0 += NJ) {
+      float o[NS][NJ];
+      #pragma unroll
+      for (int i = 0; i < NS; i++)
+        #pragma unroll
+        for (int j = 0; j < NJ; j++)
+          o[i][j] = __hip_atomic_load((const float *)(r + i * lds + (long)(c0 + min(j0 + j, nc - 1)) * REC_D + 2) + lane,
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      #pragma unroll
+      for (int j = 0; j < NJ; j++) {
+        const double wj = __shfl(w, min(j0 + j, nc - 1), 32);
+        if (j0 + j < nc && wj != 0.0) {
+          L += wj;
+          #pragma unroll
+          for (int i = 0; i < NS; i++) O[i] = fma(wj, (double)o[i][j], O[i]);
+        }
+      }
+    }
+  }
+  #pragma unroll
+  for (int i = 0; i < NS; i++) out[i] = (float)(O[i] / L);
+}
+
+// The head output of 32 dimensions on 32 consecutive lanes: the output gate when there is one
+// (src/model/forward-qwen35.js:103: o * sigmoid(gate), f64, stored f32), the f32 row, its quantisation.
+__device__ __forceinline__ void attn_emit(const AttnArgs &a, int b, int h, int dim, float o) {
+  const int col = h * a.hd + dim;
+  if (a.gate) {
+    const double g = (double)a.gate[(long)b * a.ldq + (long)h * a.qhs + dim];
+    o = (float)((double)o * (1.0 / (1.0 + exp(-g))));
+  }
+  if (a.out) a.out[(long)b * a.ldo + col] = o;
+  if (a.act.q) quant_block32(o, col, a.act, b);  // (unset: the output GEMV quantises the f32 rows itself)
+}
+
+// One block per (32-dim slice, query head, token, chunk). The slice's V rows (dimension-major in the cache) are staged
+// through LDS in pieces of AV_ROW bytes per dimension, double buffered, the first one during the softmax. The chain runs
+// on lanes 0-31 of wave 0, one output dimension each, reading 16 bytes of consecutive positions at a time. Bound by the
+// dependent fma of the chain (~4 ns per position, at most ATTN_CHUNK of them); three blocks fit a CU's LDS.
 constexpr int AV_DIMS = 32;       // output dimensions per block
-constexpr int AV_ROW = 512;       // bytes of one dimension's positions per chunk (the smaller chunk)
-constexpr int AV_ROW_BIG = 1024;  // the larger chunk
+constexpr int AV_ROW = 512;       // bytes of one dimension's positions per staged piece
 constexpr int AV_PITCH = AV_ROW + 16;   // LDS row pitch (the pad spreads the chain's rows over the banks)
-constexpr int AV_CHUNK = AV_DIMS * AV_PITCH;
+constexpr int AV_STAGE = AV_DIMS * AV_PITCH;
 constexpr int AV_UNIT = 32;       // positions per unrolled step of the weighted sum
 
-template <bool F16KV, int ROWB>
+// NSC: scores per thread (256 NSC >= the positions of a chunk), held in registers from the load to the probabilities
+template <bool F16KV, int NSC>
 __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
   extern __shared__ __align__(16) uint8_t lds[];
-  constexpr int PITCH = ROWB + 16, CHUNKB = AV_DIMS * PITCH;  // LDS row pitch and bytes of one staged chunk
   constexpr int VB = F16KV ? 2 : 4;
-  constexpr int CT = ROWB / VB;        // positions per chunk
-  constexpr int EPP = 16 / VB;           // positions per 16-byte piece
-  constexpr int PPR = ROWB / 16;       // pieces per row
-  constexpr int LPT = AV_DIMS * PPR / 256;   // 16-byte loads per thread per chunk
-  const int slice = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  constexpr int CT = AV_ROW / VB;        // positions per staged piece
+  constexpr int EPP = 16 / VB;           // positions per 16-byte load
+  constexpr int PPR = AV_ROW / 16;       // loads per row
+  constexpr int LPT = AV_DIMS * PPR / 256;   // 16-byte loads per thread per staged piece
+  constexpr int NP = 256 * NSC;          // positions per block at most
+  const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int stB = a.step->B, stPos0 = a.step->pos0;  // the pass's step record (scalar loads, read before the pins)
   pin_args(a.hd, a.nHead, a.nHeadKv, a.layer, a.vstride, a.vcache, a.scores, a.sld, a.ctx);
-  const int hd = a.hd, kvh = h / (a.nHead / a.nHeadKv);
-  float *p = (float *)lds;                                // [ctx rounded up to AV_UNIT] probabilities
-  uint8_t *vbuf = lds + (size_t)((a.ctx + AV_UNIT - 1) / AV_UNIT * AV_UNIT) * 4;  // [2][AV_DIMS][PITCH] staged V rows
+  const int hd = a.hd, kvh = h / (a.nHead / a.nHeadKv), NS = hd / AV_DIMS;
+  const int slice = blockIdx.x % NS, chunk = blockIdx.x / NS;
+  const int t00 = chunk * ATTN_CHUNK, ctxc = a.ctx - t00;  // the chunk's first position, cache positions from there on
+  float *p = (float *)lds;               // [NP] probabilities
+  uint8_t *vbuf = lds + NP * 4;          // [2][AV_DIMS][AV_PITCH] staged V rows
   __shared__ double redd[4];
   __shared__ float redf[4];
-  const uint8_t *vbase = (const uint8_t *)a.vcache + (((long)a.layer * a.nHeadKv + kvh) * hd + (long)slice * AV_DIMS) * a.vstride * VB;
+  const uint8_t *vbase =
+      (const uint8_t *)a.vcache + ((((long)a.layer * a.nHeadKv + kvh) * hd + (long)slice * AV_DIMS) * a.vstride + t00) * VB;
   uint4 pre[LPT];
-  int npos = 0;
-  // V pieces of chunk c below `lim` positions (inside the cache row); the first chunk and the first 1024 scores are
-  // requested before the pass's step record arrives, and the pieces at or past the last position are zeroed after it
+  // V of piece c below `lim` positions (inside the cache row); the first piece and the scores are requested before the
+  // pass's step record arrives, and what lies at or past the last position is zeroed after it
   auto fetch = [&](int c, int lim) {
     #pragma unroll
     for (int k = 0; k < LPT; k++) {
@@ -465,65 +570,62 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
     #pragma unroll
     for (int k = 0; k < LPT; k++) {
       const int idx = k * 256 + tid;
-      *(uint4 *)(vbuf + buf * CHUNKB + (idx / PPR) * PITCH + (idx % PPR) * 16) = pre[k];
+      *(uint4 *)(vbuf + buf * AV_STAGE + (idx / PPR) * AV_PITCH + (idx % PPR) * 16) = pre[k];
     }
   };
-  // the first 1024 scores, then the first V chunk: loads complete in order, so the softmax below waits for the scores
-  // alone while the V chunk is on its way
-  const float *srow = a.scores + ((long)b * a.nHead + h) * a.sld;
-  float v0[4];
+  // the scores, then the first V piece: loads complete in order, so the softmax below waits for the scores alone while V
+  // is on its way
+  const float *srow = a.scores + ((long)b * a.nHead + h) * a.sld + t00;
+  float v[NSC];
   #pragma unroll
-  for (int k = 0; k < 4; k++) { const int t = k * 256 + tid; v0[k] = srow[t < a.ctx ? t : 0]; }  // (t >= npos: unused)
+  for (int k = 0; k < NSC; k++) { const int t = k * 256 + tid; v[k] = srow[t < ctxc ? t : 0]; }  // (t >= npos: unused)
   __builtin_amdgcn_sched_barrier(0);
   #pragma unroll
-  for (int k = 0; k < LPT; k++) {  // unconditional loads (pieces past the cache's positions read position 0, zeroed
-                                   // below with every piece at or past the last position): a load under a branch
-                                   // would make the first use of the scores wait for it too
+  for (int k = 0; k < LPT; k++) {  // unconditional loads (what lies past the cache's positions reads position 0, zeroed
+                                   // below with all at or past the last position): a load under a branch would make
+                                   // the first use of the scores wait for it too
     const int idx = k * 256 + tid, dim = idx / PPR, t = (idx % PPR) * EPP;
-    pre[k] = *(const uint4 *)(vbase + ((long)dim * a.vstride + (t < a.ctx ? t : 0)) * VB);
+    pre[k] = *(const uint4 *)(vbase + ((long)dim * a.vstride + (t < ctxc ? t : 0)) * VB);
   }
   __builtin_amdgcn_sched_barrier(0);
   if (b >= stB) return;
-  npos = stPos0 + b + 1;
+  const int nrow = stPos0 + b + 1, npos = min(nrow - t00, ATTN_CHUNK);  // the row's positions, the chunk's
+  if (npos <= 0) return;
   const int nch = (npos + CT - 1) / CT;
-  // ---- softmax (src/compute/ref-kernels.js:313-320)
+  // ---- softmax (src/compute/ref-kernels.js:313-320): thread tid holds t = tid + 256 k, its exponentials added in k order
   float mx = -INFINITY;
   #pragma unroll
-  for (int k = 0; k < 4; k++) { const int t = k * 256 + tid; if (t < npos) p[t] = v0[k]; else v0[k] = -INFINITY; mx = fmaxf(mx, v0[k]); }
-  for (int t0 = 1024; t0 < npos; t0 += 16 * 256) {  // 16 loads per thread in flight at a time
-    float v[16];
-    #pragma unroll
-    for (int k = 0; k < 16; k++) { const int t = t0 + k * 256 + tid; v[k] = srow[t < npos ? t : 0]; }
-    #pragma unroll
-    for (int k = 0; k < 16; k++) { const int t = t0 + k * 256 + tid; if (t < npos) { p[t] = v[k]; mx = fmaxf(mx, v[k]); } }
-  }
+  for (int k = 0; k < NSC; k++) { v[k] = k * 256 + tid < npos ? v[k] : -INFINITY; mx = fmaxf(mx, v[k]); }
   mx = group_fmax(mx, 64);
   if (lane == 0) redf[wave] = mx;
   __syncthreads();
   const double m = (double)fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
-  // four independent exponentials per step (their f64 chains overlap), added to the sum in position order as before
   double sum = 0.0;
-  for (int t0 = tid; t0 < npos; t0 += 4 * 256) {
-    double e[4];
-    #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const int t = t0 + 256 * k;
-      e[k] = exp((double)p[t < npos ? t : t0] - m);
-    }
-    #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const int t = t0 + 256 * k;
-      if (t < npos) { p[t] = (float)e[k]; sum += e[k]; }
+  #pragma unroll
+  for (int k0 = 0; k0 < NSC; k0 += 4) {
+    if (k0 * 256 < npos) {  // (uniform)
+      double e[4];  // four independent chains
+      #pragma unroll
+      for (int k = 0; k < 4; k++) e[k] = exp_neg((double)v[k0 + k] - m);
+      #pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const bool on = (k0 + k) * 256 + tid < npos;
+        if (on) sum += e[k];
+        v[k0 + k] = on ? (float)e[k] : 0.f;
+      }
     }
   }
   sum = wave_sum_xor(sum, 64);
   if (lane == 0) redd[wave] = sum;
   __syncthreads();
-  const double inv = 1.0 / ((redd[0] + redd[1]) + (redd[2] + redd[3]));
-  for (int t = tid; t < npos; t += 256) p[t] = (float)((double)p[t] * inv);
-  for (int t = npos + tid; t < (npos + AV_UNIT - 1) / AV_UNIT * AV_UNIT; t += 256) p[t] = 0.f;
+  const double l = (redd[0] + redd[1]) + (redd[2] + redd[3]), inv = 1.0 / l;
   #pragma unroll
-  for (int k = 0; k < LPT; k++) {  // the first chunk's pieces from the last position on: zeros, as in later chunks
+  for (int k = 0; k < NSC; k++) {  // (zeros from the last position to the end of its unit, at least)
+    const int t = k * 256 + tid;
+    if (k * 256 < npos) p[t] = t < npos ? (float)((double)v[k] * inv) : 0.f;
+  }
+  #pragma unroll
+  for (int k = 0; k < LPT; k++) {  // the first piece from the last position on: zeros, as in later ones
     const int t = ((k * 256 + tid) % PPR) * EPP;
     if (t >= npos) pre[k] = make_uint4(0, 0, 0, 0);
     else if (t + EPP > npos) {
@@ -550,7 +652,7 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
       // p is zero past the last position, so a unit may run past `cnt`: fmaf(0, v, o) == o for the finite cached
       // values read there. The read-ahead index is clamped to the chunk's last unit (a re-read, never past it).
       const int t0 = c * CT, cnt = min(CT, npos - t0), nu = (cnt + AV_UNIT - 1) / AV_UNIT;
-      const uint8_t *row = vbuf + (c & 1) * CHUNKB + lane * PITCH;
+      const uint8_t *row = vbuf + (c & 1) * AV_STAGE + lane * AV_PITCH;
       const float *pc = p + t0;
       float4 pa[AV_UNIT / 4], pb[AV_UNIT / 4];
       uint4 va[AV_UNIT * VB / 16], vb[AV_UNIT * VB / 16];
@@ -594,956 +696,313 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
     if (c + 1 < nch) store((c + 1) & 1);
     __syncthreads();
   }
-  if (chainLane) {
-    const int col = h * hd + slice * AV_DIMS + lane;
-    if (a.gate) {  // gated attention output (src/model/forward-qwen35.js:103): o * sigmoid(gate), f64, stored f32
-      const double g = (double)a.gate[(long)b * a.ldq + (long)h * a.qhs + slice * AV_DIMS + lane];
-      o = (float)((double)o * (1.0 / (1.0 + exp(-g))));
-    }
-    if (a.out) a.out[(long)b * a.ldo + col] = o;
-    if (a.act.q) quant_block32(o, col, a.act, b);  // (unset: the output GEMV quantises the f32 rows itself)
-  }
-}
-
-// ---- k_attn_av's weighted sum with the chains on the matrix cores: v_mfma_f32_16x16x4_f32 is four sequential fmaf in k
-// order (measured), so a chain of MFMAs whose A operand holds the row's probabilities in row 0 (rows 1-15 zero) and
-// whose B operand holds V of 16 dimensions computes the position-order f32 chain of every dimension bit for bit. A
-// dependent MFMA issues every 32 cycles (8 per position, where a dependent v_fma_mix_f32 takes 9) only while the wave
-// issues nothing else but LDS reads between them (a VALU instruction there costs ~12 cycles: measured), so V is staged
-// in LDS already converted to f32 and the chain waves only read and multiply.
-// One block per (32-dim slice, query head, token), as k_attn_av: the same softmax (the same max, the exponentials
-// summed in the same thread order, p = f32(f32(e) * inv)); then waves 0-1 run the chains of dimensions 16 w .. 16 w + 15
-// of chunk c while waves 2-3 stage chunk c + 1 (V as f32, and its probabilities, whose exponentials they compute again
-// from the scores: the same bits) and request chunk c + 2. One barrier per chunk; LDS does not grow with the context.
-// LDS holds V and the probabilities by position mod 4 (section k holds positions 4 m + k, m ascending), so the 16
-// lanes of MFMA k-group g read their own positions contiguously, 4 MFMAs' operands per 16-byte read.
-constexpr int AVM_CT = 512;                 // positions per chunk
-template <bool B> struct Whole { static constexpr bool value = B; };  // a chunk below every row's last position
-constexpr int AVM_SF = AVM_CT / 4 + 4;      // floats of one position section (16-byte pad)
-constexpr int AVM_RS = 4 * AVM_SF + 4;      // floats of one dimension row (4 x an odd number: the 16 lanes of a chain
-                                            // read, rows n16 = 0..15, fall on 64 distinct banks)
-constexpr int AVM_UNIT = 32;                // positions per pipelined step of a chain (8 MFMAs)
-constexpr int AVM_NK = 72;                  // scores per thread the softmax keeps in registers
-constexpr int AVM_MAX_CTX = AVM_NK * 256;   // contexts this form takes (18432 positions)
-size_t attention_av_mfma_lds() { return ((size_t)2 * AV_DIMS * AVM_RS + (2 * 4 + 1) * AVM_SF) * 4; }
-
-template <bool F16KV>
-__global__ __launch_bounds__(256) void k_attn_av_mfma(const AttnArgs a) {
-  extern __shared__ __align__(16) uint8_t lds[];
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  constexpr int VB = F16KV ? 2 : 4;
-  constexpr int CT = AVM_CT, SF = AVM_SF, RS = AVM_RS;
-  constexpr int EPP = 16 / VB;                      // positions per 16-byte piece
-  constexpr int PPR = CT / EPP;                     // pieces per dimension row of a chunk
-  constexpr int PLT = AV_DIMS * PPR / 128;          // pieces per producer thread per chunk (16 f16, 32 f32)
-  constexpr int SPT = CT / 128;                     // probabilities per producer thread per chunk
-  constexpr int NU = CT / AVM_UNIT;                 // units per chunk
-  float *vk = (float *)lds;                         // [2][AV_DIMS][RS]: V of position 4 m + k, dimension j at j RS + k SF + m
-  float *pk = vk + 2 * AV_DIMS * RS;                // [2][4][SF]: p of position 4 m + k at [k][m]
-  float *zb = pk + 2 * 4 * SF;                      // [SF] zeros: the A operand of rows 1-15
-  __shared__ double redd[4];
-  __shared__ float redf[4];
-  __shared__ float ot[AV_DIMS];
-  const int slice = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int n16 = lane & 15, g = lane >> 4;
-  const int hd = a.hd, kvh = h / (a.nHead / a.nHeadKv);
-  const uint8_t *vbase = (const uint8_t *)a.vcache + (((long)a.layer * a.nHeadKv + kvh) * hd + (long)slice * AV_DIMS) * a.vstride * VB;
-  const float *srow = a.scores + ((long)b * a.nHead + h) * a.sld;
-  const bool producer = wave >= 2;
-  const int pt = tid - 128;                         // producer thread 0..127
-  uint4 pre[PLT];
-  float sp[SPT];
-  int npos = 0;
-  double m = 0.0, inv = 0.0;
-  // chunk c's V pieces and scores, from in-range rows and positions (what lies past the last position is zeroed when
-  // the chunk is staged)
-  auto fetch_v = [&](int c, int lim) {
-    #pragma unroll
-    for (int k = 0; k < PLT; k++) {
-      const int idx = k * 128 + pt, dim = idx / PPR, t = c * CT + (idx % PPR) * EPP;
-      pre[k] = *(const uint4 *)(vbase + ((long)dim * a.vstride + (t < lim ? t : 0)) * VB);
-    }
-  };
-  auto fetch_s = [&](int c, int lim) {
-    #pragma unroll
-    for (int i = 0; i < SPT; i++) {
-      const int t = c * CT + i * 128 + pt;
-      sp[i] = srow[t < lim ? t : 0];
-    }
-  };
-  // producers: chunk c into slot c & 1: V as f32 (zeros past the last position) ...
-  auto stage_v = [&](int c) {
-    float *vs = vk + (c & 1) * AV_DIMS * RS;
-    #pragma unroll
-    for (int k = 0; k < PLT; k++) {
-      const int idx = k * 128 + pt, dim = idx / PPR, pc = idx % PPR, t = c * CT + pc * EPP;
-      const uint32_t w[4] = {pre[k].x, pre[k].y, pre[k].z, pre[k].w};
-      float f[EPP];
-      #pragma unroll
-      for (int e = 0; e < EPP; e++) {
-        const float x = F16KV ? h2f((uint16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffff))) : __uint_as_float(w[e]);
-        f[e] = t + e < npos ? x : 0.f;
-      }
-      float *drow = vs + dim * RS;
-      #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        if (F16KV) *(float2 *)(drow + q * SF + 2 * pc) = make_float2(f[q], f[q + 4]);  // positions t + q, t + 4 + q
-        else drow[q * SF + pc] = f[q];                                                 // position t + q
-      }
-    }
-  };
-  // ... and its probabilities p = f32(f32(e) * inv) (zeros past the last position)
-  auto stage_p = [&](int c) {
-    float *ps = pk + (c & 1) * 4 * SF;
-    #pragma unroll
-    for (int i = 0; i < SPT; i++) {
-      const int tl = i * 128 + pt, t = c * CT + tl;
-      const double e = exp((double)sp[i] - m);
-      ps[(tl & 3) * SF + (tl >> 2)] = t < npos ? (float)((double)(float)e * inv) : 0.f;
-    }
-  };
-  if (producer) {
-    fetch_v(0, a.ctx);
-    fetch_s(0, a.ctx);
-  }
-  // ---- softmax (src/compute/ref-kernels.js:313-320), k_attn_av's arithmetic: thread tid takes t = tid + 256 k, its
-  // exponentials added in k order. The scores stay in registers (-inf past the last position: exp gives +0, which
-  // leaves the sum unchanged), so the producers stage chunk 0's V meanwhile; they are requested before the pass's step
-  // record arrives (up to the cache's capacity).
-  const Step *st = a.step;
-  const int sB = st->B, sp0 = st->pos0;
-  float sv[AVM_NK];
-  #pragma unroll
-  for (int k = 0; k < AVM_NK; k++) { const int t = k * 256 + tid; sv[k] = srow[t < a.ctx ? t : 0]; }
-  __asm__ volatile("" ::: "memory");  // keeps the loads above the branch (it would otherwise sink them past it)
-  if (b >= sB) return;
-  npos = sp0 + b + 1;
-  const int nch = (npos + CT - 1) / CT;
-  const int nend = (npos + AVM_UNIT - 1) / AVM_UNIT * AVM_UNIT;  // positions the chains run
-  if (producer) {
-    stage_v(0);
-    if (nch > 1) fetch_v(1, npos);
-  }
-  #pragma unroll
-  for (int k = 0; k < AVM_NK; k++) sv[k] = k * 256 + tid < npos ? sv[k] : -INFINITY;
-  float mx = -INFINITY;
-  #pragma unroll
-  for (int k = 0; k < AVM_NK; k++) mx = fmaxf(mx, sv[k]);
-  mx = group_fmax(mx, 64);
-  if (lane == 0) redf[wave] = mx;
-  __syncthreads();
-  m = (double)fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
-  double sum = 0.0;
-  #pragma unroll
-  for (int k0 = 0; k0 < AVM_NK; k0 += 8) {
-    if (k0 * 256 < npos) {  // (uniform)
-      double e[8];
-      #pragma unroll
-      for (int k = 0; k < 8; k++) e[k] = exp((double)sv[k0 + k] - m);
-      #pragma unroll
-      for (int k = 0; k < 8; k++) sum += e[k];
-    }
-  }
-  sum = wave_sum_xor(sum, 64);
-  if (lane == 0) redd[wave] = sum;
-  __syncthreads();
-  inv = 1.0 / ((redd[0] + redd[1]) + (redd[2] + redd[3]));
-  if (producer) {
-    stage_p(0);
-    if (nch > 1) fetch_s(1, npos);
-  }
-  for (int i = tid; i < SF; i += 256) zb[i] = 0.f;
-  __syncthreads();
-  // ---- chains (waves 0-1) / staging (waves 2-3)
-  f4 acc = {0.f, 0.f, 0.f, 0.f};
-  auto mfma8 = [&](const f4 &p0, const f4 &p1, const f4 &v0, const f4 &v1) {
-    #pragma unroll
-    for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[i], v0[i], acc, 0, 0, 0);
-    #pragma unroll
-    for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[i], v1[i], acc, 0, 0, 0);
-  };
-  // the producers and the chain waves run loops of their own with one barrier per chunk each (the same count), so the
-  // chains' accumulator stays in the matrix cores' registers from chunk to chunk
-  if (producer) {
-    for (int c = 0; c < nch; c++) {
-      if (c + 1 < nch) {
-        stage_v(c + 1);
-        stage_p(c + 1);
-        if (c + 2 < nch) {
-          fetch_v(c + 2, npos);
-          fetch_s(c + 2, npos);
-        }
-      }
-      __syncthreads();
-    }
-  } else {
-    // unit u: the 8 MFMAs of positions c CT + 32 u .. + 31; lane group g supplies positions 4 m + g, m = 8 u .. 8 u + 7
-    // (A: lanes of row 0 read the probabilities, the others the zeros). Units two at a time on two operand sets, the
-    // next unit's reads ahead of the current unit's MFMAs; a full chunk in straight-line code (constant offsets). The
-    // whole chunks run in a loop of their own, so the accumulator keeps one register assignment there.
-    auto chunk = [&](int c, auto whole) __attribute__((always_inline)) {
-      const float *vr = vk + ((c & 1) * AV_DIMS + wave * 16 + n16) * RS + g * SF;
-      const float *pr = n16 == 0 ? pk + ((c & 1) * 4 + g) * SF : zb;
-      auto ld = [&](const float *q, int off) { return *(const f4 *)(q + off); };
-      if constexpr (decltype(whole)::value) {
-        f4 a0 = ld(pr, 0), a1 = ld(pr, 4), a2 = ld(vr, 0), a3 = ld(vr, 4);
-        #pragma unroll
-        for (int u = 0; u < NU; u += 2) {
-          const f4 b0 = ld(pr, 8 * u + 8), b1 = ld(pr, 8 * u + 12), b2 = ld(vr, 8 * u + 8), b3 = ld(vr, 8 * u + 12);
-          __builtin_amdgcn_sched_barrier(0);
-          mfma8(a0, a1, a2, a3);
-          if (u + 2 < NU) { a0 = ld(pr, 8 * u + 16); a1 = ld(pr, 8 * u + 20); a2 = ld(vr, 8 * u + 16); a3 = ld(vr, 8 * u + 20); }
-          __builtin_amdgcn_sched_barrier(0);
-          mfma8(b0, b1, b2, b3);
-        }
-      } else {
-        const int nu = (nend - c * CT) / AVM_UNIT;
-        f4 a0 = ld(pr, 0), a1 = ld(pr, 4), a2 = ld(vr, 0), a3 = ld(vr, 4);
-        int u = 0;
-        for (; u + 2 <= nu; u += 2) {
-          const f4 b0 = ld(pr, 8 * u + 8), b1 = ld(pr, 8 * u + 12), b2 = ld(vr, 8 * u + 8), b3 = ld(vr, 8 * u + 12);
-          __builtin_amdgcn_sched_barrier(0);
-          mfma8(a0, a1, a2, a3);
-          const int un = min(u + 2, nu - 1);  // (a re-read of the last unit when past it)
-          a0 = ld(pr, 8 * un); a1 = ld(pr, 8 * un + 4); a2 = ld(vr, 8 * un); a3 = ld(vr, 8 * un + 4);
-          __builtin_amdgcn_sched_barrier(0);
-          mfma8(b0, b1, b2, b3);
-        }
-        if (u < nu) mfma8(a0, a1, a2, a3);
-      }
-      __syncthreads();
-    };
-    const int nwhole = min(nch, nend / CT);
-    int c = 0;
-    for (; c < nwhole; c++) chunk(c, Whole<true>{});
-    for (; c < nch; c++) chunk(c, Whole<false>{});
-  }
-  // ---- epilogue: row 0's outputs (element 0 of lanes 0-15 of each chain wave) to lanes 0-31 of wave 0
-  if (!producer && g == 0) ot[wave * 16 + n16] = acc[0];
-  __syncthreads();
-  if (wave == 0 && lane < AV_DIMS) {
-    const int col = h * hd + slice * AV_DIMS + lane;
-    float o = ot[lane];
-    if (a.gate) {  // gated attention output (src/model/forward-qwen35.js:103): o * sigmoid(gate), f64, stored f32
-      const double gv = (double)a.gate[(long)b * a.ldq + (long)h * a.qhs + slice * AV_DIMS + lane];
-      o = (float)((double)o * (1.0 / (1.0 + exp(-gv))));
-    }
-    if (a.out) a.out[(long)b * a.ldo + col] = o;
-    if (a.act.q) quant_block32(o, col, a.act, b);  // (unset: the output GEMV quantises the f32 rows itself)
-  }
-}
-
-// ---- the same weighted sum for long contexts, one block per (query head, token) over all HD dimensions. k_attn_av keeps
-// the block's softmax row in LDS, which at 16K positions leaves room for one block per CU, and its four slice blocks of
-// a head hold four copies. Here the exponentials are written back over the head's scores (one block per row, so no
-// other block reads them), and the probabilities p = f32(e * inv) are staged chunk by chunk with V: LDS no longer grows
-// with the context, and a head's four slices share one softmax. The arithmetic is k_attn_av's (the same max, the same
-// exponentials summed in the same thread order, the same chain per dimension), so the two give the same bits.
-constexpr int AVH_CTX = 8192;  // contexts above this take the per-head form (HD <= 128)
-
-template <int HD, bool F16KV>
-__global__ __launch_bounds__(256) void k_attn_av_head(const AttnArgs a) {
-  extern __shared__ __align__(16) uint8_t lds[];
-  constexpr int VB = F16KV ? 2 : 4;
-  constexpr int CT = AV_ROW / VB;          // positions per chunk
-  constexpr int EPP = 16 / VB;             // positions per 16-byte piece
-  constexpr int PPR = AV_ROW / 16;         // pieces per row
-  constexpr int CHUNK = HD * AV_PITCH;     // bytes of one staged chunk of V rows
-  constexpr int LPT = HD * PPR / 256;      // pieces per thread per chunk
-  constexpr int PPT = CT / 256 > 0 ? CT / 256 : 1;  // probabilities per thread per chunk
-  static_assert(HD * PPR % 256 == 0 && CT % 256 == 0 || CT == 128, "chunk geometry");
-  float *pb = (float *)(lds + 2 * CHUNK);  // [2][CT] staged probabilities
-  __shared__ double redd[4];
-  __shared__ float redf[4];
-  const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int kvh = h / (a.nHead / a.nHeadKv);
-  const uint8_t *vbase = (const uint8_t *)a.vcache + ((long)a.layer * a.nHeadKv + kvh) * HD * a.vstride * VB;
-  float *srow = a.scores + ((long)b * a.nHead + h) * a.sld;
-  uint4 pre[LPT];
-  float pp[PPT];
-  auto fetch = [&](int c, int lim) {
-    #pragma unroll
-    for (int k = 0; k < LPT; k++) {
-      const int idx = k * 256 + tid, dim = idx / PPR, t = c * CT + (idx % PPR) * EPP;
-      pre[k] = t < lim ? *(const uint4 *)(vbase + ((long)dim * a.vstride + t) * VB) : make_uint4(0, 0, 0, 0);
-    }
-  };
-  auto store = [&](int buf) {
-    #pragma unroll
-    for (int k = 0; k < LPT; k++) {
-      const int idx = k * 256 + tid;
-      *(uint4 *)(lds + buf * CHUNK + (idx / PPR) * AV_PITCH + (idx % PPR) * 16) = pre[k];
-    }
-  };
-  fetch(0, a.ctx);
-  const Step *st = a.step;
-  if (b >= st->B) return;
-  const int npos = st->pos0 + b + 1;
-  const int nch = (npos + CT - 1) / CT;
-  #pragma unroll
-  for (int k = 0; k < LPT; k++) {  // the first chunk's pieces from the last position on: zeros, as in later chunks
-    const int t = ((k * 256 + tid) % PPR) * EPP;
-    if (t >= npos) pre[k] = make_uint4(0, 0, 0, 0);
-    else if (t + EPP > npos) {
-      uint32_t w[4] = {pre[k].x, pre[k].y, pre[k].z, pre[k].w};
-      #pragma unroll
-      for (int e = 0; e < EPP; e++)
-        if (t + e >= npos) {
-          if (F16KV) w[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
-          else w[e] = 0u;
-        }
-      pre[k] = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-  }
-  // ---- softmax (src/compute/ref-kernels.js:313-320) in k_attn_av's order; the exponentials replace the scores
-  float mx = -INFINITY;
-  for (int t0 = tid; t0 < npos; t0 += 16 * 256) {  // 16 loads per thread in flight at a time
-    float v[16];
-    #pragma unroll
-    for (int k = 0; k < 16; k++) { const int t = t0 + 256 * k; v[k] = srow[t < npos ? t : t0]; }
-    #pragma unroll
-    for (int k = 0; k < 16; k++) mx = fmaxf(mx, v[k]);  // (a clamped reload repeats a value already counted)
-  }
-  mx = group_fmax(mx, 64);
-  if (lane == 0) redf[wave] = mx;
-  __syncthreads();
-  const double m = (double)fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
-  double sum = 0.0;
-  for (int t0 = tid; t0 < npos; t0 += 16 * 256) {  // positions tid + 256 j added in j order, as k_attn_av does
-    float v[16];
-    #pragma unroll
-    for (int k = 0; k < 16; k++) { const int t = t0 + 256 * k; v[k] = srow[t < npos ? t : t0]; }
-    #pragma unroll
-    for (int q = 0; q < 16; q += 4) {
-      double e[4];
-      #pragma unroll
-      for (int k = 0; k < 4; k++) e[k] = exp((double)v[q + k] - m);
-      #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const int t = t0 + 256 * (q + k);
-        if (t < npos) { srow[t] = (float)e[k]; sum += e[k]; }
-      }
-    }
-  }
-  sum = wave_sum_xor(sum, 64);
-  if (lane == 0) redd[wave] = sum;
-  __syncthreads();  // also orders this block's writes of the exponentials before their reads below
-  const double inv = 1.0 / ((redd[0] + redd[1]) + (redd[2] + redd[3]));
-  // probabilities of chunk c (zero past the last position, as k_attn_av's row)
-  auto pload = [&](int c) {
-    #pragma unroll
-    for (int k = 0; k < PPT; k++) {
-      const int t = c * CT + k * 256 + tid;
-      pp[k] = (k * 256 + tid < CT && t < npos) ? srow[t] : 0.f;
-    }
-  };
-  auto pstore = [&](int buf) {
-    #pragma unroll
-    for (int k = 0; k < PPT; k++)
-      if (k * 256 + tid < CT) pb[buf * CT + k * 256 + tid] = (float)((double)pp[k] * inv);
-  };
-  pload(0);
-  store(0);
-  pstore(0);
-  __syncthreads();
-  // ---- weighted sum: output dimension wave * 64 + lane on the first HD / 64 waves, chunk by chunk (double buffered)
-  const bool chainLane = wave < HD / 64;
-  const int dim = wave * 64 + lane;
-  float o = 0.f;
-  for (int c = 0; c < nch; c++) {
-    if (c + 1 < nch) { fetch(c + 1, npos); pload(c + 1); }
-    if (chainLane) {
-      const int cnt = min(CT, npos - c * CT), nu = (cnt + AV_UNIT - 1) / AV_UNIT;
-      const uint8_t *row = lds + (c & 1) * CHUNK + dim * AV_PITCH;
-      const float *pc = pb + (c & 1) * CT;
-      float4 pa[AV_UNIT / 4], pbv[AV_UNIT / 4];
-      uint4 va[AV_UNIT * VB / 16], vb[AV_UNIT * VB / 16];
-      auto read = [&](int u, float4 (&pv)[AV_UNIT / 4], uint4 (&vv)[AV_UNIT * VB / 16]) {
-        #pragma unroll
-        for (int k = 0; k < AV_UNIT / 4; k++) pv[k] = *(const float4 *)(pc + u * AV_UNIT + 4 * k);
-        #pragma unroll
-        for (int k = 0; k < AV_UNIT * VB / 16; k++) vv[k] = *(const uint4 *)(row + (u * AV_UNIT + k * EPP) * VB);
-      };
-      auto steps = [&](const float4 (&pv)[AV_UNIT / 4], const uint4 (&vv)[AV_UNIT * VB / 16]) {
-        #pragma unroll
-        for (int k = 0; k < AV_UNIT / 4; k++) {
-          float v0, v1, v2, v3;
-          if (F16KV) {
-            const uint4 &w = vv[k >> 1];
-            const uint32_t lo = (k & 1) ? w.z : w.x, hi = (k & 1) ? w.w : w.y;
-            v0 = h2f((uint16_t)(lo & 0xffff)); v1 = h2f((uint16_t)(lo >> 16));
-            v2 = h2f((uint16_t)(hi & 0xffff)); v3 = h2f((uint16_t)(hi >> 16));
-          } else {
-            const uint4 &w = vv[k];
-            v0 = __uint_as_float(w.x); v1 = __uint_as_float(w.y); v2 = __uint_as_float(w.z); v3 = __uint_as_float(w.w);
-          }
-          o = fmaf(pv[k].x, v0, o); o = fmaf(pv[k].y, v1, o); o = fmaf(pv[k].z, v2, o); o = fmaf(pv[k].w, v3, o);
-        }
-      };
-      read(0, pa, va);
-      int u = 0;
-      for (; u + 2 <= nu; u += 2) {
-        read(u + 1, pbv, vb);
-        __builtin_amdgcn_sched_barrier(0);
-        steps(pa, va);
-        read(min(u + 2, nu - 1), pa, va);
-        __builtin_amdgcn_sched_barrier(0);
-        steps(pbv, vb);
-      }
-      if (u < nu) steps(pa, va);
-    }
-    __syncthreads();
-    if (c + 1 < nch) { store((c + 1) & 1); pstore((c + 1) & 1); }
-    __syncthreads();
-  }
-  if (chainLane) {
-    const int col = h * HD + dim;
-    if (a.gate) {  // gated attention output (src/model/forward-qwen35.js:103): o * sigmoid(gate), f64, stored f32
-      const double g = (double)a.gate[(long)b * a.ldq + (long)h * a.qhs + dim];
-      o = (float)((double)o * (1.0 / (1.0 + exp(-g))));
-    }
-    if (a.out) a.out[(long)b * a.ldo + col] = o;
-    if (a.act.q) quant_block32(o, col, a.act, b);  // (unset: the output GEMV quantises the f32 rows itself)
-  }
-}
-
-size_t attention_head_lds(int hd) { return (size_t)2 * hd * AV_PITCH + 2 * 256 * 4; }
-
-// ---- the weighted sum of multi-token passes at long contexts, grouped by KV head. The per-head form above stages its
-// KV head's V once per (query head, token) row: at 16K positions, 4 query heads per KV head and 9 tokens that is 36
-// reads of 4 MB per KV head, 1.2 GB per layer, and the launch runs at the speed of those reads. Here the softmax runs
-// first, one block per row (k_attn_softmax_rows: the per-head form's code; the exponentials replace the scores and
-// 1 / sum goes to pinv), then one block per (32-dimension slice, KV head, group of AVG_ROWS rows) stages each V chunk
-// once for the chains of all its rows: lanes 0-31 of wave w run row 2w's 32 dimensions, lanes 32-63 row 2w + 1's. Every
-// chain is the same position-order f32 chain as in the per-head form, with the same probabilities f32(e * inv); past
-// a row's last position its probabilities are 0 (fmaf(0, v, o) leaves o as it is, V staged there being finite cache
-// values or zeros), so the bits are the per-head form's.
-constexpr int AVG_ROWS = 8;   // rows (query head, token) per block of the grouped weighted sum
-constexpr int AVG_DIMS = 32;  // dimensions per block
-
-constexpr int SMR_T = 512;     // threads of k_attn_softmax_rows
-constexpr int SMR_RP = 4096;   // positions per round of its sum
-constexpr int SMR_NK = 40;     // positions per thread kept in registers (20480 per row)
-template <bool NORM>
-__global__ __launch_bounds__(SMR_T) void k_attn_softmax_rows(const AttnArgs a) {
-  // SMR_T threads: the exponentials on two waves per SIMD. The sum keeps k_attn_av's order (slot s = t mod 256 adds
-  // its positions s, s + 256, ... in order, then the 64-lane butterfly and (w0 + w1) + (w2 + w3)): each round of
-  // SMR_RP positions parks its exponentials in LDS by slot, and the 256 slot threads add them in position order.
-  constexpr int KR = SMR_RP / SMR_T;          // positions per thread per round (8)
-  constexpr int NQ = SMR_NK / KR;             // rounds kept in registers
-  __shared__ double ex[SMR_RP];               // a round's exponentials at [k][s], t = r0 + 256 k + s
-  __shared__ double redd[4];
-  __shared__ float redf[SMR_T / 64];
-  const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const Step *st = a.step;
-  if (b >= st->B) return;
-  const int npos = st->pos0 + b + 1;
-  float *srow = a.scores + ((long)b * a.nHead + h) * a.sld;
-  // thread tid holds positions tid + SMR_T k (a clamped load reads position 0, which leaves the maximum unchanged); the
-  // loads wait for the step record: the rows of a prefill chunk are far shorter than the cache
-  float v[SMR_NK];
-  #pragma unroll
-  for (int k = 0; k < SMR_NK; k++) { const int t = tid + SMR_T * k; v[k] = srow[t < npos ? t : 0]; }
-  float mx = -INFINITY;
-  #pragma unroll
-  for (int k = 0; k < SMR_NK; k++) mx = fmaxf(mx, v[k]);
-  for (int t = SMR_NK * SMR_T + tid; t < npos; t += SMR_T) mx = fmaxf(mx, srow[t]);
-  mx = group_fmax(mx, 64);
-  if (lane == 0) redf[wave] = mx;
-  __syncthreads();
-  float mf = redf[0];
-  #pragma unroll
-  for (int w = 1; w < SMR_T / 64; w++) mf = fmaxf(mf, redf[w]);
-  const double m = (double)mf;
-  // round q: thread tid computes t = q SMR_RP + tid + SMR_T i (slot tid mod 256, k = 2 i + tid / 256)
-  double sum = 0.0;
-  auto slot_add = [&]() {
-    __syncthreads();
-    if (tid < 256) {
-      #pragma unroll
-      for (int k = 0; k < SMR_RP / 256; k++) sum += ex[k * 256 + tid];  // +0 past the last position: no change
-    }
-    __syncthreads();
-  };
-  #pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    if (q * SMR_RP < npos) {  // (uniform)
-      #pragma unroll
-      for (int i = 0; i < KR; i++) {
-        const int k = q * KR + i, t = tid + SMR_T * k;
-        const double e = exp((double)v[k] - m);
-        ex[(2 * i + (tid >> 8)) * 256 + (tid & 255)] = t < npos ? e : 0.0;
-        v[k] = (float)e;
-        if (!NORM && t < npos) srow[t] = v[k];
-      }
-      slot_add();
-    }
-  }
-  for (int r0 = SMR_NK * SMR_T; r0 < npos; r0 += SMR_RP) {  // positions past the registers
-    #pragma unroll
-    for (int i = 0; i < KR; i++) {
-      const int t = r0 + tid + SMR_T * i;
-      const double e = t < npos ? exp((double)srow[t] - m) : 0.0;
-      ex[(2 * i + (tid >> 8)) * 256 + (tid & 255)] = e;
-      if (t < npos) srow[t] = (float)e;
-    }
-    slot_add();
-  }
-  if (tid < 256) {
-    sum = wave_sum_xor(sum, 64);
-    if (lane == 0) redd[wave] = sum;
-  }
-  __syncthreads();
-  const double inv = 1.0 / ((redd[0] + redd[1]) + (redd[2] + redd[3]));
-  if (!NORM) {
-    if (tid == 0) a.pinv[(long)b * a.nHead + h] = inv;
+  if (!chainLane) return;
+  if (nrow <= ATTN_CHUNK) {
+    attn_emit(a, b, h, slice * AV_DIMS + lane, o);
     return;
   }
-  // the probabilities themselves, p = f32(f32(e) * inv)
+  chunk_store(chunk_rec(a, b, h, slice, chunk), lane, m, l, o);
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores are complete
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  const int n = (nrow + ATTN_CHUNK - 1) / ATTN_CHUNK;
+  uint32_t *cnt = a.rcnt + ((long)b * a.nHead + h) * NS + slice;
+  uint32_t at = 0;
+  if (lane == 0) at = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane(at) != (uint32_t)(n - 1)) return;
+  if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const double *r = chunk_rec(a, b, h, slice, 0);
+  auto ml = [&](int c) {
+    return make_double2(__hip_atomic_load(r + (long)c * REC_D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                        __hip_atomic_load(r + (long)c * REC_D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  };
+  float out[1];
+  chunk_join<1>(r, 0, n, lane, ml, out);
+  attn_emit(a, b, h, slice * AV_DIMS + lane, out[0]);
+}
+
+// The probabilities of every (chunk, query head, token) part of a pass of several tokens, in place of its scores, and its
+// (m_c, l_c). One wave per part: lane i takes k_attn_av's threads i, i + 64, i + 128 and i + 192 (their positions in their
+// order, then the same four 64-lane sums and (w0 + w1) + (w2 + w3)), so a part has one maximum and no barrier. Bound by
+// the f64 exponentials (~30 VALU instructions a position); with four waves per part their reductions cost as much again.
+__global__ __launch_bounds__(64) void k_attn_softmax_rows(const AttnArgs a) {
+  constexpr int NK = ATTN_CHUNK / 64;
+  const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
+  const Step *st = a.step;
+  const int t00 = chunk * ATTN_CHUNK, npos = min(st->pos0 + b + 1 - t00, ATTN_CHUNK);
+  if (b >= st->B || npos <= 0) return;
+  float *srow = a.scores + ((long)b * a.nHead + h) * a.sld + t00;
+  float v[NK], mx = -INFINITY;
   #pragma unroll
-  for (int k = 0; k < SMR_NK; k++) {
-    const int t = tid + SMR_T * k;
-    if (t < npos) srow[t] = (float)((double)v[k] * inv);
-  }
-  for (int t = SMR_NK * SMR_T + tid; t < npos; t += SMR_T) srow[t] = (float)((double)srow[t] * inv);
+  for (int k = 0; k < NK; k += 8)
+    if (k * 64 < npos) {  // (uniform; a position past the last repeats the first)
+      #pragma unroll
+      for (int j = k; j < k + 8; j++) { const int t = j * 64 + lane; v[j] = srow[t < npos ? t : 0]; }
+    }
+  #pragma unroll
+  for (int k = 0; k < NK; k += 8)
+    if (k * 64 < npos) {
+      #pragma unroll
+      for (int j = k; j < k + 8; j++) mx = fmaxf(mx, v[j]);
+    }
+  mx = group_fmax(mx, 64);
+  const double m = (double)mx;
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+  #pragma unroll
+  for (int k = 0; k < NK; k += 4)
+    if (k * 64 < npos) {  // positions 256 (k / 4) + 64 w + lane of the four waves w
+      double e[4];
+      #pragma unroll
+      for (int w = 0; w < 4; w++) e[w] = exp_neg((double)v[k + w] - m);
+      #pragma unroll
+      for (int w = 0; w < 4; w++) {
+        if ((k + w) * 64 + lane < npos) sum[w] += e[w];
+        v[k + w] = (float)e[w];
+      }
+    }
+  #pragma unroll
+  for (int w = 0; w < 4; w++) sum[w] = wave_sum_xor(sum[w], 64);
+  const double l = (sum[0] + sum[1]) + (sum[2] + sum[3]), inv = 1.0 / l;
+  #pragma unroll
+  for (int k = 0; k < NK; k += 4)
+    if (k * 64 < npos) {
+      #pragma unroll
+      for (int j = k; j < k + 4; j++) {
+        const int t = j * 64 + lane;
+        if (t < npos) srow[t] = (float)((double)v[j] * inv);
+      }
+    }
+  if (lane == 0) a.cml[((long)b * a.nHead + h) * a.nchunk + chunk] = make_double2(m, l);
 }
 
 // ---- weighted sum of passes of several tokens on the matrix cores. v_mfma_f32_16x16x4_f32 adds its four products to
 // the accumulator as four fused multiply-adds in k order (measured on gfx950, every element of random wide-range
 // operands), so a chain of them over positions t, t + 1, ... in order is the reference's f32 chain out += p_t v_t
 // (one rounding per position, src/model/forward.js:131-134) for 16 rows x 16 dimensions at once: the bits of k_attn_av.
-// Block: a 32-dimension slice of a KV head for RB = 16 or 32 rows r = b G + g (token b, query head kvh G + g), one or two
-// 16-row tiles. Waves 0 .. 2 RB / 16 - 1 run the chains of (row tile w / 2, dimensions 16 (w mod 2) .. + 15) (lane l
-// supplies A = p[row l mod 16][position 4 m + l / 16] and B = V[dimension l mod 16][4 m + l / 16] and holds (row
-// 4 (l / 16) + v, dimension l mod 16)) while as many waves more stage chunk c + 1 (the probabilities, already normalised
-// by k_attn_softmax_rows<true>,
-// zero past each row's last position; V as f32, zero past the pass's last position) and request chunk c + 3: each
-// producer unit is 16 consecutive positions of one row or dimension (16-byte loads, one 16-byte LDS store per position
-// section), two register sets in turn. As in k_attn_av_mfma the chain waves issue only MFMAs and LDS reads, one barrier
-// per chunk, operands by position mod 4 (section k holds positions 4 m + k). 32-row blocks stage V once for two tiles
-// (prefill chunks); 16-row blocks keep the chain waves on SIMDs of their own (one block per CU), for passes of few rows.
-constexpr int MMV_CT = 256;                 // positions per chunk
-constexpr int MMV_SF = MMV_CT / 4 + 4;      // floats of one position section (16-byte pad)
+// Block: one chunk of 16 rows r = b G + g (token b, query head kvh G + g) and 32 NDG dimensions of a KV head. Chain wave w
+// < NDG runs dimensions 32 w .. + 31 as two chains that share the A operand (lane l supplies A = p[row l mod 16][position
+// 4 m + l / 16], B = V[dimension l mod 16 (+ 16)][4 m + l / 16] and holds (row 4 (l / 16) + v, dimension l mod 16));
+// 2 NDG producer waves stage piece c + 1 meanwhile: V as f32 (zero past the pass's last position) and the probabilities
+// (already normalised by k_attn_softmax_rows, zero past a row's last position), with up to four pieces more on their way
+// in registers (a piece takes ~0.5 us, a load from memory 2-3); one barrier per piece. Operands lie in LDS by position mod 4 (section k holds positions 4 m + k), so a 16-byte
+// read gives four MFMAs' operands and the chain waves issue nothing but MFMAs and reads.
+// Bound by the MFMAs (32 cycles each) with the producers' instructions close behind (a wave alone on a SIMD issues one
+// every ~7 cycles, two one every ~5, so two producer waves share the staging of a SIMD's chain wave); a chain wave reads
+// 384 bytes of LDS per MFMA, 512 with one chain per wave. Pieces of 64 positions, so two blocks fit a CU.
+template <bool B> struct Whole { static constexpr bool value = B; };  // a piece below every row's last position
+constexpr int MMV_RB = 16;                  // rows per block
+constexpr int MMV_CT = 64;                  // positions per staged piece
+constexpr int MMV_SF = MMV_CT / 4;          // floats of one position section
 constexpr int MMV_RS = 4 * MMV_SF + 4;      // floats of one dimension or row (4 x an odd number: conflict-free chain reads)
-template <bool F16KV, int RB>
-__global__ __launch_bounds__(RB * 16) void k_attn_av_mm(const AttnArgs a, int nrows) {
+template <bool F16KV, int NDG>
+__global__ __launch_bounds__(NDG * 192, NDG * 6 / 4) void k_attn_av_mm(const AttnArgs a, int nrows) {
   extern __shared__ __align__(16) uint8_t lds[];
   typedef float f4 __attribute__((ext_vector_type(4)));
-  typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // a row of scores starts at any float
-  constexpr int VB = F16KV ? 2 : 4;
-  constexpr int CT = MMV_CT, SF = MMV_SF, RS = MMV_RS, NCW = RB / 8, NPT = NCW * 64;  // chain waves, producer threads
-  constexpr int EPP = 16 / VB;                      // positions per 16-byte V piece
-  constexpr int UL = 16 / EPP;                      // V pieces per unit of 16 positions (2 f16, 4 f32)
-  constexpr int UPR = CT / 16;                      // units per dimension or probability row of a chunk
-  constexpr int VU = AV_DIMS * UPR / NPT;           // V units per producer thread per chunk
-  constexpr int PU = RB * UPR / NPT;                // probability units per producer thread per chunk
-  constexpr int NU = CT / AVM_UNIT;                 // units (8 MFMAs) per chunk
-  static_assert((RB == 16 || RB == 32) && VU * NPT == AV_DIMS * UPR && PU * NPT == RB * UPR, "producer units");
-  float *vk = (float *)lds;                         // [2][AV_DIMS][RS]: V of position 4 m + k, dimension j at j RS + k SF + m
-  float *pk = vk + 2 * AV_DIMS * RS;                // [2][RB][RS]: p of row i, position 4 m + k at i RS + k SF + m
-  __shared__ float ot[RB][AV_DIMS + 1];             // the block's outputs [row][dimension] for the epilogue
+  constexpr int VB = F16KV ? 2 : 4, DB = 32 * NDG, RB = MMV_RB;
+  constexpr int CT = MMV_CT, SF = MMV_SF, RS = MMV_RS, NPT = NDG * 128;
+  constexpr int EPP = 16 / VB;                      // positions per 16-byte V load
+  constexpr int UL = 16 / EPP;                      // V loads per unit of 16 positions (2 f16, 4 f32)
+  constexpr int UPR = CT / 16;                      // units per dimension of a piece
+  constexpr int D = F16KV ? 4 : 2;                  // pieces in flight (as many as the registers hold)
+  constexpr int VU = DB * UPR / NPT;                // V units per producer thread per piece
+  constexpr int PN = RB * CT / NPT;                 // probabilities per producer thread per piece (2 or 4)
+  static_assert(VU * NPT == DB * UPR && (PN == 2 || PN == 4), "producer units");
+  float *vk = (float *)lds;                         // [2][DB][RS]: V of position 4 m + k, dimension j at j RS + k SF + m
+  float *pk = vk + 2 * DB * RS;                     // [2][RB][RS]: p of row i, position 4 m + k at i RS + k SF + m
   __shared__ long roff[RB];
-  __shared__ int rnp[RB];
+  __shared__ int rnp[RB], rfull[RB];                // the row's positions in the chunk, and in all
+  __shared__ uint32_t arrived;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n16 = lane & 15, g = lane >> 4;
-  // XCD-aware block order: workgroup i of the 1-D grid (a multiple of 8 long) goes to XCD i mod 8, and logical block
-  // L = (i mod 8) (grid / 8) + i / 8 gives each XCD a contiguous run of L, ordered slice fastest, then row block, then
-  // KV head, so the blocks that read the same probability rows (a row block's slices) and the same V (a KV head's row
-  // blocks) share one L2 instead of fetching them from HBM once per XCD
-  const int NS = a.hd / AV_DIMS, NZ = (nrows + RB - 1) / RB;
+  // XCD-aware block order: workgroup i of a chunk's blocks (a multiple of 8) goes to XCD i mod 8, and logical block
+  // L = (i mod 8) (blocks / 8) + i / 8 gives each XCD a contiguous run of L, ordered dimension block fastest, then row
+  // block, then KV head, so the blocks that read the same V share one L2
+  const int ND = a.hd / DB, NZ = (nrows + RB - 1) / RB;
   const int L = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  if (L >= NS * NZ * a.nHeadKv) return;
-  const int kvh = L / (NS * NZ), rbk = (L / NS) % NZ, d0 = (L % NS) * AV_DIMS;
+  if (L >= ND * NZ * a.nHeadKv) return;
+  const int kvh = L / (ND * NZ), rbk = (L / ND) % NZ, d0 = (L % ND) * DB;
   const int G = a.nHead / a.nHeadKv;
   const Step *st = a.step;
-  const int Bd = st->B, pos0 = st->pos0, nmax = pos0 + Bd;
-  // the block's rows: scores row offsets and positions (0: no row)
+  // positions below are relative to the chunk's first one, t00
+  const int chunk = blockIdx.y, t00 = chunk * ATTN_CHUNK;
+  const int Bd = st->B, pos0 = st->pos0, nmax = pos0 + Bd - t00;
+  if (nmax <= 0) return;
+  // the block's rows: scores row offsets, positions (0: no row; such a row reads the block's first one)
+  const long r0h = ((long)(rbk * RB / G) * a.nHead + kvh * G) * a.sld, r00 = r0h + t00;
   if (tid < RB) {
     const int r = rbk * RB + tid, b = r / G, h = kvh * G + r % G;
     const bool live = r < nrows && b < Bd;
-    roff[tid] = live ? ((long)b * a.nHead + h) * a.sld : 0;
-    rnp[tid] = live ? pos0 + b + 1 : 0;
+    roff[tid] = (live ? ((long)b * a.nHead + h) * a.sld : r0h) + t00;
+    rfull[tid] = live ? pos0 + b + 1 : 0;
+    rnp[tid] = max(0, min(rfull[tid] - t00, ATTN_CHUNK));
   }
   __syncthreads();
-  int nrmax = 0;
+  // a piece that ends at or before every live row's last position (all pieces but the last one or two) needs no load
+  // clamped and no value zeroed: fetch and stage take it in a form without those checks (rows without a live query read
+  // the block's first one there; their outputs are never stored, and row i of an MFMA result depends on row i of A only)
+  int nrmax = 0, nrfull = 0, nrmin = INT_MAX;
   #pragma unroll
-  for (int i = 0; i < RB; i++) nrmax = max(nrmax, rnp[i]);
+  for (int i = 0; i < RB; i++) {
+    nrmax = max(nrmax, rnp[i]);
+    nrfull = max(nrfull, rfull[i]);
+    nrmin = rnp[i] > 0 ? min(nrmin, rnp[i]) : nrmin;
+  }
   if (nrmax == 0) return;  // (uniform)
   const int nch = (nrmax + CT - 1) / CT;
-  const int nend = (nrmax + AVM_UNIT - 1) / AVM_UNIT * AVM_UNIT;  // positions the chains run
-  const uint8_t *vbase = (const uint8_t *)a.vcache + (((long)a.layer * a.nHeadKv + kvh) * a.hd + d0) * a.vstride * VB;
-  const bool producer = wave >= NCW;
-  const int pt = tid - NPT;                         // producer thread 0 .. NPT - 1
-  const int tr = RB == 32 ? (wave >> 1) & 1 : 0, dg = wave & 1;  // a chain wave's row tile and dimension group
-  bool tlive = false;                               // the chain wave's tile holds a row
-  #pragma unroll
-  for (int i = 0; i < 16; i++) tlive |= rnp[16 * tr + i] > 0;
-  struct Pre {
-    uint4 v[VU][UL];
-    f4 p[PU][4];
-  };
-  // a chunk that ends at or before every live row's last position (all chunks but the last one or two) needs no load
-  // clamped and no value zeroed: fetch and stage take it in a form without those checks (rows without a live query read
-  // row 0 of the scores there; their outputs are never stored, and row i of an MFMA result depends on row i of A only)
-  int nrmin = INT_MAX;
-  #pragma unroll
-  for (int i = 0; i < RB; i++) nrmin = rnp[i] > 0 ? min(nrmin, rnp[i]) : nrmin;
-  // chunk c's V pieces and probabilities (loads stay inside the cache row and the scores row; what lies past a row's or
-  // the pass's last position is zeroed when the chunk is staged)
-  auto fetch_f = [&](auto whole, int c, Pre &s) {
-    constexpr bool W = decltype(whole)::value;
-    #pragma unroll
-    for (int k = 0; k < VU; k++) {
-      const int u = k * NPT + pt, dim = u / UPR, t0 = c * CT + (u % UPR) * 16;
-      #pragma unroll
-      for (int l = 0; l < UL; l++) {
-        const int t = t0 + l * EPP;
-        s.v[k][l] = *(const uint4 *)(vbase + ((long)dim * a.vstride + (W || t < nmax ? t : 0)) * VB);
-      }
-    }
-    #pragma unroll
-    for (int k = 0; k < PU; k++) {
-      const int u = k * NPT + pt, r = u / UPR, t0 = c * CT + (u % UPR) * 16;
-      const float *src = a.scores + roff[r];
-      #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int tq = t0 + 4 * j;
-        s.p[k][j] = *(const f4u *)(src + (W || tq + 4 <= a.ctx ? tq : 0));
-      }
-    }
-  };
-  auto stage_f = [&](auto whole, int c, const Pre &s) {
-    constexpr bool W = decltype(whole)::value;
-    float *vs = vk + (c & 1) * AV_DIMS * RS;
-    #pragma unroll
-    for (int k = 0; k < VU; k++) {
-      const int u = k * NPT + pt, dim = u / UPR, uu = u % UPR, t0 = c * CT + uu * 16;
-      float f[16];
-      #pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const uint4 &pc = s.v[k][e / EPP];
-        const int w = e % EPP;
-        const uint32_t wd = (F16KV ? w >> 1 : w) == 0 ? pc.x : (F16KV ? w >> 1 : w) == 1 ? pc.y : (F16KV ? w >> 1 : w) == 2 ? pc.z : pc.w;
-        const float x = F16KV ? h2f((uint16_t)((w & 1) ? (wd >> 16) : (wd & 0xffff))) : __uint_as_float(wd);
-        f[e] = W || t0 + e < nmax ? x : 0.f;
-      }
-      float *drow = vs + dim * RS + uu * 4;
-      #pragma unroll
-      for (int q = 0; q < 4; q++) *(f4 *)(drow + q * SF) = (f4){f[q], f[q + 4], f[q + 8], f[q + 12]};
-    }
-    float *ps = pk + (c & 1) * RB * RS;
-    #pragma unroll
-    for (int k = 0; k < PU; k++) {
-      const int u = k * NPT + pt, r = u / UPR, uu = u % UPR, t0 = c * CT + uu * 16;
-      float *prow = ps + r * RS + uu * 4;
-      if (W) {
-        #pragma unroll
-        for (int e = 0; e < 4; e++) *(f4 *)(prow + e * SF) = (f4){s.p[k][0][e], s.p[k][1][e], s.p[k][2][e], s.p[k][3][e]};
-      } else {
-        const int np = rnp[r];
-        #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          f4 w;
-          #pragma unroll
-          for (int j = 0; j < 4; j++) w[j] = t0 + 4 * j + e < np ? s.p[k][j][e] : 0.f;
-          *(f4 *)(prow + e * SF) = w;
-        }
-      }
-    }
-  };
-  // (f16 V only: with f32 V both forms do not fit the registers together)
-  auto fetch = [&](int c, Pre &s) {
-    if (F16KV && (c + 1) * CT <= nrmin) fetch_f(Whole<F16KV>{}, c, s);
-    else fetch_f(Whole<false>{}, c, s);
-  };
-  auto stage = [&](int c, const Pre &s) {
-    if (F16KV && (c + 1) * CT <= nrmin) stage_f(Whole<F16KV>{}, c, s);
-    else stage_f(Whole<false>{}, c, s);
-  };
-  Pre s0, s1;
+  const int nend = (nrmax + AV_UNIT - 1) / AV_UNIT * AV_UNIT;  // positions the chains run
+  const uint8_t *vbase = (const uint8_t *)a.vcache + ((((long)a.layer * a.nHeadKv + kvh) * a.hd + d0) * a.vstride + t00) * VB;
+  const bool producer = wave >= NDG;
+  f4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+  // the producers and the chain waves run loops of their own with one barrier per piece each (the same count), so the
+  // chains' accumulators stay in their registers from piece to piece
   if (producer) {
-    fetch(0, s0);
-    if (nch > 1) fetch(1, s1);
-    stage(0, s0);
-    if (nch > 2) fetch(2, s0);
-  }
-  __syncthreads();
-  f4 acc = {0.f, 0.f, 0.f, 0.f};
-  auto mfma8 = [&](const f4 &p0, const f4 &p1, const f4 &v0, const f4 &v1) {
-    #pragma unroll
-    for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[i], v0[i], acc, 0, 0, 0);
-    #pragma unroll
-    for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[i], v1[i], acc, 0, 0, 0);
-  };
-  auto chains = [&](int c) {
-    // unit u: the 8 MFMAs of positions c CT + 32 u .. + 31 (lane group g: positions 4 m + g, m = 8 u .. 8 u + 7); two
-    // operand sets, the next unit's reads ahead of the current unit's MFMAs, a full chunk in straight-line code
-    const float *vr = vk + ((c & 1) * AV_DIMS + dg * 16 + n16) * RS + g * SF;
-    const float *pr = pk + ((c & 1) * RB + tr * 16 + n16) * RS + g * SF;
-    auto ld = [&](const float *q, int off) { return *(const f4 *)(q + off); };
-    if (c * CT + CT <= nend) {
-      f4 a0 = ld(pr, 0), a1 = ld(pr, 4), a2 = ld(vr, 0), a3 = ld(vr, 4);
+    const int pt = tid - NDG * 64;                  // producer thread 0 .. NPT - 1
+    const int pr = pt * PN / CT, pq = pt * PN % CT; // its row and first position of its PN probabilities in a piece
+    const int np = rnp[pr];
+    // both by buffer loads: the thread's offset in registers, the piece's in a scalar, and no branch around a load (past
+    // the V rows and the pass's scores zeros, without an access), so that the waits count exactly the piece they are for
+    const uint32_t vrow = (uint32_t)a.vstride * VB;
+    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc((void *)vbase, (short)0, (int)(DB * vrow - t00 * VB), 0x00020000);
+    const long pend = (long)Bd * a.nHead * a.sld - r00;  // floats from the block's first row on
+    const __amdgpu_buffer_rsrc_t pr_ =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(a.scores + r00), (short)0, (int)(uint32_t)min(pend * 4, 0xfffffff0l), 0x00020000);
+    const uint32_t poff = (uint32_t)(roff[pr] - r00 + pq) * 4;
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    struct Pre {
+      u4 v[VU][UL];
+      float p[PN];
+    };
+    // piece c's V and scores (what lies past a row's or the pass's last position is zeroed when the piece is staged)
+    auto fetch = [&](int c, Pre &s) {
       #pragma unroll
-      for (int u = 0; u < NU; u += 2) {
-        const f4 b0 = ld(pr, 8 * u + 8), b1 = ld(pr, 8 * u + 12), b2 = ld(vr, 8 * u + 8), b3 = ld(vr, 8 * u + 12);
-        __builtin_amdgcn_sched_barrier(0);
-        mfma8(a0, a1, a2, a3);
-        if (u + 2 < NU) { a0 = ld(pr, 8 * u + 16); a1 = ld(pr, 8 * u + 20); a2 = ld(vr, 8 * u + 16); a3 = ld(vr, 8 * u + 20); }
-        __builtin_amdgcn_sched_barrier(0);
-        mfma8(b0, b1, b2, b3);
+      for (int k = 0; k < VU; k++) {
+        const int u = k * NPT + pt, dim = u / UPR;
+        #pragma unroll
+        for (int l = 0; l < UL; l++)
+          s.v[k][l] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(vr, dim * vrow + ((u % UPR) * 16 + l * EPP) * VB, c * CT * VB, 0));
       }
-    } else {
-      const int nu = (nend - c * CT) / AVM_UNIT;
-      f4 a0 = ld(pr, 0), a1 = ld(pr, 4), a2 = ld(vr, 0), a3 = ld(vr, 4);
-      int u = 0;
-      for (; u + 2 <= nu; u += 2) {
-        const f4 b0 = ld(pr, 8 * u + 8), b1 = ld(pr, 8 * u + 12), b2 = ld(vr, 8 * u + 8), b3 = ld(vr, 8 * u + 12);
-        __builtin_amdgcn_sched_barrier(0);
-        mfma8(a0, a1, a2, a3);
-        const int un = min(u + 2, nu - 1);  // (a re-read of the last unit when past it)
-        a0 = ld(pr, 8 * un); a1 = ld(pr, 8 * un + 4); a2 = ld(vr, 8 * un); a3 = ld(vr, 8 * un + 4);
-        __builtin_amdgcn_sched_barrier(0);
-        mfma8(b0, b1, b2, b3);
-      }
-      if (u < nu) mfma8(a0, a1, a2, a3);
-    }
-  };
-  // the producers and the chain waves run loops of their own with one barrier per chunk each (the same count), so the
-  // chains' accumulator stays in the matrix cores' registers from chunk to chunk; chunk c + 1 sits in register set
-  // (c + 1) mod 2, which then requests chunk c + 3
-  if (producer) {
-    for (int c = 0; c < nch; c += 2) {
-      if (c + 1 < nch) {
-        stage(c + 1, s1);
-        if (c + 3 < nch) fetch(c + 3, s1);
-      }
-      __syncthreads();
-      if (c + 1 < nch) {
-        if (c + 2 < nch) {
-          stage(c + 2, s0);
-          if (c + 4 < nch) fetch(c + 4, s0);
+      #pragma unroll
+      for (int j = 0; j < PN; j++) s.p[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(pr_, poff + 4 * j, c * CT * 4, 0));
+    };
+    auto stage_f = [&](auto whole, int c, const Pre &s) {
+      constexpr bool W = decltype(whole)::value;
+      float *vs = vk + (c & 1) * DB * RS;
+      #pragma unroll
+      for (int k = 0; k < VU; k++) {
+        const int u = k * NPT + pt, dim = u / UPR, uu = u % UPR, t0 = c * CT + uu * 16;
+        float f[16];
+        #pragma unroll
+        for (int e = 0; e < 16; e++) {
+          const int w = e % EPP;
+          const uint32_t wd = s.v[k][e / EPP][F16KV ? w >> 1 : w];
+          const float x = F16KV ? h2f((uint16_t)((w & 1) ? (wd >> 16) : (wd & 0xffff))) : __uint_as_float(wd);
+          f[e] = W || t0 + e < nmax ? x : 0.f;
         }
+        float *drow = vs + dim * RS + uu * 4;
+        #pragma unroll
+        for (int q = 0; q < 4; q++) *(f4 *)(drow + q * SF) = (f4){f[q], f[q + 4], f[q + 8], f[q + 12]};
+      }
+      float *prow = pk + (c & 1) * RB * RS + pr * RS + (pq >> 2);
+      #pragma unroll
+      for (int j = 0; j < PN; j++) prow[((pq + j) & 3) * SF] = W || c * CT + pq + j < np ? s.p[j] : 0.f;
+    };
+    auto stage = [&](int c, const Pre &s) {
+      if ((c + 1) * CT <= nrmin) stage_f(Whole<true>{}, c, s);
+      else stage_f(Whole<false>{}, c, s);
+    };
+    // piece c lies in register set c mod D, which requests piece c + D as soon as it is staged
+    Pre s[D];
+    #pragma unroll
+    for (int d = 0; d < D; d++) fetch(d, s[d]);
+    stage(0, s[0]);
+    fetch(D, s[0]);
+    __syncthreads();
+    for (int c0 = 0; c0 < nch; c0 += D) {  // piece c + 1 is staged while the chains run piece c
+      #pragma unroll
+      for (int d = 0; d < D; d++) {
+        const int c = c0 + d;
+        if (c >= nch) break;
+        if (c + 1 < nch) stage(c + 1, s[(d + 1) % D]);
+        fetch(c + 1 + D, s[(d + 1) % D]);
         __syncthreads();
       }
     }
   } else {
+    __syncthreads();
+    auto ld = [&](const float *q) { return *(const f4 *)q; };
+    const float *vr0 = vk + (wave * 32 + n16) * RS + g * SF, *pr0 = pk + n16 * RS + g * SF;
     for (int c = 0; c < nch; c++) {
-      if (tlive) chains(c);
+      // 16 positions per step (4 MFMAs per chain; lane group g: positions 4 m + g, m = 4 u .. 4 u + 3), the next step's
+      // reads ahead of the current one's MFMAs; two steps per unit of 32 positions
+      const float *vr = vr0 + (c & 1) * DB * RS, *pr = pr0 + (c & 1) * RB * RS;
+      auto step = [&](const f4 &p, const f4 &v0, const f4 &v1) {
+        #pragma unroll
+        for (int i = 0; i < 4; i++) {
+          acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i], v0[i], acc0, 0, 0, 0);
+          acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i], v1[i], acc1, 0, 0, 0);
+        }
+      };
+      const int nu = min(CT, nend - c * CT) / 16;  // 2 or 4 steps
+      f4 p0 = ld(pr), x0 = ld(vr), y0 = ld(vr + 16 * RS);
+      f4 p1 = ld(pr + 4), x1 = ld(vr + 4), y1 = ld(vr + 16 * RS + 4);
+      __builtin_amdgcn_sched_barrier(0);
+      step(p0, x0, y0);
+      if (nu > 2) {
+        p0 = ld(pr + 8); x0 = ld(vr + 8); y0 = ld(vr + 16 * RS + 8);
+        __builtin_amdgcn_sched_barrier(0);
+        step(p1, x1, y1);
+        p1 = ld(pr + 12); x1 = ld(vr + 12); y1 = ld(vr + 16 * RS + 12);
+        __builtin_amdgcn_sched_barrier(0);
+        step(p0, x0, y0);
+      }
+      step(p1, x1, y1);
       __syncthreads();
     }
   }
-  // ---- epilogue: the outputs through LDS, then two rows per wave, a row's 32 dimensions on 32 consecutive lanes (one
-  // quantizeAct block)
+  // ---- epilogue: the outputs through LDS (the staged pieces are no longer read), a row's 32 dimensions on 32
+  // consecutive lanes (one quantizeAct block)
+  constexpr int OP = DB + 1;
+  float *ot = (float *)lds;
   if (!producer) {
     #pragma unroll
-    for (int v = 0; v < 4; v++) ot[16 * tr + 4 * g + v][16 * dg + n16] = acc[v];
+    for (int v = 0; v < 4; v++) {
+      ot[(4 * g + v) * OP + 32 * wave + n16] = acc0[v];
+      ot[(4 * g + v) * OP + 32 * wave + 16 + n16] = acc1[v];
+    }
   }
   __syncthreads();
-  #pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const int i = j * (RB / 2) + wave * 2 + (lane >> 5);  // (2 NCW waves: RB / 2 rows per pass)
+  constexpr int NH = 6 * NDG;                       // half-waves
+  const int hw = tid >> 5, l32 = tid & 31;
+  for (int e = hw; e < RB * NDG; e += NH) {
+    const int i = e / NDG, sl = e % NDG;
     if (rnp[i] == 0) continue;
-    const int r = rbk * RB + i, b = r / G, h = kvh * G + r % G, dim = d0 + (lane & 31), col = h * a.hd + dim;
-    float o = ot[i][lane & 31];
-    if (a.gate) {  // gated attention output (src/model/forward-qwen35.js:103): o * sigmoid(gate), f64, stored f32
-      const double gv = (double)a.gate[(long)b * a.ldq + (long)h * a.qhs + dim];
-      o = (float)((double)o * (1.0 / (1.0 + exp(-gv))));
-    }
-    if (a.out) a.out[(long)b * a.ldo + col] = o;
-    if (a.act.q) quant_block32(o, col, a.act, b);  // (unset: the output GEMV quantises the f32 rows itself)
+    const int r = rbk * RB + i, b = r / G, h = kvh * G + r % G;
+    const float o = ot[i * OP + 32 * sl + l32];
+    if (rfull[i] <= ATTN_CHUNK) attn_emit(a, b, h, d0 + 32 * sl + l32, o);
+    else __hip_atomic_store((float *)(chunk_rec(a, b, h, d0 / 32 + sl, chunk) + 2) + l32, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-}
-
-size_t attention_av_mm_lds(int rb) { return (size_t)2 * (AV_DIMS + rb) * MMV_RS * 4; }
-
-// nrows: query heads per KV head x the launch's tokens (rows r = b G + g: token b, query head kvh G + g).
-// 512 threads: waves 0-3 run the chains of chunk c while waves 4-7 store chunk c + 1 (V and probabilities) into the
-// other buffer and request chunk c + 2, so the staging never stands between two chunks' chains (one barrier per chunk).
-constexpr int AVG_THREADS = 512;
-template <bool F16KV, int ROWB>
-__global__ __launch_bounds__(AVG_THREADS) void k_attn_av_group(const AttnArgs a, int nrows) {
-  extern __shared__ __align__(16) uint8_t lds[];
-  constexpr int VB = F16KV ? 2 : 4;
-  constexpr int CT = ROWB / VB;                       // positions per chunk
-  constexpr int EPP = 16 / VB;                        // positions per 16-byte piece
-  constexpr int PPR = ROWB / 16;                      // pieces per row
-  constexpr int PITCH = ROWB + 16;                    // LDS pitch of a staged V row
-  constexpr int CHUNK = AVG_DIMS * PITCH;             // bytes of one staged chunk of V rows
-  constexpr int LPT = AVG_DIMS * PPR / 256;           // V pieces per staging thread per chunk
-  constexpr int PPT = AVG_ROWS * CT / 256;            // probabilities per staging thread per chunk
-  static_assert(AVG_DIMS * PPR % 256 == 0 && AVG_ROWS * CT % 256 == 0 && AVG_ROWS == 8, "chunk geometry");
-  constexpr int CTP = CT + 4;                         // row pitch of the staged probabilities (the two rows a wave
-                                                      // reads at once fall on different banks)
-  float *pb = (float *)(lds + 2 * CHUNK);             // [2][AVG_ROWS][CTP] staged probabilities
-  __shared__ int rnpos[AVG_ROWS];
-  __shared__ long roff[AVG_ROWS];
-  __shared__ double rinv[AVG_ROWS];
-  const int slice = blockIdx.x, kvh = blockIdx.y, r0 = blockIdx.z * AVG_ROWS, tid = threadIdx.x, wave = tid >> 6,
-            lane = tid & 63;
-  const bool stager = tid >= 256;
-  const int sid = tid - 256;                          // staging thread index (stagers only)
-  const int G = a.nHead / a.nHeadKv;
-  const uint8_t *vbase = (const uint8_t *)a.vcache +
-                         (((long)a.layer * a.nHeadKv + kvh) * a.hd + (long)slice * AVG_DIMS) * a.vstride * VB;
-  uint4 pre[LPT];
-  float pp[PPT];
-  auto fetch = [&](int c, int lim) {
-    #pragma unroll
-    for (int k = 0; k < LPT; k++) {
-      const int idx = k * 256 + sid, dim = idx / PPR, t = c * CT + (idx % PPR) * EPP;
-      pre[k] = t < lim ? *(const uint4 *)(vbase + ((long)dim * a.vstride + t) * VB) : make_uint4(0, 0, 0, 0);
-    }
-  };
-  auto store = [&](int buf) {
-    #pragma unroll
-    for (int k = 0; k < LPT; k++) {
-      const int idx = k * 256 + sid;
-      *(uint4 *)(lds + buf * CHUNK + (idx / PPR) * PITCH + (idx % PPR) * 16) = pre[k];
-    }
-  };
-  if (stager) fetch(0, a.ctx);
-  const Step *st = a.step;
-  const int Bd = st->B, pos0 = st->pos0;
-  // the group's rows: their scores rows, last positions (0: no row) and 1 / sum
-  if (tid < AVG_ROWS) {
-    const int r = r0 + tid, b = r / G, h = kvh * G + r % G;
-    const bool live = r < nrows && b < Bd;
-    rnpos[tid] = live ? pos0 + b + 1 : 0;
-    roff[tid] = live ? ((long)b * a.nHead + h) * a.sld : 0;
-    rinv[tid] = live ? a.pinv[(long)b * a.nHead + h] : 0.0;
-  }
+  if (nrfull <= ATTN_CHUNK) return;  // (uniform)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores are complete
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __syncthreads();
-  int nmax = 0;
-  #pragma unroll
-  for (int i = 0; i < AVG_ROWS; i++) nmax = max(nmax, rnpos[i]);
-  if (nmax == 0) return;  // (uniform over the block)
-  const int nch = (nmax + CT - 1) / CT;
-  // probabilities of chunk c for the group's rows (zero past each row's last position)
-  auto pload = [&](int c) {
-    #pragma unroll
-    for (int k = 0; k < PPT; k++) {
-      const int idx = k * 256 + sid, rr = idx / CT, t = c * CT + idx % CT;
-      pp[k] = t < rnpos[rr] ? a.scores[roff[rr] + t] : 0.f;
-    }
-  };
-  auto pstore = [&](int buf) {
-    #pragma unroll
-    for (int k = 0; k < PPT; k++) {
-      const int idx = k * 256 + sid, rr = idx / CT;
-      pb[(buf * AVG_ROWS + rr) * CTP + idx % CT] = (float)((double)pp[k] * rinv[rr]);
-    }
-  };
-  if (stager) {
-    #pragma unroll
-    for (int k = 0; k < LPT; k++) {  // the first chunk's pieces from the group's last position on: zeros
-      const int t = ((k * 256 + sid) % PPR) * EPP;
-      if (t >= nmax) pre[k] = make_uint4(0, 0, 0, 0);
-      else if (t + EPP > nmax) {
-        uint32_t w[4] = {pre[k].x, pre[k].y, pre[k].z, pre[k].w};
-        #pragma unroll
-        for (int e = 0; e < EPP; e++)
-          if (t + e >= nmax) {
-            if (F16KV) w[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
-            else w[e] = 0u;
-          }
-        pre[k] = make_uint4(w[0], w[1], w[2], w[3]);
-      }
-    }
-    pload(0);
-    store(0);
-    pstore(0);
-    if (nch > 1) { fetch(1, nmax); pload(1); }
-  }
+  uint32_t *cnt = a.rcnt + L;
+  if (tid == 0) arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  // ---- weighted sum: row rl = 2 wave + lane / 32, dimension d = lane mod 32 of the slice, chunk by chunk (waves 0-3)
-  const int rl = 2 * (wave & 3) + (lane >> 5), d = lane & 31;
-  float o = 0.f;
-  for (int c = 0; c < nch; c++) {
-    if (stager) {
-      // chunk c + 1 into the buffer the chains left at the last barrier, then the loads of chunk c + 2
-      if (c + 1 < nch) {
-        store((c + 1) & 1);
-        pstore((c + 1) & 1);
-        if (c + 2 < nch) { fetch(c + 2, nmax); pload(c + 2); }
-      }
-    } else {
-      const int cnt = min(CT, nmax - c * CT), nu = (cnt + AV_UNIT - 1) / AV_UNIT;
-      const uint8_t *row = lds + (c & 1) * CHUNK + d * PITCH;
-      const float *pc = pb + ((c & 1) * AVG_ROWS + rl) * CTP;
-      float4 pa[AV_UNIT / 4], pbv[AV_UNIT / 4];
-      uint4 va[AV_UNIT * VB / 16], vb[AV_UNIT * VB / 16];
-      auto read = [&](int u, float4 (&pv)[AV_UNIT / 4], uint4 (&vv)[AV_UNIT * VB / 16]) {
-        #pragma unroll
-        for (int k = 0; k < AV_UNIT / 4; k++) pv[k] = *(const float4 *)(pc + u * AV_UNIT + 4 * k);
-        #pragma unroll
-        for (int k = 0; k < AV_UNIT * VB / 16; k++) vv[k] = *(const uint4 *)(row + (u * AV_UNIT + k * EPP) * VB);
-      };
-      auto steps = [&](const float4 (&pv)[AV_UNIT / 4], const uint4 (&vv)[AV_UNIT * VB / 16]) {
-        #pragma unroll
-        for (int k = 0; k < AV_UNIT / 4; k++) {
-          float v0, v1, v2, v3;
-          if (F16KV) {
-            const uint4 &w = vv[k >> 1];
-            const uint32_t lo = (k & 1) ? w.z : w.x, hi = (k & 1) ? w.w : w.y;
-            v0 = h2f((uint16_t)(lo & 0xffff)); v1 = h2f((uint16_t)(lo >> 16));
-            v2 = h2f((uint16_t)(hi & 0xffff)); v3 = h2f((uint16_t)(hi >> 16));
-          } else {
-            const uint4 &w = vv[k];
-            v0 = __uint_as_float(w.x); v1 = __uint_as_float(w.y); v2 = __uint_as_float(w.z); v3 = __uint_as_float(w.w);
-          }
-          o = fmaf(pv[k].x, v0, o); o = fmaf(pv[k].y, v1, o); o = fmaf(pv[k].z, v2, o); o = fmaf(pv[k].w, v3, o);
-        }
-      };
-      read(0, pa, va);
-      int u = 0;
-      for (; u + 2 <= nu; u += 2) {
-        read(u + 1, pbv, vb);
-        __builtin_amdgcn_sched_barrier(0);
-        steps(pa, va);
-        read(min(u + 2, nu - 1), pa, va);
-        __builtin_amdgcn_sched_barrier(0);
-        steps(pbv, vb);
-      }
-      if (u < nu) steps(pa, va);
-    }
-    __syncthreads();
-  }
-  if (!stager && rnpos[rl] > 0) {  // (the same for the 32 lanes of the row)
-    const int r = r0 + rl, b = r / G, h = kvh * G + r % G, dim = slice * AVG_DIMS + d, col = h * a.hd + dim;
-    if (a.gate) {  // gated attention output (src/model/forward-qwen35.js:103): o * sigmoid(gate), f64, stored f32
-      const double g = (double)a.gate[(long)b * a.ldq + (long)h * a.qhs + dim];
-      o = (float)((double)o * (1.0 / (1.0 + exp(-g))));
-    }
-    if (a.out) a.out[(long)b * a.ldo + col] = o;
-    if (a.act.q) quant_block32(o, col, a.act, b);  // (unset: the output GEMV quantises the f32 rows itself)
+  if (arrived != (uint32_t)((nrfull + ATTN_CHUNK - 1) / ATTN_CHUNK - 1)) return;  // (the chunks this block's rows have)
+  if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int i = hw; i < RB; i += NH) {  // a row's slices together
+    if (rfull[i] <= ATTN_CHUNK) continue;
+    const int r = rbk * RB + i, b = r / G, h = kvh * G + r % G;
+    const double2 *mlr = a.cml + ((long)b * a.nHead + h) * a.nchunk;
+    float out[NDG];
+    chunk_join<NDG>(chunk_rec(a, b, h, d0 / 32, 0), (long)a.nchunk * REC_D, (rfull[i] + ATTN_CHUNK - 1) / ATTN_CHUNK, l32,
+                    [&](int c) { return mlr[c]; }, out);
+    #pragma unroll
+    for (int sl = 0; sl < NDG; sl++) attn_emit(a, b, h, d0 + 32 * sl + l32, out[sl]);
   }
 }
 
-// LDS of a grouped block with chunks of rowb bytes per dimension: two staged V chunks and two chunks of probabilities
-size_t attention_group_lds(int kvF16, int rowb) {
-  return (size_t)2 * AVG_DIMS * (rowb + 16) + (size_t)2 * AVG_ROWS * (rowb / (kvF16 ? 2 : 4) + 4) * 4;
-}
-
-template <bool F16KV, int ROWB>
-static void launch_av_group_k(const AttnArgs &a, dim3 grid, int nrows, hipStream_t st) {
-  static size_t attr = 64 * 1024;  // dynamic LDS above 64 KB must be requested per kernel
-  const size_t lds = attention_group_lds(F16KV, ROWB);
-  if (lds > attr) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_group<F16KV, ROWB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = lds;
-  }
-  hipLaunchKernelGGL((k_attn_av_group<F16KV, ROWB>), grid, dim3(AVG_THREADS), lds, st, a, nrows);
-}
-
-template <int HD, bool F16KV>
-static void launch_av_head_k(const AttnArgs &a, int B, hipStream_t st) {
-  static size_t attr = 64 * 1024;
-  const size_t lds = attention_head_lds(HD);
-  if (lds > attr) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_head<HD, F16KV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = lds;
-  }
-  hipLaunchKernelGGL((k_attn_av_head<HD, F16KV>), dim3(1, a.nHead, B), dim3(256), lds, st, a);
-}
+static size_t attention_av_mm_lds(int ndg) { return (size_t)2 * (32 * ndg + MMV_RB) * MMV_RS * 4; }
 
 // ---- position-split weighted sum (long contexts). The exact chain above runs one dependent f32 step per position, so
 // at 16K positions it is ~40 us per output element. Here one block per (256-position chunk, query head, token) takes
@@ -1639,57 +1098,34 @@ __global__ __launch_bounds__(256) void k_attn_merge(const AttnArgs a) {
 
 size_t attention_split_lds(int hd, int kvF16) { return (size_t)hd * (ATTN_SPLIT_C * (kvF16 ? 2 : 4) + 4); }
 
-// Dynamic LDS of one k_attn_av block: the probabilities of ctx positions and two staged V chunks (of AV_ROW or rowb
-// bytes per dimension).
-size_t attention_lds(int ctx, int rowb) {
-  return (size_t)((ctx + AV_UNIT - 1) / AV_UNIT * AV_UNIT) * 4 + 2 * (size_t)AV_DIMS * (rowb + 16);
-}
-size_t attention_lds(int ctx) { return attention_lds(ctx, AV_ROW); }
-constexpr size_t ATTN_LDS_MAX = 150 * 1024;
+// Dynamic LDS of one k_attn_av block: the probabilities of its positions and two staged pieces of V.
+static size_t attention_lds(int nsc) { return (size_t)256 * nsc * 4 + 2 * (size_t)AV_STAGE; }
 
-// Contexts above AVH_CTX positions take the per-head weighted sum (heads of at most 128 dimensions), whose LDS does not
-// depend on the context, for passes of several tokens; single-token passes keep the slice form wherever its softmax
-// row fits LDS. ZEROLLM_ATTN_HEAD_CTX / ZEROLLM_ATTN_HEAD1_CTX override the two thresholds (tests). Read once per model.
-AttnForm attention_form(int ctx, int hd) {
-  const char *e = getenv("ZEROLLM_ATTN_HEAD_CTX"), *e1 = getenv("ZEROLLM_ATTN_HEAD1_CTX");
+constexpr int LONG_CTX = 8192;  // contexts from which passes of 2 tokens or more take the matrix-core forms
+
+AttnForm attention_form(int ctx) {
   AttnForm f;
-  f.headCtx = hd > 128 ? INT_MAX : e ? atoi(e) : AVH_CTX;
-  // single-token passes: the per-head form once the slice form's LDS no longer holds the row
-  int fit = 0;
-  while (fit < ctx && attention_lds(fit + AV_UNIT) <= ATTN_LDS_MAX) fit += AV_UNIT;
-  f.head1Ctx = hd > 128 ? INT_MAX : e1 ? atoi(e1) : std::max(f.headCtx, fit);
-  f.split = ctx > f.headCtx ? false : attention_lds(ctx) > ATTN_LDS_MAX;
   // matrix-core score dots for passes of 16 tokens or more (prefill chunks), and of 2 or more where the context is long
   // (verify passes at long contexts); ZEROLLM_ATTN_MM_B overrides the token count (tests)
   const char *em = getenv("ZEROLLM_ATTN_MM_B");
-  f.mmMinB = em ? atoi(em) : ctx >= AVH_CTX ? 2 : 16;
+  f.mmMinB = em ? atoi(em) : ctx >= LONG_CTX ? 2 : 16;
   // their weighted sums on the matrix cores likewise: from 16 tokens on (32-row blocks), and from 2 where the context
-  // is long (16-row blocks: 9-token verify passes at 16K positions 10.77 -> 10.52 ms against the grouped lane chains)
+  // is long (16-row blocks)
   const char *ea = getenv("ZEROLLM_ATTN_MMAV_B");
-  f.mmAvMinB = ea ? atoi(ea) : em ? f.mmMinB : ctx >= AVH_CTX ? 2 : 16;
-  // where the slice form's softmax row would not fit LDS (256-dimension heads beyond ~29,900 positions) every pass
-  // takes the matrix-core weighted sum, whose staging does not grow with the context: the exact chain at any context
-  if (f.split) {
-    f.split = false;
-    f.mmAvMinB = 1;
-  }
-  // the slice form's chains on the matrix cores from AV_BIG_CTX positions, where the lane-chain form's LDS already
-  // holds a CU to one block (ZEROLLM_ATTN_AVMF=1 / 0: at any context / never; the same bits)
-  const char *ev = getenv("ZEROLLM_ATTN_AVMF");
-  f.avmf = ctx <= AVM_MAX_CTX && (ev ? ev[0] == '1' : ctx >= AV_BIG_CTX);
+  f.mmAvMinB = ea ? atoi(ea) : em ? f.mmMinB : ctx >= LONG_CTX ? 2 : 16;
   return f;
 }
 
-template <bool F16KV, int RB>
+template <bool F16KV, int NDG>
 static void launch_av_mm_k(const AttnArgs &a, int nrows, hipStream_t st) {
   static bool attr = false;  // dynamic LDS above 64 KB must be requested per kernel
   if (!attr) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_mm<F16KV, RB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)attention_av_mm_lds(RB)));
+    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_mm<F16KV, NDG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)attention_av_mm_lds(NDG)));
     attr = true;
   }
-  const int nb = a.hd / AV_DIMS * a.nHeadKv * ((nrows + RB - 1) / RB);  // (slice, KV head, row block) blocks
-  const dim3 grid((nb + 7) / 8 * 8);
-  hipLaunchKernelGGL((k_attn_av_mm<F16KV, RB>), grid, dim3(RB * 16), attention_av_mm_lds(RB), st, a, nrows);
+  const int nb = a.hd / (32 * NDG) * a.nHeadKv * ((nrows + MMV_RB - 1) / MMV_RB);  // (dimensions, KV head, rows) blocks
+  const dim3 grid((nb + 7) / 8 * 8, a.nchunk);
+  hipLaunchKernelGGL((k_attn_av_mm<F16KV, NDG>), grid, dim3(NDG * 192), attention_av_mm_lds(NDG), st, a, nrows);
 }
 
 template <int HD, bool F16KV>
@@ -1726,33 +1162,11 @@ static void launch_scores_k(const AttnArgs &a, dim3 grid, int B, hipStream_t st)
   hipLaunchKernelGGL((k_attn_scores<HD, F16KV>), grid, dim3(256), kn, st, a);
 }
 
-template <bool F16KV, int ROWB>
-static void launch_av_rows(const AttnArgs &a, dim3 grid, size_t lds, hipStream_t st) {
-  static size_t attr = 64 * 1024;  // dynamic LDS above 64 KB must be requested per kernel
-  if (lds > attr) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av<F16KV, ROWB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = lds;
-  }
-  hipLaunchKernelGGL((k_attn_av<F16KV, ROWB>), grid, dim3(256), lds, st, a);
-}
-
-// the larger chunk for long contexts where it fits (the same bits: only the staging changes); at short contexts its
-// LDS would halve the blocks a CU holds (measured: 5-token verify pass 3.11 -> 3.32 ms at 1024 positions)
 template <bool F16KV>
-static void launch_av_k(const AttnArgs &a, dim3 grid, size_t lds, hipStream_t st) {
-  const size_t big = attention_lds(a.ctx, AV_ROW_BIG);
-  if (a.ctx >= AV_BIG_CTX && big <= ATTN_LDS_MAX) launch_av_rows<F16KV, AV_ROW_BIG>(a, grid, big, st);
-  else launch_av_rows<F16KV, AV_ROW>(a, grid, lds, st);
-}
-
-template <bool F16KV>
-static void launch_av_mfma_k(const AttnArgs &a, dim3 grid, size_t lds, hipStream_t st) {
-  static size_t attr = 64 * 1024;  // dynamic LDS above 64 KB must be requested per kernel
-  if (lds > attr) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_mfma<F16KV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = lds;
-  }
-  hipLaunchKernelGGL((k_attn_av_mfma<F16KV>), grid, dim3(256), lds, st, a);
+static void launch_av_k(const AttnArgs &a, int B, hipStream_t st) {
+  const dim3 grid(a.hd / AV_DIMS * a.nchunk, a.nHead, B);
+  if (a.ctx <= 1024) hipLaunchKernelGGL((k_attn_av<F16KV, 4>), grid, dim3(256), attention_lds(4), st, a);
+  else hipLaunchKernelGGL((k_attn_av<F16KV, 8>), grid, dim3(256), attention_lds(8), st, a);
 }
 
 template <bool F16KV>
@@ -1767,14 +1181,10 @@ static void launch_av_split_k(const AttnArgs &a, dim3 grid, size_t lds, hipStrea
 
 void launch_attention(const AttnArgs &a0, int B, hipStream_t st) {
   AttnArgs a = a0;
-  // the per-head form for passes of several tokens at long contexts (single-token passes keep the four slice blocks
-  // per head, which stage a quarter of the rows each, wherever their softmax row fits LDS); both give the same bits
-  const bool head = !a.part && a.ctx > (B > 1 ? a.headCtx : a.head1Ctx);
-  // the weighted-sum form: split, the matrix cores, or the lane chains (grouped, per-head or slice form); only the
-  // slice form's LDS grows with the context
+  // the weighted-sum form: split, the matrix cores, or the lane chains
   const bool avmm = !a.part && a.qr && a.mmAvMinB > 0 && B >= a.mmAvMinB;
-  const size_t lds = a.part ? attention_split_lds(a.hd, a.kvF16) : avmm ? 0 : head ? attention_head_lds(a.hd) : attention_lds(a.ctx);
-  ZL_REQUIRE(lds <= ATTN_LDS_MAX, ZL_ERR_UNSUPPORTED, "context too long for the attention kernel");
+  ZL_REQUIRE(a.nchunk == (a.ctx + ATTN_CHUNK - 1) / ATTN_CHUNK && a.cml && (a.nchunk == 1 || (a.rec && a.rcnt)), ZL_ERR_ARG,
+             "attention: chunk records missing");
   ZL_REQUIRE(!a.part || a.nch * ATTN_SPLIT_C >= a.ctx, ZL_ERR_ARG, "attention: split partials below the context");
   ZL_REQUIRE(a.hd == 64 || a.hd == 128 || a.hd == 256, ZL_ERR_UNSUPPORTED, "attention: head_dim must be 64, 128 or 256");
   ZL_REQUIRE(a.sld >= a.ctx, ZL_ERR_ARG, "attention: score stride below the context");
@@ -1807,6 +1217,7 @@ void launch_attention(const AttnArgs &a0, int B, hipStream_t st) {
   ZL_HIP(hipGetLastError());
   if (a.part) {
     const dim3 gv(a.nch, a.nHead, B);
+    const size_t lds = attention_split_lds(a.hd, a.kvF16);
     if (a.kvF16) launch_av_split_k<true>(a, gv, lds, st);
     else launch_av_split_k<false>(a, gv, lds, st);
     ZL_HIP(hipGetLastError());
@@ -1815,54 +1226,21 @@ void launch_attention(const AttnArgs &a0, int B, hipStream_t st) {
     return;
   }
   if (avmm) {
-    // the probabilities of every row, then the weighted sums on the matrix cores, 16 or 32 rows x 32 dimensions per block
-    hipLaunchKernelGGL(k_attn_softmax_rows<true>, dim3(1, a.nHead, B), dim3(SMR_T), 0, st, a);
+    // the probabilities of every row part, then the weighted sums on the matrix cores
+    hipLaunchKernelGGL(k_attn_softmax_rows, dim3(a.nchunk, a.nHead, B), dim3(64), 0, st, a);
     const int nrows = group * B;
-    // 32-row blocks (V staged once for two tiles) where they still give every CU a block (prefill chunks of the 8B
-    // shapes), 16-row blocks otherwise (verify passes, the 0.6B shapes' chunks: 128 rows per KV head)
-    const bool rb32 = (nrows + 31) / 32 * (a.hd / AV_DIMS) * a.nHeadKv >= 256;
     if (a.kvF16) {
-      if (rb32) launch_av_mm_k<true, 32>(a, nrows, st);
-      else launch_av_mm_k<true, 16>(a, nrows, st);
+      if (a.hd == 64) launch_av_mm_k<true, 2>(a, nrows, st);
+      else launch_av_mm_k<true, 4>(a, nrows, st);
     } else {
-      if (rb32) launch_av_mm_k<false, 32>(a, nrows, st);
-      else launch_av_mm_k<false, 16>(a, nrows, st);
+      if (a.hd == 64) launch_av_mm_k<false, 2>(a, nrows, st);
+      else launch_av_mm_k<false, 4>(a, nrows, st);
     }
     ZL_HIP(hipGetLastError());
     return;
   }
-  if (head && B > 1 && a.pinv) {
-    // grouped by KV head: the softmax rows, then each V chunk staged once for a group's rows
-    hipLaunchKernelGGL(k_attn_softmax_rows<false>, dim3(1, a.nHead, B), dim3(SMR_T), 0, st, a);
-    const int nrows = (a.nHead / a.nHeadKv) * B;
-    const dim3 gg(a.hd / AVG_DIMS, a.nHeadKv, (nrows + AVG_ROWS - 1) / AVG_ROWS);
-    // 1024-byte chunks (512 f16 / 256 f32 positions): each chunk's chain is long enough to cover the next chunk's loads
-    if (a.kvF16) launch_av_group_k<true, AV_ROW_BIG>(a, gg, nrows, st);
-    else launch_av_group_k<false, AV_ROW_BIG>(a, gg, nrows, st);
-    ZL_HIP(hipGetLastError());
-    return;
-  }
-  if (head) {
-    switch (a.hd * 2 + a.kvF16) {
-      case 128: launch_av_head_k<64, false>(a, B, st); break;
-      case 129: launch_av_head_k<64, true>(a, B, st); break;
-      case 256: launch_av_head_k<128, false>(a, B, st); break;
-      case 257: launch_av_head_k<128, true>(a, B, st); break;
-    }
-    ZL_HIP(hipGetLastError());
-    return;
-  }
-  dim3 ga(a.hd / AV_DIMS, a.nHead, B);
-  if (a.avmf) {
-    ZL_REQUIRE(a.ctx <= AVM_MAX_CTX, ZL_ERR_ARG, "attention: matrix-core slice form beyond its context");
-    const size_t lm = attention_av_mfma_lds();
-    if (a.kvF16) launch_av_mfma_k<true>(a, ga, lm, st);
-    else launch_av_mfma_k<false>(a, ga, lm, st);
-  } else if (a.kvF16) {
-    launch_av_k<true>(a, ga, lds, st);
-  } else {
-    launch_av_k<false>(a, ga, lds, st);
-  }
+  if (a.kvF16) launch_av_k<true>(a, B, st);
+  else launch_av_k<false>(a, B, st);
   ZL_HIP(hipGetLastError());
 }
 

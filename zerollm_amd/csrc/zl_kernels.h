@@ -133,16 +133,21 @@ struct AttnArgs {
   // position-order f32 chain
   double *part;
   int nch;              // chunks per (token, head) row of part
-  double *pinv;         // [token][head] 1 / sum of a row's exponentials (grouped weighted sum of long multi-token passes)
-  // contexts above headCtx take the per-head / grouped weighted sum for passes of several tokens, contexts above
-  // head1Ctx also for single-token passes (decided once per model when it is loaded: attention_form)
-  int headCtx, head1Ctx;
+  // nchunk = ceil(ctx / ATTN_CHUNK) chunks per row: (max, sum of exponentials) pairs [token][head][chunk], and where a row
+  // may have more than one chunk, their records and arrival counters (zero between launches; null otherwise)
+  int nchunk;
+  double2 *cml;
+  double *rec;
+  uint32_t *rcnt;
   // passes of at least mmMinB tokens take the matrix-core score dots (k_attn_prep + k_attn_scores_mm), which need qr,
   // the pass's normed and rotated query rows [B][nHead][hd] f32
   int mmMinB, mmAvMinB;  // ... and at least mmAvMinB tokens the matrix-core weighted sums (k_attn_av_mm)
   float *qr;
-  int avmf;  // the slice form's chains on the matrix cores (k_attn_av_mfma) instead of the lanes (k_attn_av)
 };
+// Positions per chunk of a row. Rows of up to this many positions are the reference's f32 chain over the whole row; the
+// chunks of longer ones run side by side.
+constexpr int ATTN_CHUNK = 2048;
+constexpr int ATTN_REC_DOUBLES = 18;  // a chunk's record of one 32-dimension slice: max, sum, 32 floats
 constexpr int ATTN_SPLIT_C = 256;  // positions per chunk of the position-split weighted sum
 
 // One Gated DeltaNet layer over the B tokens of a pass (src/model/forward-qwen35.js:45-61). Conv window and delta-rule
@@ -295,13 +300,11 @@ __device__ inline double rms_scale256(const float *xr, int n, double eps, int ti
 }
 
 void launch_attention(const AttnArgs &a, int B, hipStream_t st);
-size_t attention_lds(int ctx);
+// The attention form of a model, decided once at load from its context (the environment overrides ZEROLLM_ATTN_MM_B and
+// ZEROLLM_ATTN_MMAV_B move the thresholds, for tests): mmMinB / mmAvMinB as in AttnArgs.
+struct AttnForm { int mmMinB, mmAvMinB; };
+AttnForm attention_form(int ctx);
 size_t attention_split_lds(int hd, int kvF16);
-// The attention form of a model, decided once at load from its context and head size (the environment overrides
-// ZEROLLM_ATTN_HEAD_CTX and ZEROLLM_ATTN_HEAD1_CTX move the thresholds, for tests): headCtx / head1Ctx as in AttnArgs
-// (INT_MAX: never), split = whether the model needs the position-split weighted sum (its exact chain would not fit).
-struct AttnForm { int headCtx, head1Ctx, mmMinB, mmAvMinB; bool split, avmf; };
-AttnForm attention_form(int ctx, int hd);
 void launch_norm_quant(const float *x, int ldx, int row0, int nrows, const float *w, double eps, int n, int npad,
                        const Act &act, hipStream_t st);
 void launch_embed(const MatView &m, const Step *step, int B, float *x, int ldx, hipStream_t st);

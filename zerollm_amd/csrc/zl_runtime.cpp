@@ -229,10 +229,12 @@ struct zl_model {
   float *x = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *hb = nullptr, *logits = nullptr;
   float *scores = nullptr;  // attention scores [maxBatch][n_head][ctx]
   double *attnPart = nullptr;  // position-split weighted-sum partials (contexts beyond ZEROLLM_ATTN_EXACT_CTX), or null
-  double *attnInv = nullptr;   // [maxBatch][n_head] 1 / sum of exponentials (grouped weighted sum)
   int attnNch = 0;
-  int attnHeadCtx = 0, attnHead1Ctx = 0, attnMmMinB = 0, attnMmAvMinB = 0;  // attention form thresholds, at load
-  bool attnAvmf = false;
+  int attnChunks = 1;            // chunks of the longest row; with more than one, their records (AttnArgs)
+  double *attnRec = nullptr;
+  double2 *attnMl = nullptr;
+  uint32_t *attnCnt = nullptr;
+  int attnMmMinB = 0, attnMmAvMinB = 0;  // attention form thresholds, at load
   float *qr = nullptr;  // the pass's normed and rotated query rows [maxBatch][n_head][head_dim] (matrix-core scores)
   zl::Act act{};    // quantised input of the q/k/v, attention-output and gate/up GEMVs
   zl::Act act2{};   // quantised FFN hidden state (written by the gate/up GEMV, read by the down GEMV)
@@ -403,20 +405,14 @@ static void finish_model(zl_model *m, const float *ropeFreqs) {
   ZL_REQUIRE(c.head_dim == 128 || c.head_dim == 64 || c.head_dim == 256, ZL_ERR_UNSUPPORTED,
              "head_dim " + std::to_string(c.head_dim) + " is not supported (64, 128 or 256)");
   ZL_REQUIRE(c.n_head % c.n_head_kv == 0, ZL_ERR_UNSUPPORTED, "n_head must be a multiple of n_head_kv");
-  // The weighted sum of attention is the reference's position-order f32 chain, bit for bit: for heads of at most 128
-  // dimensions at any context (the per-head form beyond AVH_CTX positions keeps its softmax row in the scores buffer),
-  // for larger heads wherever the softmax row fits the kernel's LDS (about 29900 positions). Longer contexts of larger
-  // heads, or contexts beyond ZEROLLM_ATTN_EXACT_CTX when that is set, take the position-split weighted sum (f64 chunk
-  // sums, online-softmax merge): more accurate than the chain, but not its bits, and on random-weight models the
-  // difference is amplified through the int8 activation quantisation (see the split-path tests).
+  // The weighted sum of attention is the reference's position-order f32 chain, bit for bit, for rows of up to ATTN_CHUNK
+  // positions, and its chunks joined in f64 for longer ones. Models whose context exceeds ZEROLLM_ATTN_EXACT_CTX, when
+  // that is set, take the position-split weighted sum (f64 chunk sums, online-softmax merge) for every row.
   const char *ex = getenv("ZEROLLM_ATTN_EXACT_CTX");
-  const AttnForm form = attention_form(m->ctx, c.head_dim);
-  const bool split = form.split || (ex && m->ctx > atoi(ex));
-  m->attnHeadCtx = form.headCtx;
-  m->attnHead1Ctx = form.head1Ctx;
+  const AttnForm form = attention_form(m->ctx);
+  const bool split = ex && m->ctx > atoi(ex);
   m->attnMmMinB = form.mmMinB;
   m->attnMmAvMinB = form.mmAvMinB;
-  m->attnAvmf = form.avmf;
   const int half = c.n_rot / 2;
   // RoPE tables exactly as ropeTables (src/compute/ref-kernels.js:329-342), in f64 on the host, stored f32
   std::vector<float> cs((size_t)m->ctx * half), sn((size_t)m->ctx * half);
@@ -474,7 +470,14 @@ static void finish_model(zl_model *m, const float *ropeFreqs) {
   m->logits = (float *)m->ar.alloc((size_t)m->logitsBatch * c.vocab * 4);
   m->scores = (float *)m->ar.alloc((size_t)B * c.n_head * m->ctx * 4);
   m->qr = (float *)m->ar.alloc((size_t)B * c.n_head * c.head_dim * 4);
-  m->attnInv = (double *)m->ar.alloc((size_t)B * c.n_head * 8);
+  m->attnChunks = (m->ctx + ATTN_CHUNK - 1) / ATTN_CHUNK;
+  const size_t rows = (size_t)B * c.n_head, ns = c.head_dim / 32;
+  m->attnMl = (double2 *)m->ar.alloc(rows * m->attnChunks * sizeof(double2));
+  if (m->attnChunks > 1) {
+    m->attnRec = (double *)m->ar.alloc(rows * ns * m->attnChunks * ATTN_REC_DOUBLES * 8);
+    m->attnCnt = (uint32_t *)m->ar.alloc(rows * ns * 4);
+    zero_now(m->attnCnt, rows * ns * 4);
+  }
   if (split) {
     m->attnNch = (m->ctx + ATTN_SPLIT_C - 1) / ATTN_SPLIT_C;
     m->attnPart = (double *)m->ar.alloc((size_t)B * c.n_head * m->attnNch * (c.head_dim + 2) * 8);
@@ -713,10 +716,9 @@ static void enqueue_forward(zl_model *m, int B, int want) {
       aa.step = m->dstep; aa.out = m->act.f; aa.ldo = m->act.ld; aa.act = m->act;
       aa.qhs = m->hybrid ? 2 * c.head_dim : c.head_dim;
       aa.gate = m->hybrid ? m->q + c.head_dim : nullptr;
-      aa.part = m->attnPart; aa.nch = m->attnNch; aa.pinv = m->attnInv;
-      aa.headCtx = m->attnHeadCtx; aa.head1Ctx = m->attnHead1Ctx;
+      aa.part = m->attnPart; aa.nch = m->attnNch;
+      aa.nchunk = m->attnChunks; aa.rec = m->attnRec; aa.cml = m->attnMl; aa.rcnt = m->attnCnt;
       aa.mmMinB = m->attnMmMinB; aa.mmAvMinB = m->attnMmAvMinB; aa.qr = m->qr;
-      aa.avmf = m->attnAvmf ? 1 : 0;
       // a single-token Q8_0 attn_output GEMV quantises the f32 head outputs itself: the attention writes them alone
       if (rg_path({&L.wo}, B)) aa.act.q = nullptr;
       launch_attention(aa, B, m->st);
