@@ -3,8 +3,8 @@
 // each weight tile once for every token of a chunk (src/compute/wasm/kernels.js:127-240,
 // src/compute/wasm/kquant-kernels.js:337-504); the int8 block dots run on the matrix cores and the f64 block terms are
 // the reference's (src/compute/ref-kernels.js:132-277), per (row, token) in exactly the order of k_gemv_tiles
-// (zl_gemv.h): the same slabs per wave, slab by slab, block 0 then block 1 (Q6_K: its four 16-value groups in order),
-// the same halving tree over the waves and the same K parts. A token therefore gets the same bits whatever the size of
+// (zl_gemv.h): the same slabs per wave, slab by slab, block 0 then block 1 (Q6_K: both blocks in one term), the same
+// halving tree over the waves and the same K parts. A token therefore gets the same bits whatever the size of
 // the pass it is in (1..9 tokens through the GEMV kernels, 10..64 here).
 //
 // Mapping. The workgroup is the GEMV's (K part, 64-row tile) with its W waves (gate/up pairs: W / 2 per matrix); wave
@@ -18,7 +18,7 @@
 //
 // Accumulators. Lane l holds acc[j][u][v] = the running f64 sum of row 16 j + l mod 16 (j = 0..3 row groups of the
 // tile) and token 16 u + 4 g + v (u = 0..U-1 token groups): 16 U doubles. Its f64 factors (Q4_K/Q5_K d*sc and dmin*mn
-// of the two blocks, Q6_K d*scale of the four groups, Q8_0 the two block scales) are formed per slab for its four rows.
+// of the two blocks, Q6_K d, Q8_0 the two block scales) are formed per slab for its four rows.
 //
 // Activations. Per round i (slabs s0 + WH i + wl of every wave wl of a matrix) the workgroup stages the int8 values and
 // block records of those WH slabs for all tokens in LDS ([wl][token][64 B], then [wl][token][32 B]), double-buffered:
@@ -76,10 +76,12 @@ __device__ __forceinline__ void gm_load(const Rsrc &R, int ts, int sbi, int n16,
 }
 
 // B operands (the 16 values of quarter g of the lane's four rows, as int8) and the exact f64 factors of the rows:
-//   Q8_0 f = {d0, d1};  Q4_K/Q5_K f = {d*sc0, d*sc1, dmin*mn0, dmin*mn1};  Q6_K f = {d*scale of groups 0..3}.
+//   Q8_0 f = {d0, d1};  Q4_K/Q5_K f = {d*sc0, d*sc1, dmin*mn0, dmin*mn1};  Q6_K f = {d} and the four group scales, a byte each, in gs.
 // The products are those k_gemv_tiles forms (zl_gemv.h unpack), so every term below is bit for bit its term.
 template <int FMT>
-__device__ __forceinline__ void gm_unpack(const GmRaw<FMT> &o, int g, gm_i32x4 B[4], double f[4][4]) {
+constexpr int gm_nf = FMT == T_Q6_K ? 1 : FMT == T_Q8_0 ? 2 : 4;
+template <int FMT>
+__device__ __forceinline__ void gm_unpack(const GmRaw<FMT> &o, int g, gm_i32x4 B[4], double f[4][gm_nf<FMT>], uint32_t gs[4]) {
   #pragma unroll
   for (int j = 0; j < 4; j++) {
     #pragma unroll
@@ -90,7 +92,8 @@ __device__ __forceinline__ void gm_unpack(const GmRaw<FMT> &o, int g, gm_i32x4 B
         // bit 16 (g & 1) + 4 k + i of the word is the fifth bit of byte i of this dword
         w |= ((((o.h[j][0] >> (16 * (g & 1) + 4 * k)) & 15u) * 0x00204081u) & 0x01010101u) << 4;
       }
-      if constexpr (FMT == T_Q6_K) w |= ((o.h[j][k] >> (2 * g)) & 0x03030303u) << 4;  // top two bits of value 16 g + byte
+      // top two bits of value 16 g + byte; the codes 0..63 become the signed values -32..31 (no carry between the bytes)
+      if constexpr (FMT == T_Q6_K) w = ((w | (((o.h[j][k] >> (2 * g)) & 0x03030303u) << 4)) + 0x60606060u) ^ 0x80808080u;
       B[j][k] = (int)w;
     }
     const double d0 = (double)h2f((uint16_t)(o.dw[j] & 0xffff)), d1 = (double)h2f((uint16_t)(o.dw[j] >> 16));
@@ -100,10 +103,10 @@ __device__ __forceinline__ void gm_unpack(const GmRaw<FMT> &o, int g, gm_i32x4 B
       f[j][2] = d1 * (double)((o.sc[j] >> 16) & 0xff);
       f[j][3] = d1 * (double)((o.sc[j] >> 24) & 0xff);
     } else if constexpr (FMT == T_Q6_K) {
-      #pragma unroll
-      for (int k = 0; k < 4; k++) f[j][k] = d0 * (double)(int8_t)((o.sc[j] >> (8 * k)) & 0xff);
+      f[j][0] = d0;
+      gs[j] = o.sc[j];
     } else {
-      f[j][0] = d0; f[j][1] = d1; f[j][2] = 0.0; f[j][3] = 0.0;
+      f[j][0] = d0; f[j][1] = d1;
     }
   }
 }
@@ -113,12 +116,11 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
   extern __shared__ __align__(16) uint8_t xl[];
   constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1;
   constexpr int WH = NR == 2 ? W / 2 : W;                 // waves per matrix
-  constexpr int DEPTH = U <= 2 ? 2 : 1;                   // slabs of weights in flight beyond the one computed
+  constexpr int DEPTH = U <= 2 && FMT != T_Q6_K ? 2 : 1;                   // slabs of weights in flight beyond the one computed
   constexpr int MP = 16 * U;                               // staged tokens (the last group padded with the last token)
   constexpr int RB = WH * MP * 96;                         // LDS bytes of one round: values, then records
   constexpr int CH = RB / 1024;                            // 1 KB staging chunks per round
   constexpr int SPW = (CH + W - 1) / W;                    // staging loads per wave and round
-  constexpr int NG = FMT == T_Q6_K ? 4 : 2;                // dots per slab: 16-value groups or 32-value blocks
   static_assert(RB % 1024 == 0, "whole staging chunks");
   const int kp = blockIdx.x, tile = blockIdx.y;
   // token group z of the launch's G (blockIdx.z): tokens tb .. tb + Ml - 1, staged as rows 0 .. MP - 1. A (row, token)
@@ -196,15 +198,17 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
   // one round: the wave's slab r (weights in `slot`, activations in buffer r & 1), the next round's activations staged
   auto round = [&](int r, GmRaw<FMT> &slot) {
     gm_i32x4 B[4];
-    double f[4][4];
-    gm_unpack<FMT>(slot, g, B, f);
+    double f[4][gm_nf<FMT>];
+    uint32_t gs[4];
+    gm_unpack<FMT>(slot, g, B, f, gs);
     // the operands are formed here, before the slot is reloaded (not sunk to their uses below), so the reload can
     // land in the slot's own registers
     #pragma unroll
     for (int j = 0; j < 4; j++) {
       asm volatile("" : "+v"(B[j]));
       #pragma unroll
-      for (int k = 0; k < (FMT == T_Q8_0 ? 2 : 4); k++) asm volatile("" : "+v"(f[j][k]));
+      for (int k = 0; k < gm_nf<FMT>; k++) asm volatile("" : "+v"(f[j][k]));
+      if constexpr (FMT == T_Q6_K) asm volatile("" : "+v"(gs[j]));
     }
     u32x4 sg[SPW];
     __builtin_amdgcn_sched_barrier(0);  // issue order: the staging loads, then the weights (the stores below wait for
@@ -218,28 +222,60 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
       #pragma unroll
       for (int u = 0; u < U; u++) {
         const uint4 av = *(const uint4 *)(vals + (16 * u + n16) * 64 + 16 * g);
-        #pragma unroll
-        for (int b = 0; b < NG; b++) {
-          const bool on = (NG == 2 ? (g >> 1) : g) == b;  // this lane's quarter lies in block / group b
-          const gm_i32x4 A = on ? gm_i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w} : gm_i32x4{0, 0, 0, 0};
-          gm_i32x4 D[4];
+        if constexpr (FMT == T_Q6_K) {
+          // the two groups of a block join in integers, the slab's two blocks in one product with d: 9 VALU instructions
+          // per (row, token) and slab where a term per group took 16 (4096 x 12288 at 64 tokens 73.8 -> 48.9 us, bound by
+          // their issue). One slab ahead in flight: two (40 registers each) spilled. Row group j's sums are formed while the matrix cores run j + 1's dots (the
+          // barriers keep the scheduler from holding all four row groups' dots in registers at once)
+          gm_i32x4 A[4], D[2][4];
+          double xd[2][4];
           #pragma unroll
-          for (int j = 0; j < 4; j++) D[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
-          const int blk = NG == 2 ? b : b >> 1;
+          for (int b = 0; b < 4; b++) A[b] = g == b ? gm_i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w} : gm_i32x4{0, 0, 0, 0};
           #pragma unroll
-          for (int v = 0; v < 4; v++) {
-            const uint4 rc = *(const uint4 *)(recs + (16 * u + 4 * g + v) * 32 + blk * 16);
-            const double xd = dbl(rc.x, rc.y);
+          for (int v = 0; v < 4; v++)
             #pragma unroll
-            for (int j = 0; j < 4; j++) {
-              double &s = acc[j][u][v];
-              if constexpr (FMT == T_Q6_K) {
-                const int c = D[j][v] - (int)((b & 1) ? rc.w : rc.z);  // dot minus 32 x the group's activation sum
-                s = fma(f[j][b] * (double)c, xd, s);
-              } else if constexpr (FMT == T_Q8_0) {
-                s = fma((double)D[j][v] * f[j][b], xd, s);
-              } else {
-                s = fma(xd, fma(f[j][b], (double)D[j][v], -(f[j][2 + b] * dbl(rc.z, rc.w))), s);
+            for (int blk = 0; blk < 2; blk++) xd[blk][v] = *(const double *)(recs + (16 * u + 4 * g + v) * 32 + blk * 16);
+          auto dots = [&](int j) {
+            #pragma unroll
+            for (int b = 0; b < 4; b++) D[j & 1][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[b], B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
+          };
+          dots(0);
+          #pragma unroll
+          for (int j = 0; j < 4; j++) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (j < 3) dots(j + 1);
+            const gm_i32x4 (&d)[4] = D[j & 1];
+            int sc[4];
+            #pragma unroll
+            for (int k = 0; k < 4; k++) sc[k] = (int)(int8_t)(gs[j] >> (8 * k));
+            #pragma unroll
+            for (int v = 0; v < 4; v++) {
+              const int e0 = __mul24(d[0][v], sc[0]) + __mul24(d[1][v], sc[1]);
+              const int e1 = __mul24(d[2][v], sc[2]) + __mul24(d[3][v], sc[3]);
+              acc[j][u][v] = fma(f[j][0], fma(xd[1][v], (double)e1, xd[0][v] * (double)e0), acc[j][u][v]);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        } else {
+          #pragma unroll
+          for (int b = 0; b < 2; b++) {
+            const bool on = (g >> 1) == b;  // this lane's quarter lies in block b
+            const gm_i32x4 A = on ? gm_i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w} : gm_i32x4{0, 0, 0, 0};
+            gm_i32x4 D[4];
+            #pragma unroll
+            for (int j = 0; j < 4; j++) D[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
+            #pragma unroll
+            for (int v = 0; v < 4; v++) {
+              const uint4 rc = *(const uint4 *)(recs + (16 * u + 4 * g + v) * 32 + b * 16);
+              const double xd = dbl(rc.x, rc.y);
+              #pragma unroll
+              for (int j = 0; j < 4; j++) {
+                double &s = acc[j][u][v];
+                if constexpr (FMT == T_Q8_0) {
+                  s = fma((double)D[j][v] * f[j][b], xd, s);
+                } else {
+                  s = fma(xd, fma(f[j][b], (double)D[j][v], -(f[j][2 + b] * dbl(rc.z, rc.w))), s);
+                }
               }
             }
           }

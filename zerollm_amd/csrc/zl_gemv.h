@@ -79,11 +79,12 @@ __device__ inline void raw_load(const Rsrc &R, int ts, int sbi, int lane, bool v
 
 // Token-independent data of one (row, slab): int8 lanes of the 64 values (words 0-7 block 0 = values 0-31, words
 // 8-15 block 1; unsigned codes for the offset formats) and exact f64 factors per 32-value block h:
-//   Q8_0/Q4_0/Q5_0: fa = d;  Q4_K/Q5_K: fa = d*sc, fb = dmin*mn;  Q6_K: fa, fb = d*scale of the block's 16-groups
+//   Q8_0/Q4_0/Q5_0: fa = d;  Q4_K/Q5_K: fa = d*sc, fb = dmin*mn;  Q6_K: fa[0] = d (and the group scales as integers)
 template <int FMT>
 struct Unp {
   uint32_t w[16];
   double fa[2], fb[2];
+  int gs[FMT == T_Q6_K ? 4 : 1];
 };
 
 template <int FMT>
@@ -124,11 +125,9 @@ __device__ inline void unpack(const Raw<FMT> &o, Unp<FMT> &u) {
       u.fb[h] = d1 * (double)((o.sc >> (16 + 8 * h)) & 0xff);
     }
   } else if constexpr (FMT == T_Q6_K) {
+    u.fa[0] = d0;
     #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      u.fa[h] = d0 * (double)(int8_t)((o.sc >> (16 * h)) & 0xff);
-      u.fb[h] = d0 * (double)(int8_t)((o.sc >> (16 * h + 8)) & 0xff);
-    }
+    for (int k = 0; k < 4; k++) u.gs[k] = (int)(int8_t)((o.sc >> (8 * k)) & 0xff);
   } else {
     u.fa[0] = d0; u.fa[1] = d1;
     u.fb[0] = 0.0; u.fb[1] = 0.0;
@@ -179,17 +178,18 @@ __device__ inline void slab_dots(uint32_t xw, const uint32_t *w, int c[4]) {
 // arithmetic up to where f64 rounds:
 //   Q8_0 (s*d)*xd;  Q4_0/Q5_0 ((s - 8|16 sum) * d) * xd;  Q4_K/Q5_K xd*(d*sc*s - dmin*mn*sum);
 //   Q6_K per 16-group (d*scale*(s - 32 sum)) * xd.  The products before the last one are exact; the last multiply
-//   and the accumulation are one fma. The integer dots are exact in any order.
+//   and the accumulation are one fma. The integer dots are exact in any order. Q6_K's scales and the two groups of a
+//   block meet in integers, e = scale (s - 32 sum) + scale' (s' - 32 sum') with |e| < 2^24, and the slab adds
+//   d (xd0 e0 + xd1 e1): xd e is exact, so the slab has two roundings where a term per group has four, and 9 VALU
+//   instructions where that has 16 (4096 x 12288 at 5 tokens 16.4 -> 15.6 us; the head at 1 token, bound by HBM, 90.3).
 template <int FMT>
 __device__ inline double slab_terms(const Unp<FMT> &u, uint32_t xw, const u32x4 &R0, const u32x4 &R1, double acc) {
   const double xd0 = dbl(R0[0], R0[1]), xd1 = dbl(R1[0], R1[1]);
   if constexpr (FMT == T_Q6_K) {
     int c[4] = {-(int)R0[2], -(int)R0[3], -(int)R1[2], -(int)R1[3]};
     slab_dots<1>(xw, u.w, c);
-    acc = fma(u.fa[0] * (double)c[0], xd0, acc);
-    acc = fma(u.fb[0] * (double)c[1], xd0, acc);
-    acc = fma(u.fa[1] * (double)c[2], xd1, acc);
-    return fma(u.fb[1] * (double)c[3], xd1, acc);
+    const int e0 = __mul24(c[0], u.gs[0]) + __mul24(c[1], u.gs[1]), e1 = __mul24(c[2], u.gs[2]) + __mul24(c[3], u.gs[3]);
+    return fma(u.fa[0], fma(xd1, (double)e1, xd0 * (double)e0), acc);
   } else {
     constexpr int CI = FMT == T_Q4_0 ? 2 : 3;  // Q4_0 / Q5_0: the block starts at -8 | -16 x its activation sum
     const bool off = FMT == T_Q4_0 || FMT == T_Q5_0;
