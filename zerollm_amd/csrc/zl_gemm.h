@@ -31,6 +31,7 @@
 namespace zl {
 
 constexpr int GEMM_MAX_M = 64;   // tokens per launch at most (four groups of 16)
+constexpr int gemm_ub(int U) { return U < 2 ? U : 2; }  // token groups of a launch whose sums lie in LDS together
 
 typedef int gm_i32x4 __attribute__((ext_vector_type(4)));
 
@@ -292,14 +293,21 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
     if constexpr (DEPTH == 2) round(r + 1, ring[1]);
   }
 
-  // ---- per token group: each wave parks its sums, then the wave of token t adds that token's sums over the waves of
-  // each matrix in the order of a halving tree (as k_gemv_tiles) and runs the epilogue (or stores a K part)
-  double *red = (double *)xl;  // [W][4 j][4 v][64 lanes] of one token group
+  // ---- every wave parks its sums, then wave w adds those of tokens w, w + W, ... over the waves of each matrix in the
+  // order of a halving tree (as k_gemv_tiles) and runs the epilogue (or stores a K part). A wave's TPW tokens go through
+  // each step together, so its loads and chains overlap: token by token the hand-off's loads alone were TPW round trips.
+  constexpr int TPW = MP / W;
+  double *red = (double *)xl;  // [token group of a batch][W][4 j][4 v][64 lanes]
   const int PW = NR * MP * 64;  // doubles per K part
   double *pp = a.part + (((long)tile * G + zg) * ks + kp) * PW;
   const int row = lt * 64 + lane;
   const bool live = row < rows;
-  auto epilogue = [&](int t, double g0, double u0) {
+  float rres[TPW];  // the residual values, requested ahead of the reduction
+  if constexpr (EPI == EPI_RESID) {
+    #pragma unroll
+    for (int k = 0; k < TPW; k++) rres[k] = a.resid[(long)(tb + min(wave + W * k, M - 1)) * a.ldr + min(row, rows - 1)];
+  }
+  auto epilogue = [&](int k, int t, double g0, double u0) {
     if constexpr (EPI == EPI_SWIGLU) {
       const double gv = (double)(float)g0, uu = (double)(float)u0;
       const float hv = live ? (float)(gv / (1.0 + exp(-gv)) * uu) : 0.f;  // src/compute/ref-kernels.js:322
@@ -307,10 +315,7 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
       if (a.qout.q) quant_block32(hv, row, a.qout, t);
     } else if constexpr (EPI == EPI_RESID) {
       const double y = (double)(float)g0;
-      if (live) {
-        float *o = a.resid + (long)t * a.ldr + row;
-        *o = (float)((double)*o + y);
-      }
+      if (live) a.resid[(long)t * a.ldr + row] = (float)((double)rres[k] + y);
     } else {
       const float y = (float)g0;
       if (live) {
@@ -319,78 +324,87 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
       }
     }
   };
+  double sums[TPW][NR];
+  constexpr int UB = gemm_ub(U);  // token groups parked at a time
   #pragma unroll
-  for (int u = 0; u < U; u++) {
+  for (int u0 = 0; u0 < U; u0 += UB) {
+    if (u0 > 0) __syncthreads();  // the previous groups' sums have been read
     #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int u = u0; u < u0 + UB && u < U; u++)
       #pragma unroll
-      for (int v = 0; v < 4; v++) red[((wave * 4 + j) * 4 + v) * 64 + lane] = acc[j][u][v];
+      for (int j = 0; j < 4; j++)
+        #pragma unroll
+        for (int v = 0; v < 4; v++) red[((((u - u0) * W + wave) * 4 + j) * 4 + v) * 64 + lane] = acc[j][u][v];
     __syncthreads();
-    for (int tt = wave; tt < 16; tt += W) {
-      const int t = 16 * u + tt;
-      if (t >= M) break;
+    #pragma unroll
+    for (int k = u0 * 16 / W; k < TPW && k < (u0 + UB) * 16 / W; k++) {
+      const int t = wave + W * k, tt = t & 15;  // (tokens past M: sums of padding, not stored)
       // (row = lane, token t): row group lane / 16 in lane 16 (tt / 4) + lane mod 16, slot v = tt mod 4
       const int src = 16 * (tt >> 2) + n16, jv = (lane >> 4) * 4 + (tt & 3);
-      double sums[NR];
       #pragma unroll
       for (int r = 0; r < NR; r++) {
-        double vv[8];
+        double vv[WH];
         #pragma unroll
-        for (int w = 0; w < 8; w++) vv[w] = red[(((r * WH + min(w, WH - 1)) * 16) + jv) * 64 + src];
+        for (int w = 0; w < WH; w++) vv[w] = red[(((((t >> 4) - u0) * W + r * WH + w) * 16) + jv) * 64 + src];
         #pragma unroll
-        for (int half = 4; half >= 1; half >>= 1)
-          if (2 * half <= WH) {
-            #pragma unroll
-            for (int w = 0; w < half; w++) vv[w] = vv[w] + vv[w + half];
-          }
-        sums[r] = vv[0];
-      }
-      if (ks == 1) {
-        epilogue(tb + t, sums[0], sums[NR - 1]);
-      } else {
-        #pragma unroll
-        for (int r = 0; r < NR; r++) __hip_atomic_store(pp + (r * MP + t) * 64 + lane, sums[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int half = WH / 2; half >= 1; half >>= 1)
+          #pragma unroll
+          for (int w = 0; w < half; w++) vv[w] = vv[w] + vv[w + half];
+        sums[k][r] = vv[0];
       }
     }
-    __syncthreads();
   }
-  if (ks == 1) return;
-
-  // ---- K parts: the last part of the tile to arrive adds all parts' sums in part order (as k_gemv_tiles)
-  __shared__ uint32_t last;
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores are complete
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __syncthreads();
-  uint32_t *cnt = a.cnt + (long)tile * G + zg;
-  if (threadIdx.x == 0) last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(ks - 1);
-  __syncthreads();
-  if (!last) return;
-  if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  for (int t = wave; t < M; t += W) {
-    double sums[NR];
+  if (ks > 1) {
+    // ---- K parts: the last part of the tile to arrive adds all parts' sums in part order (as k_gemv_tiles)
+    __shared__ uint32_t last;
     #pragma unroll
-    for (int r = 0; r < NR; r++) {
-      const double *pt = a.part + ((long)tile * G + zg) * ks * PW + (r * MP + t) * 64 + lane;
-      constexpr int KSMAX = 8;  // the parts' loads of one sum are issued together
-      double pv[KSMAX];
+    for (int k = 0; k < TPW; k++)
+      if (wave + W * k < M) {
+        #pragma unroll
+        for (int r = 0; r < NR; r++)
+          __hip_atomic_store(pp + (r * MP + wave + W * k) * 64 + lane, sums[k][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores are complete
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __syncthreads();
+    uint32_t *cnt = a.cnt + (long)tile * G + zg;
+    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(ks - 1);
+    __syncthreads();
+    if (!last) return;
+    if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double *p0 = a.part + ((long)tile * G + zg) * ks * PW + lane;
+    for (int q0 = 0; q0 < ks; q0 += 4) {  // four parts' loads of all the wave's sums are issued together
+      double pv[TPW][NR][4];
       #pragma unroll
-      for (int k = 0; k < KSMAX; k++) pv[k] = __hip_atomic_load(pt + (long)min(k, ks - 1) * PW, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      double v = pv[0];
+      for (int k = 0; k < TPW; k++)
+        #pragma unroll
+        for (int r = 0; r < NR; r++)
+          #pragma unroll
+          for (int q = 0; q < 4; q++)
+            pv[k][r][q] = __hip_atomic_load(p0 + (long)min(q0 + q, ks - 1) * PW + (r * MP + min(wave + W * k, M - 1)) * 64,
+                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       #pragma unroll
-      for (int k = 1; k < KSMAX; k++)
-        if (k < ks) v += pv[k];
-      sums[r] = v;
+      for (int k = 0; k < TPW; k++)
+        #pragma unroll
+        for (int r = 0; r < NR; r++)
+          #pragma unroll
+          for (int q = 0; q < 4; q++) {
+            if (q0 + q == 0) sums[k][r] = pv[k][r][0];
+            else if (q0 + q < ks) sums[k][r] += pv[k][r][q];
+          }
     }
-    epilogue(tb + t, sums[0], sums[NR - 1]);
   }
+  #pragma unroll
+  for (int k = 0; k < TPW; k++)
+    if (wave + W * k < M) epilogue(k, tb + wave + W * k, sums[k][0], sums[k][NR - 1]);
 #undef ZL_SEG
 }
 
-// LDS bytes of a launch: two staging rounds, or the sums of one token group.
+// LDS bytes of a launch: two staging rounds, or the waves' sums.
 template <int W, int U>
 constexpr size_t gemm_lds(bool swiglu) {
-  return std::max((size_t)2 * (swiglu ? W / 2 : W) * 16 * U * 96, (size_t)W * 16 * 64 * 8);
+  return std::max((size_t)2 * (swiglu ? W / 2 : W) * 16 * U * 96, (size_t)gemm_ub(U) * W * 16 * 64 * 8);
 }
 
 template <int FMT, int EPI, int W, int U>
@@ -398,7 +412,7 @@ inline void launch_gemm_k(const GemvArgs &a, int G, hipStream_t st) {
   const size_t lds = gemm_lds<W, U>(EPI == EPI_SWIGLU);
   static bool done = false;
   if (!done) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_gemm<FMT, EPI, W, U>, hipFuncAttributeMaxDynamicSharedMemorySize, 112 * 1024));
+    ZL_HIP(hipFuncSetAttribute((const void *)k_gemm<FMT, EPI, W, U>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     done = true;
   }
   hipLaunchKernelGGL((k_gemm<FMT, EPI, W, U>), dim3((unsigned)a.ks, (unsigned)a.ntiles, (unsigned)G), dim3(W * 64), lds, st, a);
