@@ -7,7 +7,8 @@
 // halving tree over the waves and the same K parts. A token therefore gets the same bits whatever the size of
 // the pass it is in (1..9 tokens through the GEMV kernels, 10..64 here).
 //
-// Mapping. The workgroup is the GEMV's (K part, 64-row tile) with its W waves (gate/up pairs: W / 2 per matrix); wave
+// Mapping (tiles; in 96-row blocks a wave takes six row groups, three at a time). The workgroup is the GEMV's (K part,
+// 64-row tile) with its W waves (gate/up pairs: W / 2 per matrix); wave
 // wl of a matrix walks slabs s0 + wl + WH i as in k_gemv_tiles, but for every token of the launch at once. One
 // v_mfma_i32_16x16x64_i8 multiplies A (16 tokens: lane l supplies token l mod 16's values of the slab's value quarter
 // g = l / 16) by B (16 rows of the tile: lane l supplies row l mod 16's values of quarter g) into D[token][row]; lane l
@@ -31,60 +32,65 @@
 namespace zl {
 
 constexpr int GEMM_MAX_M = 64;   // tokens per launch at most (four groups of 16)
-constexpr int gemm_ub(int U) { return U < 2 ? U : 2; }  // token groups of a launch whose sums lie in LDS together
+// token groups of a launch whose sums lie in LDS together (96-row blocks: 96 KB each)
+constexpr int gemm_ub(int U, int RG) { return U < 2 || RG == 6 ? 1 : 2; }
 
 typedef int gm_i32x4 __attribute__((ext_vector_type(4)));
 
-// One slab of one lane as loaded: for each row group j (row 16 j + lane mod 16 of the tile) the 16 bytes of value
+// One slab of one lane as loaded: for each of J row groups j (lane mod 16 = row of the group) the 16 bytes of value
 // quarter g's plane part, the extra-bit word(s), the scale-code word and the super-block / block scale word.
-template <int FMT>
+template <int FMT, int J>
 struct GmRaw {
   static constexpr int HW = FMT == T_Q6_K ? 4 : FMT == T_Q5_K ? 1 : 0;
-  uint32_t q[4][4];
-  uint32_t h[4][HW > 0 ? HW : 1];
-  uint32_t sc[4];
-  uint32_t dw[4];
+  uint32_t q[J][4];
+  uint32_t h[J][HW > 0 ? HW : 1];
+  uint32_t sc[J];
+  uint32_t dw[J];
 };
 
-template <int FMT>
-__device__ __forceinline__ void gm_load(const Rsrc &R, int ts, int sbi, int n16, int g, bool valid, GmRaw<FMT> &o) {
+// Slab s of the row groups q0 .. q0 + J - 1 (16 rows each) of a matrix of nq row groups; groups past the last one read
+// it again (their sums are not stored). J = 4: one whole tile, q0 a multiple of 4.
+template <int FMT, int J>
+__device__ __forceinline__ void gm_load(const Rsrc &R, int q0, int nq, int s, int nslab, int n16, int g, bool valid, GmRaw<FMT, J> &o) {
   const int oob = valid ? 0 : 0x40000000;
-  ts = valid ? ts : 0;
-  sbi = valid ? sbi : 0;
+  s = valid ? s : 0;
   #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int r = 16 * j + n16;
+  for (int j = 0; j < J; j++) {
+    const int q = J == 4 ? q0 : min(q0 + j, nq - 1);
+    const int ts = (q >> 2) * nslab + s, sbi = (q >> 2) * (nslab >> 2) + (s >> 2);
+    const int r = (J == 4 ? 16 * j : 0) + n16;  // row of the tile, in the lane's offset
+    const int rs = J == 4 ? 0 : 16 * (q & 3);   // and what the wave's offset adds to it
     u32x4 v;
     if constexpr (FMT == T_Q8_0) {
       // part g (values 16 g .. 16 g + 15) of row r is 16-byte unit 64 g + r of the tile-slab
-      v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(R.qs, oob + (g * 64 + r) * 16, ts * 4096, 0));
+      v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(R.qs, oob + (g * 64 + r) * 16, ts * 4096 + rs * 16, 0));
     } else {
       // 4-bit planes: part (g & 1) holds the low nibbles of values 16 (g & 1) .. + 15 and the high nibbles 32 later
-      v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(R.qs, oob + ((g & 1) * 64 + r) * 16, ts * 2048, 0));
+      v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(R.qs, oob + ((g & 1) * 64 + r) * 16, ts * 2048 + rs * 16, 0));
     }
     o.q[j][0] = v.x; o.q[j][1] = v.y; o.q[j][2] = v.z; o.q[j][3] = v.w;
     if constexpr (FMT == T_Q6_K) {
-      const u32x4 x = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(R.qx, oob + r * 16, ts * 1024, 0));
+      const u32x4 x = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(R.qx, oob + r * 16, ts * 1024 + rs * 16, 0));
       o.h[j][0] = x.x; o.h[j][1] = x.y; o.h[j][2] = x.z; o.h[j][3] = x.w;
     } else if constexpr (FMT == T_Q5_K) {
-      o.h[j][0] = __builtin_amdgcn_raw_buffer_load_b32(R.qx, oob + r * 8 + 4 * (g >> 1), ts * 512, 0);
+      o.h[j][0] = __builtin_amdgcn_raw_buffer_load_b32(R.qx, oob + r * 8 + 4 * (g >> 1), ts * 512 + rs * 8, 0);
     }
-    if constexpr (FMT == T_Q4_K || FMT == T_Q5_K || FMT == T_Q6_K) o.sc[j] = __builtin_amdgcn_raw_buffer_load_b32(R.sc, oob + r * 4, ts * 256, 0);
-    if constexpr (FMT == T_Q4_K || FMT == T_Q5_K) o.dw[j] = __builtin_amdgcn_raw_buffer_load_b32(R.dd, oob + r * 4, sbi * 256, 0);
-    else if constexpr (FMT == T_Q6_K) o.dw[j] = __builtin_amdgcn_raw_buffer_load_b16(R.dd, oob + r * 2, sbi * 128, 0);
-    else o.dw[j] = __builtin_amdgcn_raw_buffer_load_b32(R.dd, oob + r * 4, ts * 256, 0);
+    if constexpr (FMT == T_Q4_K || FMT == T_Q5_K || FMT == T_Q6_K) o.sc[j] = __builtin_amdgcn_raw_buffer_load_b32(R.sc, oob + r * 4, ts * 256 + rs * 4, 0);
+    if constexpr (FMT == T_Q4_K || FMT == T_Q5_K) o.dw[j] = __builtin_amdgcn_raw_buffer_load_b32(R.dd, oob + r * 4, sbi * 256 + rs * 4, 0);
+    else if constexpr (FMT == T_Q6_K) o.dw[j] = __builtin_amdgcn_raw_buffer_load_b16(R.dd, oob + r * 2, sbi * 128 + rs * 2, 0);
+    else o.dw[j] = __builtin_amdgcn_raw_buffer_load_b32(R.dd, oob + r * 4, ts * 256 + rs * 4, 0);
   }
 }
 
-// B operands (the 16 values of quarter g of the lane's four rows, as int8) and the exact f64 factors of the rows:
+// B operands (the 16 values of quarter g of the lane's J rows, as int8) and the exact f64 factors of the rows:
 //   Q8_0 f = {d0, d1};  Q4_K/Q5_K f = {d*sc0, d*sc1, dmin*mn0, dmin*mn1};  Q6_K f = {d} and the four group scales, a byte each, in gs.
 // The products are those k_gemv_tiles forms (zl_gemv.h unpack), so every term below is bit for bit its term.
 template <int FMT>
 constexpr int gm_nf = FMT == T_Q6_K ? 1 : FMT == T_Q8_0 ? 2 : 4;
-template <int FMT>
-__device__ __forceinline__ void gm_unpack(const GmRaw<FMT> &o, int g, gm_i32x4 B[4], double f[4][gm_nf<FMT>], uint32_t gs[4]) {
+template <int FMT, int J>
+__device__ __forceinline__ void gm_unpack(const GmRaw<FMT, J> &o, int g, gm_i32x4 B[J], double f[J][gm_nf<FMT>], uint32_t gs[J]) {
   #pragma unroll
-  for (int j = 0; j < 4; j++) {
+  for (int j = 0; j < J; j++) {
     #pragma unroll
     for (int k = 0; k < 4; k++) {
       uint32_t w = o.q[j][k];
@@ -112,18 +118,22 @@ __device__ __forceinline__ void gm_unpack(const GmRaw<FMT> &o, int g, gm_i32x4 B
   }
 }
 
-template <int FMT, int EPI, int W, int U>
+// RG: 16-row groups per workgroup. 4: a tile. 6: 96 rows, taken three groups at a time against the same staged tokens,
+// for launches whose workgroups of 64 rows would fill the last of their rounds of 256 (one per CU) badly: see gemm_plan.
+template <int FMT, int EPI, int W, int U, int RG>
 __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
   extern __shared__ __align__(16) uint8_t xl[];
   constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1;
   constexpr int WH = NR == 2 ? W / 2 : W;                 // waves per matrix
-  constexpr int DEPTH = U <= 2 && FMT != T_Q6_K ? 2 : 1;                   // slabs of weights in flight beyond the one computed
+  constexpr int NH = RG == 6 ? 2 : 1, JH = RG / NH;       // row groups JH at a time
+  constexpr int DEPTH = U <= 2 && FMT != T_Q6_K && NH == 1 ? 2 : 1;  // slabs of weights in flight beyond the one computed
+  constexpr int BR = RG * 16;                              // rows per workgroup
   constexpr int MP = 16 * U;                               // staged tokens (the last group padded with the last token)
   constexpr int RB = WH * MP * 96;                         // LDS bytes of one round: values, then records
   constexpr int CH = RB / 1024;                            // 1 KB staging chunks per round
   constexpr int SPW = (CH + W - 1) / W;                    // staging loads per wave and round
   static_assert(RB % 1024 == 0, "whole staging chunks");
-  const int kp = blockIdx.x, tile = blockIdx.y;
+  const int kp = blockIdx.x, blk = blockIdx.y;
   // token group z of the launch's G (blockIdx.z): tokens tb .. tb + Ml - 1, staged as rows 0 .. MP - 1. A (row, token)
   // sum does not depend on which workgroup holds the token, so the groups only spread a small matrix over more CUs.
   const int zg = blockIdx.z, G = gridDim.z, tb = zg * MP, Ml = min(MP, a.M - tb);
@@ -132,11 +142,12 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
   const int grp = NR == 2 ? __builtin_amdgcn_readfirstlane(wave / WH) : 0;
   const int wl = wave - grp * WH;
   const int ks = a.ks, M = Ml;  // this group's tokens
-  const int si = __builtin_amdgcn_readfirstlane(
-      EPI == EPI_SWIGLU ? 0 : (a.nseg > 2 && tile >= a.seg[2].tile0) ? 2 : (a.nseg > 1 && tile >= a.seg[1].tile0) ? 1 : 0);
+  // first row blocks of the second and third segment
+  const int blk1 = RG == 4 ? a.seg[1].tile0 : gemm_blocks6(a.seg[0].rows), blk2 = RG == 4 ? a.seg[2].tile0 : blk1 + gemm_blocks6(a.seg[1].rows);
+  const int si = __builtin_amdgcn_readfirstlane(EPI == EPI_SWIGLU ? 0 : (a.nseg > 2 && blk >= blk2) ? 2 : (a.nseg > 1 && blk >= blk1) ? 1 : 0);
 #define ZL_SEG(f) (si == 0 ? a.seg[0].f : si == 1 ? a.seg[1].f : a.seg[2].f)
-  const int lt = tile - ZL_SEG(tile0), rows = ZL_SEG(rows);
-  const int nslab = a.nslab, nsb = nslab >> 2;
+  const int lb = blk - (si == 0 ? 0 : si == 1 ? blk1 : blk2), rows = ZL_SEG(rows), nq = (rows + 15) >> 4;
+  const int nslab = a.nslab;
   const Rsrc R0 = {make_rsrc(ZL_SEG(m.qs), ZL_SEG(nqs)), make_rsrc(ZL_SEG(m.qx), ZL_SEG(nqx)), make_rsrc(ZL_SEG(m.sc), ZL_SEG(nsc)),
                    make_rsrc(ZL_SEG(m.dd), ZL_SEG(ndd))};
   const Rsrc R1 = NR == 2 ? Rsrc{make_rsrc(a.seg[1].m.qs, a.seg[1].nqs), make_rsrc(a.seg[1].m.qx, a.seg[1].nqx),
@@ -174,48 +185,51 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
     }
   };
 
-  double acc[4][U][4];
+  double acc[RG][U][4];
   #pragma unroll
-  for (int j = 0; j < 4; j++)
+  for (int j = 0; j < RG; j++)
     #pragma unroll
     for (int u = 0; u < U; u++)
       #pragma unroll
       for (int v = 0; v < 4; v++) acc[j][u][v] = 0.0;
 
-  auto load = [&](int i, GmRaw<FMT> &b) {
-    const int s = s0 + wl + WH * i;
-    gm_load<FMT>(R, lt * nslab + s, lt * nsb + (s >> 2), n16, g, i < n, b);
+  auto load = [&](int i, int h, GmRaw<FMT, JH> &b) {
+    gm_load<FMT, JH>(R, lb * RG + h * JH, nq, s0 + wl + WH * i, nslab, n16, g, i < n, b);
   };
-  GmRaw<FMT> ring[DEPTH];
+  GmRaw<FMT, JH> ring[DEPTH * NH];
   {
     u32x4 sg[SPW];
     stage_load(0, sg);
     #pragma unroll
-    for (int d = 0; d < DEPTH; d++) load(d, ring[d]);
+    for (int d = 0; d < DEPTH; d++)
+      #pragma unroll
+      for (int h = 0; h < NH; h++) load(d, h, ring[d * NH + h]);
     stage_store(0, sg);
     __syncthreads();
   }
 
-  // one round: the wave's slab r (weights in `slot`, activations in buffer r & 1), the next round's activations staged
-  auto round = [&](int r, GmRaw<FMT> &slot) {
-    gm_i32x4 B[4];
-    double f[4][gm_nf<FMT>];
-    uint32_t gs[4];
-    gm_unpack<FMT>(slot, g, B, f, gs);
+  // one round: the wave's slab r (weights in `slots`, activations in buffer r & 1), the next round's activations staged
+  auto round = [&](int r, GmRaw<FMT, JH> *slots) {
+    u32x4 sg[SPW];
+    #pragma unroll
+    for (int h = 0; h < NH; h++) {
+    gm_i32x4 B[JH];
+    double f[JH][gm_nf<FMT>];
+    uint32_t gs[JH];
+    gm_unpack<FMT, JH>(slots[h], g, B, f, gs);
     // the operands are formed here, before the slot is reloaded (not sunk to their uses below), so the reload can
     // land in the slot's own registers
     #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < JH; j++) {
       asm volatile("" : "+v"(B[j]));
       #pragma unroll
       for (int k = 0; k < gm_nf<FMT>; k++) asm volatile("" : "+v"(f[j][k]));
       if constexpr (FMT == T_Q6_K) asm volatile("" : "+v"(gs[j]));
     }
-    u32x4 sg[SPW];
     __builtin_amdgcn_sched_barrier(0);  // issue order: the staging loads, then the weights (the stores below wait for
-    stage_load(r + 1, sg);              // the former only)
+    if (h == 0) stage_load(r + 1, sg);  // the former only)
     __builtin_amdgcn_sched_barrier(0);
-    load(r + DEPTH, slot);  // past the wave's last slab: no memory access
+    load(r + DEPTH, h, slots[h]);  // past the wave's last slab: no memory access
     __builtin_amdgcn_sched_barrier(0);
     if (r < n) {
       const uint8_t *buf = xl + (r & 1) * RB;
@@ -242,9 +256,9 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
           };
           dots(0);
           #pragma unroll
-          for (int j = 0; j < 4; j++) {
+          for (int j = 0; j < JH; j++) {
             __builtin_amdgcn_sched_barrier(0);
-            if (j < 3) dots(j + 1);
+            if (j < JH - 1) dots(j + 1);
             const gm_i32x4 (&d)[4] = D[j & 1];
             int sc[4];
             #pragma unroll
@@ -253,7 +267,8 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
             for (int v = 0; v < 4; v++) {
               const int e0 = __mul24(d[0][v], sc[0]) + __mul24(d[1][v], sc[1]);
               const int e1 = __mul24(d[2][v], sc[2]) + __mul24(d[3][v], sc[3]);
-              acc[j][u][v] = fma(f[j][0], fma(xd[1][v], (double)e1, xd[0][v] * (double)e0), acc[j][u][v]);
+              double &s = acc[h * JH + j][u][v];
+              s = fma(f[j][0], fma(xd[1][v], (double)e1, xd[0][v] * (double)e0), s);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
@@ -262,16 +277,16 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
           for (int b = 0; b < 2; b++) {
             const bool on = (g >> 1) == b;  // this lane's quarter lies in block b
             const gm_i32x4 A = on ? gm_i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w} : gm_i32x4{0, 0, 0, 0};
-            gm_i32x4 D[4];
+            gm_i32x4 D[JH];
             #pragma unroll
-            for (int j = 0; j < 4; j++) D[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
+            for (int j = 0; j < JH; j++) D[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
             #pragma unroll
             for (int v = 0; v < 4; v++) {
               const uint4 rc = *(const uint4 *)(recs + (16 * u + 4 * g + v) * 32 + b * 16);
               const double xd = dbl(rc.x, rc.y);
               #pragma unroll
-              for (int j = 0; j < 4; j++) {
-                double &s = acc[j][u][v];
+              for (int j = 0; j < JH; j++) {
+                double &s = acc[h * JH + j][u][v];
                 if constexpr (FMT == T_Q8_0) {
                   s = fma((double)D[j][v] * f[j][b], xd, s);
                 } else {
@@ -283,36 +298,44 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
         }
       }
     }
+    }
     stage_store(r + 1, sg);  // buffer (r + 1) & 1 was last read in round r - 1, before the previous barrier
     __syncthreads();
   };
   // whole groups of DEPTH rounds (a round past the last only stages and loads unused bytes), so each slot of the ring
   // keeps its registers from one iteration to the next
   for (int r = 0; r < nr; r += DEPTH) {
-    round(r, ring[0]);
-    if constexpr (DEPTH == 2) round(r + 1, ring[1]);
+    round(r, ring);
+    if constexpr (DEPTH == 2) round(r + 1, ring + NH);
   }
 
-  // ---- every wave parks its sums, then wave w adds those of tokens w, w + W, ... over the waves of each matrix in the
-  // order of a halving tree (as k_gemv_tiles) and runs the epilogue (or stores a K part). A wave's TPW tokens go through
-  // each step together, so its loads and chains overlap: token by token the hand-off's loads alone were TPW round trips.
-  constexpr int TPW = MP / W;
-  double *red = (double *)xl;  // [token group of a batch][W][4 j][4 v][64 lanes]
-  const int PW = NR * MP * 64;  // doubles per K part
-  double *pp = a.part + (((long)tile * G + zg) * ks + kp) * PW;
-  const int row = lt * 64 + lane;
-  const bool live = row < rows;
-  float rres[TPW];  // the residual values, requested ahead of the reduction
+  // ---- every wave parks its sums, then each wave adds its share of the (row, token) sums over the waves of each matrix
+  // in the order of a halving tree (as k_gemv_tiles) and runs the epilogue (or stores a K part). Its NU units of 64 sums
+  // go through each step together, so their loads and chains overlap: one by one the hand-off's loads alone were NU
+  // round trips. Unit k: 64-row tiles, token wave + W k and row `lane`; 96-row blocks, 32 rows (a whole block of the
+  // quantised output) of two tokens.
+  constexpr int UPG = RG / (W / 4);  // units per wave and token group
+  constexpr int NU = U * UPG;
+  auto unit_t = [&](int k) {
+    return RG == 4 ? wave + W * k : 16 * (k / UPG) + 2 * (wave + W * ((k % UPG) / 3)) + (lane >> 5);
+  };
+  auto unit_r = [&](int k) { return RG == 4 ? lane : 32 * ((k % UPG) % 3) + (lane & 31); };
+  double *red = (double *)xl;  // [token group of a batch][W][RG j][4 v][64 lanes]
+  const int PW = NR * MP * BR;  // doubles per K part
+  double *pp = a.part + (((long)blk * G + zg) * ks + kp) * PW;
+  const int row0 = lb * BR;
+  float rres[NU];  // the residual values, requested ahead of the reduction
   if constexpr (EPI == EPI_RESID) {
     #pragma unroll
-    for (int k = 0; k < TPW; k++) rres[k] = a.resid[(long)(tb + min(wave + W * k, M - 1)) * a.ldr + min(row, rows - 1)];
+    for (int k = 0; k < NU; k++) rres[k] = a.resid[(long)(tb + min(unit_t(k), M - 1)) * a.ldr + min(row0 + unit_r(k), rows - 1)];
   }
-  auto epilogue = [&](int k, int t, double g0, double u0) {
+  auto epilogue = [&](int k, int t, int row, double g0, double u0) {
+    const bool live = row < rows;
     if constexpr (EPI == EPI_SWIGLU) {
       const double gv = (double)(float)g0, uu = (double)(float)u0;
       const float hv = live ? (float)(gv / (1.0 + exp(-gv)) * uu) : 0.f;  // src/compute/ref-kernels.js:322
       if (live) a.hb[(long)t * a.ldh + row] = hv;
-      if (a.qout.q) quant_block32(hv, row, a.qout, t);
+      if (a.qout.q && (RG == 4 || row < ((rows + 63) & ~63))) quant_block32(hv, row, a.qout, t);
     } else if constexpr (EPI == EPI_RESID) {
       const double y = (double)(float)g0;
       if (live) a.resid[(long)t * a.ldr + row] = (float)((double)rres[k] + y);
@@ -324,28 +347,28 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
       }
     }
   };
-  double sums[TPW][NR];
-  constexpr int UB = gemm_ub(U);  // token groups parked at a time
+  double sums[NU][NR];
+  constexpr int UB = gemm_ub(U, RG);  // token groups parked at a time
   #pragma unroll
   for (int u0 = 0; u0 < U; u0 += UB) {
     if (u0 > 0) __syncthreads();  // the previous groups' sums have been read
     #pragma unroll
     for (int u = u0; u < u0 + UB && u < U; u++)
       #pragma unroll
-      for (int j = 0; j < 4; j++)
+      for (int j = 0; j < RG; j++)
         #pragma unroll
-        for (int v = 0; v < 4; v++) red[((((u - u0) * W + wave) * 4 + j) * 4 + v) * 64 + lane] = acc[j][u][v];
+        for (int v = 0; v < 4; v++) red[((((u - u0) * W + wave) * RG + j) * 4 + v) * 64 + lane] = acc[j][u][v];
     __syncthreads();
     #pragma unroll
-    for (int k = u0 * 16 / W; k < TPW && k < (u0 + UB) * 16 / W; k++) {
-      const int t = wave + W * k, tt = t & 15;  // (tokens past M: sums of padding, not stored)
-      // (row = lane, token t): row group lane / 16 in lane 16 (tt / 4) + lane mod 16, slot v = tt mod 4
-      const int src = 16 * (tt >> 2) + n16, jv = (lane >> 4) * 4 + (tt & 3);
+    for (int k = u0 * UPG; k < NU && k < (u0 + UB) * UPG; k++) {
+      const int t = unit_t(k), tt = t & 15, rr = unit_r(k);  // (tokens past M: sums of padding, not stored)
+      // (row rr, token t): row group rr / 16 in lane 16 (tt / 4) + rr mod 16, slot v = tt mod 4
+      const int src = 16 * (tt >> 2) + n16, jv = (rr >> 4) * 4 + (tt & 3);
       #pragma unroll
       for (int r = 0; r < NR; r++) {
         double vv[WH];
         #pragma unroll
-        for (int w = 0; w < WH; w++) vv[w] = red[(((((t >> 4) - u0) * W + r * WH + w) * 16) + jv) * 64 + src];
+        for (int w = 0; w < WH; w++) vv[w] = red[((((k / UPG - u0) * W + r * WH + w) * RG * 4) + jv) * 64 + src];
         #pragma unroll
         for (int half = WH / 2; half >= 1; half >>= 1)
           #pragma unroll
@@ -355,37 +378,37 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
     }
   }
   if (ks > 1) {
-    // ---- K parts: the last part of the tile to arrive adds all parts' sums in part order (as k_gemv_tiles)
+    // ---- K parts: the last part of the row block to arrive adds all parts' sums in part order (as k_gemv_tiles)
     __shared__ uint32_t last;
     #pragma unroll
-    for (int k = 0; k < TPW; k++)
-      if (wave + W * k < M) {
+    for (int k = 0; k < NU; k++)
+      if (unit_t(k) < M) {
         #pragma unroll
         for (int r = 0; r < NR; r++)
-          __hip_atomic_store(pp + (r * MP + wave + W * k) * 64 + lane, sums[k][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(pp + (r * MP + unit_t(k)) * BR + unit_r(k), sums[k][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores are complete
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __syncthreads();
-    uint32_t *cnt = a.cnt + (long)tile * G + zg;
+    uint32_t *cnt = a.cnt + (long)blk * G + zg;
     if (threadIdx.x == 0) last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(ks - 1);
     __syncthreads();
     if (!last) return;
     if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const double *p0 = a.part + ((long)tile * G + zg) * ks * PW + lane;
+    const double *p0 = a.part + ((long)blk * G + zg) * ks * PW;
     for (int q0 = 0; q0 < ks; q0 += 4) {  // four parts' loads of all the wave's sums are issued together
-      double pv[TPW][NR][4];
+      double pv[NU][NR][4];
       #pragma unroll
-      for (int k = 0; k < TPW; k++)
+      for (int k = 0; k < NU; k++)
         #pragma unroll
         for (int r = 0; r < NR; r++)
           #pragma unroll
           for (int q = 0; q < 4; q++)
-            pv[k][r][q] = __hip_atomic_load(p0 + (long)min(q0 + q, ks - 1) * PW + (r * MP + min(wave + W * k, M - 1)) * 64,
+            pv[k][r][q] = __hip_atomic_load(p0 + (long)min(q0 + q, ks - 1) * PW + (r * MP + min(unit_t(k), M - 1)) * BR + unit_r(k),
                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       #pragma unroll
-      for (int k = 0; k < TPW; k++)
+      for (int k = 0; k < NU; k++)
         #pragma unroll
         for (int r = 0; r < NR; r++)
           #pragma unroll
@@ -396,38 +419,40 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
     }
   }
   #pragma unroll
-  for (int k = 0; k < TPW; k++)
-    if (wave + W * k < M) epilogue(k, tb + wave + W * k, sums[k][0], sums[k][NR - 1]);
+  for (int k = 0; k < NU; k++)
+    if (unit_t(k) < M) epilogue(k, tb + unit_t(k), row0 + unit_r(k), sums[k][0], sums[k][NR - 1]);
 #undef ZL_SEG
 }
 
 // LDS bytes of a launch: two staging rounds, or the waves' sums.
-template <int W, int U>
+template <int W, int U, int RG>
 constexpr size_t gemm_lds(bool swiglu) {
-  return std::max((size_t)2 * (swiglu ? W / 2 : W) * 16 * U * 96, (size_t)gemm_ub(U) * W * 16 * 64 * 8);
+  return std::max((size_t)2 * (swiglu ? W / 2 : W) * 16 * U * 96, (size_t)gemm_ub(U, RG) * W * RG * 4 * 64 * 8);
 }
 
-template <int FMT, int EPI, int W, int U>
-inline void launch_gemm_k(const GemvArgs &a, int G, hipStream_t st) {
-  const size_t lds = gemm_lds<W, U>(EPI == EPI_SWIGLU);
+template <int FMT, int EPI, int W, int U, int RG = 4>
+inline void launch_gemm_k(const GemvArgs &a, const GemmPlan &p, hipStream_t st) {
+  const size_t lds = gemm_lds<W, U, RG>(EPI == EPI_SWIGLU);
   static bool done = false;
   if (!done) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_gemm<FMT, EPI, W, U>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    ZL_HIP(hipFuncSetAttribute((const void *)k_gemm<FMT, EPI, W, U, RG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     done = true;
   }
-  hipLaunchKernelGGL((k_gemm<FMT, EPI, W, U>), dim3((unsigned)a.ks, (unsigned)a.ntiles, (unsigned)G), dim3(W * 64), lds, st, a);
+  hipLaunchKernelGGL((k_gemm<FMT, EPI, W, U, RG>), dim3((unsigned)a.ks, (unsigned)p.blocks, (unsigned)p.G), dim3(W * 64), lds, st, a);
 }
 
 template <int FMT, int EPI, int W>
 inline void launch_gemm_w(const GemvArgs &a, hipStream_t st) {
-  int U, G;
-  gemm_groups(a, U, G);
-  ZL_REQUIRE(a.ks == 1 || (long)a.ntiles * G <= GEMV_CNT_TILES, ZL_ERR_ARG, "gemm: too many split-K counters");
-  switch (U) {
-    case 1: launch_gemm_k<FMT, EPI, W, 1>(a, G, st); break;
-    case 2: launch_gemm_k<FMT, EPI, W, 2>(a, G, st); break;
-    case 3: launch_gemm_k<FMT, EPI, W, 3>(a, G, st); break;
-    default: launch_gemm_k<FMT, EPI, W, 4>(a, G, st); break;
+  const GemmPlan p = gemm_plan(a, EPI == EPI_SWIGLU);
+  ZL_REQUIRE(a.ks == 1 || (long)p.blocks * p.G <= GEMV_CNT_TILES, ZL_ERR_ARG, "gemm: too many split-K counters");
+  if constexpr (gemm_has6(FMT)) {
+    if (p.RG == 6) return launch_gemm_k<FMT, EPI, W, 2, 6>(a, p, st);
+  }
+  switch (p.U) {
+    case 1: launch_gemm_k<FMT, EPI, W, 1>(a, p, st); break;
+    case 2: launch_gemm_k<FMT, EPI, W, 2>(a, p, st); break;
+    case 3: launch_gemm_k<FMT, EPI, W, 3>(a, p, st); break;
+    default: launch_gemm_k<FMT, EPI, W, 4>(a, p, st); break;
   }
 }
 

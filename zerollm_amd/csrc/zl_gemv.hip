@@ -92,12 +92,18 @@ bool gemm_takes(const GemvArgs &a) {
 
 long gemv_part_need(const GemvArgs &a) {
   if (a.ks == 1) return 0;
-  if (gemm_takes(a)) {  // a chunk of at most min(M, cap) tokens in G groups of 16 U (the most for the largest chunk)
-    GemvArgs c = a;
-    c.M = std::min(a.M, gemm_max_m());
-    int U, G;
-    gemm_groups(c, U, G);
-    return (long)a.ntiles * a.ks * 2 * 16 * U * G * 64;
+  if (gemm_takes(a)) {  // the split of the chunks' sizes that takes the most (chunks differ by one token at most)
+    const int cap = gemm_max_m(), nch = (a.M + cap - 1) / cap;
+    long need = 0;
+    for (int k = 0; k < 2; k++) {
+      GemvArgs c = a;
+      c.M = k ? (a.M + nch - 1) / nch : std::max(1, a.M / nch);
+      for (const bool swiglu : {false, true}) {
+        const GemmPlan p = gemm_plan(c, swiglu);
+        need = std::max(need, (long)p.blocks * a.ks * 2 * 16 * p.U * p.G * 16 * p.RG);
+      }
+    }
+    return need;
   }
   return (long)a.ntiles * a.ks * 2 * GEMV_MAX_MT * 64;
 }
