@@ -1,45 +1,137 @@
 // GEMV dispatch: K-part choice, token chunks, per-format tile kernels (zl_gemv.h, instantiated in zl_gemv_*.hip) and
 // the float-weight kernel.
+#include <type_traits>
+
 #include "zl_kernels.h"
 
 namespace zl {
 
-// Float weights (F32/F16/BF16) use the f32 activation (src/compute/ref-kernels.js:278-299): one wave per row,
-// sequential f64 sum per lane over a strided subset, then a butterfly.
-template <int EPI>
+// Float weights (F32/F16/BF16) use the f32 activation (src/compute/ref-kernels.js:278-299): a wave takes R rows and MT
+// tokens; lane l adds the products of columns l, l + 64, ... in order in f64 (each product is exact), a butterfly joins
+// the lanes, so a sum's bits depend on neither R nor MT.
+//
+// Bound by HBM where M is small (the matrix is read once per MT tokens) and by the f64 multiply-adds beyond. UN columns
+// of every row and token are requested together: one element at a time each step waited out a memory latency, and a
+// pass per token read the matrix M times. F16: 151936 x 4096 at 1 token 1120 -> 201 us (6.2 TB/s), 4096 x 12288 at 16
+// tokens 1779 -> 69, 512 x 1024 at 1 and 5 tokens 12.0 -> 7.9 and 37.2 -> 8.0.
+template <int TY>
+__device__ __forceinline__ float float_weight(const uint8_t *row, int c) {
+  if constexpr (TY == T_F32) return ((const float *)row)[c];
+  else if constexpr (TY == T_F16) return h2f(((const uint16_t *)row)[c]);
+  else return __uint_as_float((uint32_t)((const uint16_t *)row)[c] << 16);
+}
+
+template <int TY, int EPI, int MT, int R>
 __global__ __launch_bounds__(256) void k_gemv_float(const GemvArgs a, int rows_total, const float *__restrict__ xf, int ldx) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = blockIdx.x * 4 + wave;
-  const bool swig = EPI == EPI_SWIGLU;
-  if (row >= rows_total) return;
-  for (int t = 0; t < a.M; t++) {
-    double accs[2] = {0.0, 0.0};
-    for (int r = 0; r < (swig ? 2 : 1); r++) {
-      int g = row, si = swig ? r : 0, base = 0;
-      if (!swig) while (si + 1 < a.nseg && g >= base + a.seg[si].rows) { base += a.seg[si].rows; si++; }
-      const MatView &m = a.seg[si].m;
-      int lr = g - base;
-      double acc = 0;
-      for (int c = lane; c < m.cols; c += 64) {
-        long e = (long)lr * m.cols + c;
-        float wv = m.type == T_F32 ? ((const float *)m.qs)[e] : m.type == T_F16 ? h2f(((const uint16_t *)m.qs)[e])
-                                                                                : __uint_as_float((uint32_t)((const uint16_t *)m.qs)[e] << 16);
-        acc = acc + (double)wv * (double)xf[(long)t * ldx + c];
-      }
-      acc = wave_sum_xor(acc, 64);
-      accs[r] = acc;
-      if (!swig && lane == 0) {
-        const GemvSeg &sg = a.seg[si];
-        float y = (float)acc;
-        if (EPI == EPI_RESID) { float *xp = a.resid + (long)t * a.ldr + lr; *xp = (float)((double)*xp + (double)y); }
-        else { if (sg.bias) y = (float)((double)y + (double)sg.bias[lr]); sg.out[(long)t * sg.ldo + lr] = y; }
-      }
+  constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1;  // matrices per output row: gate and up
+  constexpr int NW = NR * R;                     // weight rows of the wave
+  constexpr int UN = NW + MT <= 5 ? 8 : NW + MT <= 8 ? 4 : 2;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row0 = (blockIdx.x * 4 + wave) * R, t0 = blockIdx.y * MT;
+  if (row0 >= rows_total) return;
+  const uint8_t *wr[NW];
+  int seg[R], lr[R];  // (rows past the last one repeat it; not stored)
+  #pragma unroll
+  for (int i = 0; i < R; i++) {
+    const int row = min(row0 + i, rows_total - 1);
+    int si = 0, base = 0;
+    if constexpr (EPI == EPI_STORE) {
+      if (a.nseg > 1 && row >= a.seg[0].rows) { si = 1; base = a.seg[0].rows; }
+      if (a.nseg > 2 && row >= a.seg[0].rows + a.seg[1].rows) { si = 2; base = a.seg[0].rows + a.seg[1].rows; }
     }
-    if (swig && lane == 0) {
-      double g = (double)(float)accs[0], u = (double)(float)accs[1];
-      a.hb[(long)t * a.ldh + row] = (float)(g / (1.0 + exp(-g)) * u);
-    }
+    seg[i] = si;
+    lr[i] = row - base;
   }
+#define ZL_SEG(i, f) (seg[i] == 0 ? a.seg[0].f : seg[i] == 1 ? a.seg[1].f : a.seg[2].f)
+  const int cols = a.seg[0].m.cols;
+  const long rb = (long)cols * (TY == T_F32 ? 4 : 2);
+  #pragma unroll
+  for (int i = 0; i < R; i++) {
+    wr[i] = ZL_SEG(i, m.qs) + lr[i] * rb;
+    if constexpr (NR == 2) wr[R + i] = a.seg[1].m.qs + lr[i] * rb;
+  }
+  const float *xr[MT];  // (tokens past M repeat the last one; not stored)
+  #pragma unroll
+  for (int t = 0; t < MT; t++) xr[t] = xf + (long)min(t0 + t, a.M - 1) * ldx;
+  double acc[NW][MT];
+  #pragma unroll
+  for (int i = 0; i < NW; i++)
+    #pragma unroll
+    for (int t = 0; t < MT; t++) acc[i][t] = 0.0;
+  int c = lane;
+  for (; c + 64 * (UN - 1) < cols; c += 64 * UN) {
+    float w[UN][NW], x[UN][MT];
+    #pragma unroll
+    for (int k = 0; k < UN; k++) {
+      #pragma unroll
+      for (int i = 0; i < NW; i++) w[k][i] = float_weight<TY>(wr[i], c + 64 * k);
+      #pragma unroll
+      for (int t = 0; t < MT; t++) x[k][t] = xr[t][c + 64 * k];
+    }
+    #pragma unroll
+    for (int k = 0; k < UN; k++)
+      #pragma unroll
+      for (int i = 0; i < NW; i++)
+        #pragma unroll
+        for (int t = 0; t < MT; t++) acc[i][t] = fma((double)w[k][i], (double)x[k][t], acc[i][t]);
+  }
+  for (; c < cols; c += 64)
+    #pragma unroll
+    for (int i = 0; i < NW; i++) {
+      const double w = (double)float_weight<TY>(wr[i], c);
+      #pragma unroll
+      for (int t = 0; t < MT; t++) acc[i][t] = fma(w, (double)xr[t][c], acc[i][t]);
+    }
+  #pragma unroll
+  for (int i = 0; i < NW; i++)
+    #pragma unroll
+    for (int t = 0; t < MT; t++) acc[i][t] = wave_sum_xor(acc[i][t], 64);
+  #pragma unroll
+  for (int i = 0; i < R; i++)
+    #pragma unroll
+    for (int t = 0; t < MT; t++) {
+      const int tt = t0 + t;
+      if (lane != i * MT + t || row0 + i >= rows_total || tt >= a.M) continue;  // lane i MT + t stores sum (i, t)
+      if constexpr (EPI == EPI_SWIGLU) {
+        const double g = (double)(float)acc[i][t], u = (double)(float)acc[R + i][t];
+        a.hb[(long)tt * a.ldh + lr[i]] = (float)(g / (1.0 + exp(-g)) * u);
+      } else if constexpr (EPI == EPI_RESID) {
+        float *xp = a.resid + (long)tt * a.ldr + lr[i];
+        *xp = (float)((double)*xp + (double)(float)acc[i][t]);
+      } else {
+        float y = (float)acc[i][t];
+        const float *bias = ZL_SEG(i, bias);
+        if (bias) y = (float)((double)y + (double)bias[lr[i]]);
+        ZL_SEG(i, out)[(long)tt * ZL_SEG(i, ldo) + lr[i]] = y;
+      }
+    }
+#undef ZL_SEG
+}
+
+// Four rows per wave share its activation loads where that still leaves four waves per CU, one row otherwise; the
+// tokens in the fewest groups of at most 8, spread evenly.
+template <int TY, int EPI>
+static void launch_gemv_float(const GemvArgs &a, int rows, const float *xf, int ldx, hipStream_t st) {
+  const int groups = (a.M + 7) / 8, per = (a.M + groups - 1) / groups;
+  auto go = [&](auto mt, auto r) {
+    constexpr int MT = mt.value, R = r.value;
+    hipLaunchKernelGGL((k_gemv_float<TY, EPI, MT, R>), dim3((rows + 4 * R - 1) / (4 * R), (a.M + MT - 1) / MT), dim3(256), 0, st, a, rows, xf, ldx);
+  };
+  auto tokens = [&](auto r) {
+    if (per <= 1) go(std::integral_constant<int, 1>{}, r);
+    else if (per <= 2) go(std::integral_constant<int, 2>{}, r);
+    else if (per <= 4) go(std::integral_constant<int, 4>{}, r);
+    else if (per <= 6) go(std::integral_constant<int, 6>{}, r);
+    else go(std::integral_constant<int, 8>{}, r);
+  };
+  if (rows >= 4096) tokens(std::integral_constant<int, 4>{});
+  else tokens(std::integral_constant<int, 1>{});
+}
+template <int TY>
+static void launch_gemv_float_epi(const GemvArgs &a, int epi, int rows, const float *xf, int ldx, hipStream_t st) {
+  if (epi == EPI_STORE) launch_gemv_float<TY, EPI_STORE>(a, rows, xf, ldx, st);
+  else if (epi == EPI_RESID) launch_gemv_float<TY, EPI_RESID>(a, rows, xf, ldx, st);
+  else launch_gemv_float<TY, EPI_SWIGLU>(a, rows, xf, ldx, st);
 }
 
 // Launch shape, a function of the matrix shape only (so every summation order is independent of the token count):
@@ -115,10 +207,10 @@ void launch_gemv(const GemvArgs &a0, int epi, const float *xf, int ldx, hipStrea
   if (!is_quant(fmt)) {
     int rows_total = 0;
     for (int i = 0; i < a0.nseg; i++) rows_total += (epi == EPI_SWIGLU && i > 0) ? 0 : a0.seg[i].rows;
-    const int blocks = (rows_total + 3) / 4;
-    if (epi == EPI_STORE) hipLaunchKernelGGL((k_gemv_float<EPI_STORE>), dim3(blocks), dim3(256), 0, st, a0, rows_total, xf, ldx);
-    else if (epi == EPI_RESID) hipLaunchKernelGGL((k_gemv_float<EPI_RESID>), dim3(blocks), dim3(256), 0, st, a0, rows_total, xf, ldx);
-    else hipLaunchKernelGGL((k_gemv_float<EPI_SWIGLU>), dim3(blocks), dim3(256), 0, st, a0, rows_total, xf, ldx);
+    if (fmt == T_F32) launch_gemv_float_epi<T_F32>(a0, epi, rows_total, xf, ldx, st);
+    else if (fmt == T_F16) launch_gemv_float_epi<T_F16>(a0, epi, rows_total, xf, ldx, st);
+    else if (fmt == T_BF16) launch_gemv_float_epi<T_BF16>(a0, epi, rows_total, xf, ldx, st);
+    else throw Error(ZL_ERR_UNSUPPORTED, "gemv: unsupported weight type");
     ZL_HIP(hipGetLastError());
     return;
   }
