@@ -1,0 +1,43 @@
+"""Short f32 rows that a matvec quantises in its own workgroups, against the call that quantises them in a launch before
+(zl_mat_gemv), bit for bit: chunks per wave up to and past the limit, half slabs, uneven K parts, blocks of zeros."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_kernels import Mat, float_raw
+from zerollm_amd import gguf as G
+from zerollm_amd import synth
+from zerollm_amd._lib import call
+
+pytestmark = pytest.mark.gpu
+
+# 4096 columns: two slabs per wave (4 tokens reach 8 chunks, 5 pass it); 2816 and 2304: K parts of 11 and 9 slabs
+SHAPES = [(t, r, c) for t in (G.Q8_0, G.Q4_0, G.Q5_0, G.Q4_K, G.Q5_K, G.Q6_K)
+          for r, c in ((64, 256), (70, 768), (1100, 2304), (1500, 2816), (2048, 4096))]
+SHAPES += [(t, 100, c) for t in (G.Q8_0, G.Q4_0, G.Q5_0) for c in (32, 96, 1056)] + [(G.F16, 70, 100), (G.F32, 33, 511)]
+
+
+@pytest.mark.parametrize("type_,rows,cols", SHAPES)
+def test_fused_rows_equal_a_launch_before(gpu, type_, rows, cols):
+    raw = (float_raw(type_, rows, cols, rows) if type_ in (G.F16, G.F32)
+           else synth.tensor_bytes(synth.TensorSpec("w", type_, rows, cols, seed=rows + cols), use_device=True))
+    m = Mat(type_, raw, rows, cols)
+    X = np.random.default_rng(cols).standard_normal((9, cols)).astype(np.float32)
+    X[:, : min(cols, 32)] = 0
+    X[1] *= 1e-30
+    X[2, ::7] *= 1e4
+    x, y = torch.from_numpy(X).cuda(), torch.empty((9, rows), device="cuda")
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for M in range(1, 10):
+        print(f"case type {type_} {rows} x {cols} tokens {M}", flush=True)
+        y.fill_(7.0)
+        torch.cuda.synchronize()
+        call("zl_mat_gemv_noalloc", m.h, C.c_void_p(x.data_ptr()), M, C.c_void_p(y.data_ptr()), C.c_void_p(st.cuda_stream))
+        st.synchronize()
+        want = m.gemv(X[:M])
+        assert (y[:M].cpu().numpy().view(np.uint32) == want.view(np.uint32)).all(), M
+        assert bool((y[M:] == 7.0).all())
+    m.free()

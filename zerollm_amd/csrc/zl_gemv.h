@@ -214,9 +214,71 @@ __device__ inline const void *recs_of(const Act &a) {
   else return a.ra;
 }
 
+// ---- f32 rows quantised by the workgroup that multiplies them (a.xf without norm weights, at most XQ 64-value chunks of
+// the M tokens' slab range per wave; wave w takes chunks w, w + W, ..., chunk c = slab c mod nsl of token c / nsl).
+struct XqWalk {  // the wave's chunks in order
+  int t, sl, dt, ds, nsl;
+  __device__ XqWalk(int wave, int W, int n) : nsl(max(n, 1)) {
+    t = __builtin_amdgcn_readfirstlane(wave / nsl); sl = wave - t * nsl;
+    dt = __builtin_amdgcn_readfirstlane(W / nsl); ds = W - dt * nsl;
+  }
+  __device__ void next() {
+    t += dt; sl += ds;
+    if (sl >= nsl) { sl -= nsl; t++; }
+  }
+};
+
+// The chunks' values, requested ahead of the weights (loads complete in order); chunks past the last read a value in range.
+template <int XQ>
+__device__ __forceinline__ void xq_load(const GemvArgs &a, int s0, int nsl, int M, int W, int wave, int lane, float (&xv)[XQ]) {
+  XqWalk c(wave, W, nsl);
+  #pragma unroll
+  for (int k = 0; k < XQ; k++, c.next()) {
+    const int col = (s0 + c.sl) * 64 + lane;
+    xv[k] = a.xf[(long)(a.xrow0 + min(c.t, M - 1)) * a.ldxf + (col < a.n ? col : 0)];
+  }
+}
+
+// quant32 of every chunk into the staged layout (tb bytes per token). The f64 divisions of the chunks' block scales run
+// once, chunk k on lane k of each 16-lane row (a row lies in one block), and come back by a DPP row broadcast.
+template <int FMT, int XQ, int K = 0>
+__device__ __forceinline__ void xq_store(XqWalk c, int s0, int nsl, int nch, int W, int wave, int lane, int n, const float (&xv)[XQ],
+                                         float df, double inv, uint8_t *xl, int tb) {
+  if constexpr (K < XQ) {
+    if (wave + W * K >= nch) return;
+    const float v = (s0 + c.sl) * 64 + lane < n ? xv[K] : 0.f;
+    QBlock b;
+    b.q = (int)round((double)v * dpp_move<0x150 + K>(inv));
+    b.d = dpp_move<0x150 + K>(df);
+    b.s16a = wave_sum_xor(b.q, 16);
+    b.s16b = swizzle_xor16(b.s16a);
+    b.s32 = b.s16a + b.s16b;
+    uint8_t *t = xl + c.t * tb + c.sl * 64;
+    t[lane] = (uint8_t)(int8_t)b.q;
+    if ((lane & 31) == 0) *(uint4 *)(xl + c.t * tb + nsl * 64 + c.sl * 32 + (lane >> 5) * 16) = block_record<FMT>(b);
+    c.next();
+    xq_store<FMT, XQ, K + 1>(c, s0, nsl, nch, W, wave, lane, n, xv, df, inv, xl, tb);
+  }
+}
+template <int FMT, int XQ>
+__device__ __forceinline__ void xq_stage(int s0, int nsl, int M, int W, int wave, int lane, int n, const float (&xv)[XQ], uint8_t *xl, int tb) {
+  const int nch = M * nsl;
+  XqWalk c(wave, W, nsl), w = c;
+  float am = 0.f;
+  #pragma unroll
+  for (int k = 0; k < XQ; k++, w.next()) {
+    if (wave + W * k >= nch) break;
+    const float m = group_fmax(fabsf((s0 + w.sl) * 64 + lane < n ? xv[k] : 0.f), 32);
+    am = (lane & 15) == k ? m : am;
+  }
+  const double scale = (double)am / 127.0, inv = scale != 0.0 ? 1.0 / scale : 0.0;
+  xq_store<FMT, XQ>(c, s0, nsl, nch, W, wave, lane, n, xv, (float)scale, inv, xl, tb);
+}
+
 // The workgroup (kp, tile) of a launch: K part kp of 64-row tile `tile`; xl is the launch's dynamic LDS. Written as a
-// device function so that one kernel can hold two launches of different formats side by side (k_gemv_mix).
-template <int FMT, int MT, int EPI, int DEPTH>
+// device function so that one kernel can hold two launches of different formats side by side (k_gemv_mix). XQ: see above
+// (0: staged from the quantised activations, or the prologue with norm weights).
+template <int FMT, int MT, int EPI, int DEPTH, int XQ = 0>
 __device__ __forceinline__ void gemv_tiles_body(const GemvArgs a, const int kp, const int tile, uint8_t *xl) {
   constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1;  // matrices per output row: gate and up for SwiGLU
   // staged activations, per token: [nsl][64] int8 values, then [nsl][32] records; after the slab loop the same bytes
@@ -257,9 +319,16 @@ __device__ __forceinline__ void gemv_tiles_body(const GemvArgs a, const int kp, 
     const int ts = lt * nslab + s, sbi = lt * nsb + (s >> 2);
     raw_load<FMT>(R, ts, sbi, lane, i < n, b);
   };
+  float xv[XQ > 0 ? XQ : 1];
+  if constexpr (XQ > 0) {
+    xq_load<XQ>(a, s0, nsl, M, W, wave, lane, xv);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   #pragma unroll
   for (int d = 0; d < DEPTH; d++) load(d, buf[d]);
-  if (a.xf) {
+  if constexpr (XQ > 0) {
+    xq_stage<FMT, XQ>(s0, nsl, M, W, wave, lane, a.n, xv, xl, nsl * GT_REC);
+  } else if (a.xf) {
     // ---- fused prologue: RMSNorm scale per token (groups of 4 waves, each in k_norm_quant's order), then quantise the
     // slab range of every token into LDS in the staged layout
     __shared__ double ssr[4][4];
@@ -334,7 +403,7 @@ __device__ __forceinline__ void gemv_tiles_body(const GemvArgs a, const int kp, 
   // (and the K parts' hand-off), where its latency would follow the kernel's last step
   float rres = 0.f;
   if constexpr (EPI == EPI_RESID) rres = a.resid[(long)min(wave, M - 1) * a.ldr + min(lt * 64 + lane, rows - 1)];
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the staged bytes are in LDS
+  if constexpr (XQ == 0) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the staged bytes are in LDS
   __syncthreads();
   // fully unrolled over the most slabs a wave can hold (no loop-carried registers: each slot's reload lands in the
   // registers it was loaded into, and the waits count exactly the loads still needed)
@@ -445,10 +514,10 @@ __device__ __forceinline__ void gemv_tiles_body(const GemvArgs a, const int kp, 
 #undef ZL_SEG
 }
 
-template <int FMT, int MT, int EPI, int DEPTH>
+template <int FMT, int MT, int EPI, int DEPTH, int XQ = 0>
 __global__ __launch_bounds__(1024) void k_gemv_tiles(const GemvArgs a) {
   extern __shared__ __align__(16) uint8_t xl[];
-  gemv_tiles_body<FMT, MT, EPI, DEPTH>(a, blockIdx.x, blockIdx.y, xl);  // grid: (K parts, tiles)
+  gemv_tiles_body<FMT, MT, EPI, DEPTH, XQ>(a, blockIdx.x, blockIdx.y, xl);  // grid: (K parts, tiles)
 }
 
 template <auto K>
@@ -471,6 +540,13 @@ inline void launch_tiles_mt(const GemvArgs &a, int epi, hipStream_t st) {
   const dim3 grid((unsigned)a.ks, (unsigned)a.ntiles), blk((unsigned)a.nwave * 64);
   // [M][kr] staged records of 96 bytes, then (same bytes) the waves' sums
   const size_t lds = std::max((size_t)a.M * a.kr * GT_REC, (size_t)a.nwave * MT * 64 * 8);
+  if constexpr ((FMT != T_Q4_K && FMT != T_Q8_0) || MT == 1) {  // (2..9 tokens of Q4_K and Q8_0: on the matrix cores)
+    if (gemv_xq_ok(a, epi)) {
+      allow_big_lds<k_gemv_tiles<FMT, MT, EPI_STORE, 4, XQ_MAX>>();
+      hipLaunchKernelGGL((k_gemv_tiles<FMT, MT, EPI_STORE, 4, XQ_MAX>), grid, blk, lds, st, a);
+      return;
+    }
+  }
   if (epi == EPI_STORE) {
     allow_big_lds<k_gemv_tiles<FMT, MT, EPI_STORE, 4>>();
     hipLaunchKernelGGL((k_gemv_tiles<FMT, MT, EPI_STORE, 4>), grid, blk, lds, st, a);

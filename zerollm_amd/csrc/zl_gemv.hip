@@ -248,7 +248,7 @@ void launch_gemv(const GemvArgs &a0, int epi, const float *xf, int ldx, hipStrea
       ZL_HIP(hipGetLastError());
       continue;
     }
-    if (gemv_mfma_ok(b)) {  // Q4_K and Q8_0 at 2..8 tokens: the int8 dots on the matrix cores, same results
+    if (gemv_mfma_ok(b, epi)) {  // Q4_K and Q8_0 at 2..8 tokens: the int8 dots on the matrix cores, same results
       launch_gemv_mfma(b, epi, st);
       ZL_HIP(hipGetLastError());
       continue;

@@ -34,7 +34,8 @@ constexpr int mf_slots(int mc) { return mc == 3 ? 9 : 8; }
 constexpr int MF_TPAD = 16;
 
 // MC: token class of the launch, 0 = 2..4 tokens, 1 = 5 tokens, 2 = 6..8 tokens, 3 = 9 tokens
-template <int FMT, int EPI, int MC>
+// XQ: the f32 rows a.xf are quantised here (zl_gemv.h), else the quantised activations are staged
+template <int FMT, int EPI, int MC, int XQ = 0>
 __device__ __forceinline__ void gemv_mfma_body(const GemvArgs a, const int kp, const int tile, uint8_t *xl) {
   static_assert(FMT == T_Q4_K || FMT == T_Q8_0, "matrix-core formats");
   constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1;
@@ -92,9 +93,16 @@ __device__ __forceinline__ void gemv_mfma_body(const GemvArgs a, const int kp, c
       b.dw = __builtin_amdgcn_raw_buffer_load_b32(R.dd, oob + lane * 4, tsv * 256, 0);
     }
   };
+  float xv[XQ > 0 ? XQ : 1];
+  if constexpr (XQ > 0) {
+    xq_load<XQ>(a, s0, nsl, M, W, wave, lane, xv);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   #pragma unroll
   for (int d = 0; d < DEPTH; d++) load(d, buf[d]);
-  {
+  if constexpr (XQ > 0) {
+    xq_stage<FMT, XQ>(s0, nsl, M, W, wave, lane, a.n, xv, xl, ts);
+  } else {
     // ---- stage the activations of the workgroup's slab range in LDS (as k_gemv_tiles does)
     const int xb = nsl * 64, rb = nsl * 32, xc = (xb + 1023) >> 10, rc = (rb + 1023) >> 10, per = xc + rc;
     for (int c = wave; c < M * per; c += W) {
@@ -112,7 +120,7 @@ __device__ __forceinline__ void gemv_mfma_body(const GemvArgs a, const int kp, c
   // (and the K parts' hand-off), where its latency would follow the kernel's last step
   float rres = 0.f;
   if constexpr (EPI == EPI_RESID) rres = a.resid[(long)min(wave, M - 1) * a.ldr + min(lt * 64 + lane, rows - 1)];
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the staged bytes are in LDS
+  if constexpr (XQ == 0) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the staged bytes are in LDS
   __syncthreads();
   // A-fragment row rho = n16 of this lane: token n16 / 4 (n16 mod 4 < 2) or 4 + n16 / 4, block n16 & 1; its quarter g
   // holds values of that block
@@ -313,10 +321,10 @@ __device__ __forceinline__ void gemv_mfma_body(const GemvArgs a, const int kp, c
 }
 
 // (9 tokens: at most 8 waves, so that the second fragment's sums stay in registers)
-template <int FMT, int EPI, int MC>
+template <int FMT, int EPI, int MC, int XQ = 0>
 __global__ __launch_bounds__(MC == 3 ? 512 : 1024) void k_gemv_mfma(const GemvArgs a) {
   extern __shared__ __align__(16) uint8_t xl[];
-  gemv_mfma_body<FMT, EPI, MC>(a, blockIdx.x, blockIdx.y, xl);
+  gemv_mfma_body<FMT, EPI, MC, XQ>(a, blockIdx.x, blockIdx.y, xl);
 }
 
 // Two store launches reading the same activations in one kernel: a Q4_K launch on the matrix cores (a1) and a launch of
@@ -331,10 +339,11 @@ __global__ __launch_bounds__(MT2 == 9 ? 512 : 1024) void k_gemv_mix(const GemvAr
   else gemv_tiles_body<FMT2, MT2, EPI_STORE, 4>(a2, (id - n1) % a2.ks, (id - n1) / a2.ks, xl);
 }
 
-// Q4_K matrices with their fragment plane, and Q8_0 matrices, at 2..9 tokens without a fused prologue.
-bool gemv_mfma_ok(const GemvArgs &a) {
+// Q4_K matrices with their fragment plane, and Q8_0 matrices, at 2..9 tokens, of quantised activations or f32 rows that
+// the kernel quantises itself (store launches alone: gemv_xq_ok).
+bool gemv_mfma_ok(const GemvArgs &a, int epi) {
   const int t = a.seg[0].m.type;
-  if ((t != T_Q4_K && t != T_Q8_0) || a.M < 2 || a.M > 9 || (a.M == 9 && a.nwave > 8) || a.xf) return false;
+  if ((t != T_Q4_K && t != T_Q8_0) || a.M < 2 || a.M > 9 || (a.M == 9 && a.nwave > 8) || (a.xf && !gemv_xq_ok(a, epi))) return false;
   for (int i = 0; i < a.nseg; i++)
     if (a.seg[i].m.type != t || (t == T_Q4_K && !a.seg[i].m.fq)) return false;
   return true;
@@ -342,7 +351,10 @@ bool gemv_mfma_ok(const GemvArgs &a) {
 
 template <int FMT, int MC>
 static void launch_mfma_mc(const GemvArgs &a, int epi, dim3 grid, dim3 blk, size_t lds, hipStream_t st) {
-  if (epi == EPI_STORE) {
+  if (a.xf) {  // (gemv_mfma_ok: a store launch within gemv_xq_ok)
+    allow_big_lds<k_gemv_mfma<FMT, EPI_STORE, MC, XQ_MAX>>();
+    hipLaunchKernelGGL((k_gemv_mfma<FMT, EPI_STORE, MC, XQ_MAX>), grid, blk, lds, st, a);
+  } else if (epi == EPI_STORE) {
     allow_big_lds<k_gemv_mfma<FMT, EPI_STORE, MC>>();
     hipLaunchKernelGGL((k_gemv_mfma<FMT, EPI_STORE, MC>), grid, blk, lds, st, a);
   } else if (epi == EPI_RESID) {
@@ -364,7 +376,7 @@ static void launch_mfma_fmt(const GemvArgs &a, int epi, dim3 grid, dim3 blk, siz
 
 void launch_gemv_mfma(const GemvArgs &a, int epi, hipStream_t st) {
   const int wpm = epi == EPI_SWIGLU ? a.nwave / 2 : a.nwave;
-  ZL_REQUIRE(gemv_mfma_ok(a) && a.kr <= GT_KR_MAX && a.ks <= 8 && wpm >= 1 && a.nwave <= 16 &&
+  ZL_REQUIRE(gemv_mfma_ok(a, epi) && a.kr <= GT_KR_MAX && a.ks <= 8 && wpm >= 1 && a.nwave <= 16 &&
                  (epi != EPI_SWIGLU || (a.nwave % 2 == 0 && wpm <= 8)) && (a.kr + wpm - 1) / wpm <= GT_NMAX,
              ZL_ERR_ARG, "gemv (matrix cores): launch shape out of range");
   const dim3 grid((unsigned)a.ks, (unsigned)a.ntiles), blk((unsigned)a.nwave * 64);
@@ -377,7 +389,7 @@ void launch_gemv_mfma(const GemvArgs &a, int epi, hipStream_t st) {
 // and workgroup size, neither with a fused prologue, one chunk of tokens.
 bool gemv_mix_ok(const GemvArgs &a1, const GemvArgs &a2) {
   const int f2 = a2.seg[0].m.type;
-  if (!gemv_mfma_ok(a1) || a1.seg[0].m.type != T_Q4_K || (f2 != T_Q6_K && f2 != T_Q8_0) || a1.xf || a2.xf ||
+  if (!gemv_mfma_ok(a1, EPI_STORE) || a1.seg[0].m.type != T_Q4_K || (f2 != T_Q6_K && f2 != T_Q8_0) || a1.xf || a2.xf ||
       a1.M != a2.M || a1.nwave != a2.nwave)
     return false;
   for (int i = 1; i < a2.nseg; i++)

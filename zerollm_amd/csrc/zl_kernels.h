@@ -184,7 +184,18 @@ void launch_deltanet(const DeltaArgs &a, int D, hipStream_t st);
 void gemv_shape(int ntiles, int nslab, bool swiglu, int *ks, int *nw);
 // Launch a GEMV of a.M tokens (chunks of at most GEMV_MAX_MT); float weights read the f32 activation xf (stride ldx).
 void launch_gemv(const GemvArgs &a, int epi, const float *xf, int ldx, hipStream_t st);
-bool gemv_mfma_ok(const GemvArgs &a);
+bool gemv_mfma_ok(const GemvArgs &a, int epi);
+
+// Whether a store launch of f32 rows xf without norm weights quantises them in the workgroups that multiply them, each
+// its own K part's: where a wave then has at most XQ_MAX chunks of 64 values and the launch at most two workgroups per
+// CU. Beyond either the work repeated in every workgroup costs more than the k_norm_quant launch it saves. Launch before
+// against fused: Q8_0 1024 x 1024 at 2 tokens (4 chunks) 8.2 -> 6.0 us, Q4_0 64 x 256 at 1 token 8.3 -> 4.4, Q6_K 4096 x 4096
+// at 2 (4 chunks) 10.0 -> 8.5 and 4096 x 12288 at 1 (6) 13.6 -> 11.8; at 10 chunks Q4_K 4096 x 4096 at 5 tokens 10.25
+// and 10.56, Q5_K 8192 x 1024 at 5 9.1 and 9.4.
+constexpr int XQ_MAX = 8;
+inline bool gemv_xq_ok(const GemvArgs &a, int epi) {
+  return epi == EPI_STORE && a.xf && !a.nw && a.nseg == 1 && a.M <= GEMV_MAX_MT && a.M * a.kr <= XQ_MAX * a.nwave && a.ntiles * a.ks <= 512;
+}
 void launch_gemv_mfma(const GemvArgs &a, int epi, hipStream_t st);
 // Two store launches of the same tokens in one kernel (a1 Q4_K on the matrix cores, a2 Q6_K or Q8_0 on the VALU tiles);
 // their split-K work spaces must be disjoint.

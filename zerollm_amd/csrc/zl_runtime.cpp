@@ -1723,6 +1723,16 @@ static void mat_gemv_noalloc(zl_mat *m, const float *x, int M, float *y, hipStre
     launch_gemv_rg(a, EPI_STORE, st);
     return;
   }
+  if (!is_quant(mm.type)) {  // float weights read the f32 rows as they are
+    launch_gemv(a, EPI_STORE, x, mm.cols, st);
+    return;
+  }
+  GemvArgs f = a;  // short rows: quantised by the GEMV itself, no launch before it
+  f.xf = x; f.ldxf = mm.cols; f.xrow0 = 0; f.n = mm.cols; f.nw = nullptr; f.eps = 0.0;
+  if (gemv_xq_ok(f, EPI_STORE)) {
+    launch_gemv(f, EPI_STORE, act.f, act.ld, st);
+    return;
+  }
   launch_norm_quant(x, mm.cols, 0, M, nullptr, 0.0, mm.cols, ld, act, st);
   launch_gemv(a, EPI_STORE, act.f, act.ld, st);
 }
