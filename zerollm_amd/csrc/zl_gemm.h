@@ -48,18 +48,18 @@ struct GmRaw {
   uint32_t dw[J];
 };
 
-// Slab s of the row groups q0 .. q0 + J - 1 (16 rows each) of a matrix of nq row groups; groups past the last one read
-// it again (their sums are not stored). J = 4: one whole tile, q0 a multiple of 4.
-template <int FMT, int J>
-__device__ __forceinline__ void gm_load(const Rsrc &R, int q0, int nq, int s, int nslab, int n16, int g, bool valid, GmRaw<FMT, J> &o) {
+// Slab s of the row groups RG lb + j0 .. + J - 1 (16 rows each) of a matrix of nq row groups; groups past the last one
+// read it again (their sums are not stored). RG = 4: row groups j0 .. of tile lb.
+template <int FMT, int J, int RG>
+__device__ __forceinline__ void gm_load(const Rsrc &R, int lb, int j0, int nq, int s, int nslab, int n16, int g, bool valid, GmRaw<FMT, J> &o) {
   const int oob = valid ? 0 : 0x40000000;
   s = valid ? s : 0;
   #pragma unroll
   for (int j = 0; j < J; j++) {
-    const int q = J == 4 ? q0 : min(q0 + j, nq - 1);
+    const int q = RG == 4 ? 4 * lb : min(RG * lb + j0 + j, nq - 1);
     const int ts = (q >> 2) * nslab + s, sbi = (q >> 2) * (nslab >> 2) + (s >> 2);
-    const int r = (J == 4 ? 16 * j : 0) + n16;  // row of the tile, in the lane's offset
-    const int rs = J == 4 ? 0 : 16 * (q & 3);   // and what the wave's offset adds to it
+    const int r = (RG == 4 ? 16 * (j0 + j) : 0) + n16;  // row of the tile, in the lane's offset
+    const int rs = RG == 4 ? 0 : 16 * (q & 3);           // and what the wave's offset adds to it
     u32x4 v;
     if constexpr (FMT == T_Q8_0) {
       // part g (values 16 g .. 16 g + 15) of row r is 16-byte unit 64 g + r of the tile-slab
@@ -125,13 +125,14 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
   extern __shared__ __align__(16) uint8_t xl[];
   constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1;
   constexpr int WH = NR == 2 ? W / 2 : W;                 // waves per matrix
-  constexpr int NH = RG == 6 ? 2 : 1, JH = RG / NH;       // row groups JH at a time
+  constexpr int NH = RG == 6 || (U > 2 && FMT != T_Q6_K) ? 2 : 1, JH = RG / NH;  // row groups JH at a time (fewer operand registers)
   constexpr int DEPTH = U <= 2 && FMT != T_Q6_K && NH == 1 ? 2 : 1;  // slabs of weights in flight beyond the one computed
   constexpr int BR = RG * 16;                              // rows per workgroup
   constexpr int MP = 16 * U;                               // staged tokens (the last group padded with the last token)
   constexpr int RB = WH * MP * 96;                         // LDS bytes of one round: values, then records
   constexpr int CH = RB / 1024;                            // 1 KB staging chunks per round
-  constexpr int SPW = (CH + W - 1) / W;                    // staging loads per wave and round
+  constexpr int SPW = (CH + W - 1) / W;                    // staging loads per wave and round,
+  constexpr int SPH = (SPW + NH - 1) / NH;                 // and with each of its NH parts
   static_assert(RB % 1024 == 0, "whole staging chunks");
   const int kp = blockIdx.x, blk = blockIdx.y;
   // token group z of the launch's G (blockIdx.z): tokens tb .. tb + Ml - 1, staged as rows 0 .. MP - 1. A (row, token)
@@ -164,24 +165,24 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
   // ---- staging of round r into buffer r & 1 (chunk c of the round is LDS bytes [1024 c, 1024 c + 1024) of the
   // buffer), through registers: the loads are issued at the start of the previous round and the LDS stores follow its
   // compute, so the compiler's load counters track them exactly and the weight loads in flight are never waited for
-  auto stage_load = [&](int r, u32x4 *sg) {
+  auto stage_load = [&](int r, int k0, u32x4 *sg) {  // loads k0 .. of the wave's SPW
     #pragma unroll
-    for (int k = 0; k < SPW; k++) {
+    for (int k = k0; k < k0 + SPH; k++) {
       const int c = min(wave + W * k, CH - 1);  // surplus loads repeat the last chunk (the same bytes)
       const bool isv = c < WH * U;
       const int o = (isv ? c : c - WH * U) * 1024 + lane * 16;
       const int per = isv ? MP * 64 : MP * 32, rb = isv ? 64 : 32;
       const int w_ = o / per, rem = o - w_ * per, t = min(rem / rb, M - 1), e = rem % rb;
       const int s = min(s0 + w_ + WH * r, nslab - 1);  // rounds past the last one read a slab in range (unused)
-      sg[k] = *(const u32x4 *)(isv ? xq + (long)(tb + t) * ldq + (long)s * 64 + e : xr + (long)(tb + t) * ldr + (long)s * 32 + e);
+      sg[k - k0] = *(const u32x4 *)(isv ? xq + (long)(tb + t) * ldq + (long)s * 64 + e : xr + (long)(tb + t) * ldr + (long)s * 32 + e);
     }
   };
-  auto stage_store = [&](int r, const u32x4 *sg) {
+  auto stage_store = [&](int r, int k0, const u32x4 *sg) {
     uint8_t *buf = xl + (r & 1) * RB;
     #pragma unroll
-    for (int k = 0; k < SPW; k++) {
+    for (int k = k0; k < k0 + SPH; k++) {
       const int c = min(wave + W * k, CH - 1);
-      *(u32x4 *)(buf + c * 1024 + lane * 16) = sg[k];
+      *(u32x4 *)(buf + c * 1024 + lane * 16) = sg[k - k0];
     }
   };
 
@@ -194,25 +195,27 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
       for (int v = 0; v < 4; v++) acc[j][u][v] = 0.0;
 
   auto load = [&](int i, int h, GmRaw<FMT, JH> &b) {
-    gm_load<FMT, JH>(R, lb * RG + h * JH, nq, s0 + wl + WH * i, nslab, n16, g, i < n, b);
+    gm_load<FMT, JH, RG>(R, lb, h * JH, nq, s0 + wl + WH * i, nslab, n16, g, i < n, b);
   };
   GmRaw<FMT, JH> ring[DEPTH * NH];
   {
-    u32x4 sg[SPW];
-    stage_load(0, sg);
+    u32x4 sg[NH * SPH];
+    #pragma unroll
+    for (int h = 0; h < NH; h++) stage_load(0, h * SPH, sg + h * SPH);
     #pragma unroll
     for (int d = 0; d < DEPTH; d++)
       #pragma unroll
       for (int h = 0; h < NH; h++) load(d, h, ring[d * NH + h]);
-    stage_store(0, sg);
+    #pragma unroll
+    for (int h = 0; h < NH; h++) stage_store(0, h * SPH, sg + h * SPH);
     __syncthreads();
   }
 
   // one round: the wave's slab r (weights in `slots`, activations in buffer r & 1), the next round's activations staged
   auto round = [&](int r, GmRaw<FMT, JH> *slots) {
-    u32x4 sg[SPW];
     #pragma unroll
     for (int h = 0; h < NH; h++) {
+    u32x4 sg[SPH];
     gm_i32x4 B[JH];
     double f[JH][gm_nf<FMT>];
     uint32_t gs[JH];
@@ -227,7 +230,7 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
       if constexpr (FMT == T_Q6_K) asm volatile("" : "+v"(gs[j]));
     }
     __builtin_amdgcn_sched_barrier(0);  // issue order: the staging loads, then the weights (the stores below wait for
-    if (h == 0) stage_load(r + 1, sg);  // the former only)
+    stage_load(r + 1, h * SPH, sg);     // the former only)
     __builtin_amdgcn_sched_barrier(0);
     load(r + DEPTH, h, slots[h]);  // past the wave's last slab: no memory access
     __builtin_amdgcn_sched_barrier(0);
@@ -298,8 +301,8 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
         }
       }
     }
+    stage_store(r + 1, h * SPH, sg);  // buffer (r + 1) & 1 was last read in round r - 1, before the previous barrier
     }
-    stage_store(r + 1, sg);  // buffer (r + 1) & 1 was last read in round r - 1, before the previous barrier
     __syncthreads();
   };
   // whole groups of DEPTH rounds (a round past the last only stages and loads unused bytes), so each slot of the ring

@@ -216,35 +216,42 @@ void launch_gemm_fmt(const GemvArgs &a, int epi, hipStream_t st);
 bool gemm_takes(const GemvArgs &a);
 long gemv_part_need(const GemvArgs &a);
 // Split of a GEMM launch of a.M <= 64 tokens: workgroups of RG 16-row groups and 16 U tokens, `blocks` of them along the
-// rows and G along the tokens per K part, each token group re-reading the matrix (no group is empty).
-// - 64-row tiles (RG 4): up to 4 token groups while the launch stays within 512 workgroups: at 64 tokens the 8B-shaped
-//   target's attn_v takes 4 (64 workgroups otherwise), attn_output and ffn_down 2, the 0.6B-shaped draft's projections 4
-//   (16-64 workgroups otherwise); measured on 16K-token prefills, target + draft: 3.91 + 1.88 s in one group,
-//   3.63 + 1.63 s within 320 workgroups, 3.23 + 1.55 s within 512, 3.31 + 1.59 s within 1024.
-// - 96-row blocks of 32 tokens (RG 6, U 2): the registers leave room for one workgroup per CU, so a launch takes whole
-//   rounds of 256, and 12288 rows of gate/up at 64 tokens were 384 workgroups, two rounds of which the second was half
-//   empty. In 96-row blocks they are 256. A workgroup of these costs about 1.5 of a 64-row one of 32 tokens (more row
-//   groups to unpack, the same staged tokens), one of 16, 48 and 64 tokens costs 0.7, 1.4 and 1.8: the plan takes the
-//   split with the lower rounds x cost. Measured at 64 tokens: Q4_K gate/up 12288 x 4096 72 -> 55 us, 9216 x 2560
-//   50 -> 38, q+k 5120 x 4096 30.6 -> 22.0, q with gates 9216 x 2560 30.7 -> 21.4; Q5_K 2560 x 4096 26.0 -> 18.2. Q6_K
-//   stays on tiles: its 8B and 4B shapes fill their rounds.
+// rows and G along the tokens per K part, each token group re-reading the matrix (no group is empty): 64-row tiles
+// (RG 4) in 1, 2 or 4 token groups, or 96-row blocks of 32 tokens (RG 6, U 2).
+// The registers leave room for one workgroup per CU, so a launch takes whole rounds of 256, and a round costs a
+// workgroup's start, reduction and hand-off (about 7 us) and its slabs' compute. The plan takes the split of the lowest
+// rounds x cost, the slabs' costs as measured with Q4_K at 64 tokens (in 0.1 us per slab and wave: 19 for 32 tokens, 31 in
+// 96-row blocks; 16, 48 and 64 tokens after their instruction counts). At 64 tokens (8B and 4B shapes), two token groups
+// against the split taken: Q4_K gate/up 12288 x 4096 (384 workgroups, the second round half empty; 96-row blocks: 256)
+// 72 -> 55 us, 9216 x 2560 50 -> 38, q+k 5120 x 4096 30.6 -> 22.0; Q5_K 8192 x 2560 (one group) 31.6 -> 27.1, Q4_K
+// 4096 x 2560 (two, of four) 20.0 -> 15.8, attn_output 4096 x 4096 (one) 23.8 -> 22.3. Q6_K takes the most token groups
+// within 512 workgroups: the operands of its four dots leave no registers for more tokens (4096 x 12288 in two groups 45 us,
+// in one 72).
 struct GemmPlan { int RG, U, G, blocks; };
 __host__ __device__ constexpr bool gemm_has6(int fmt) { return fmt == T_Q4_K || fmt == T_Q5_K || fmt == T_Q8_0; }
 __host__ __device__ inline int gemm_blocks6(int rows) { return (rows + 95) / 96; }
 inline GemmPlan gemm_plan(const GemvArgs &a, bool swiglu) {
-  const int n16 = (a.M + 15) / 16, blocks = a.ks * a.ntiles;
-  GemmPlan p{4, 0, 1, a.ntiles};
-  while (p.G < 4 && 2 * p.G <= n16 && 2 * p.G * blocks <= 512) p.G *= 2;
-  p.U = (n16 + p.G - 1) / p.G;
+  const int n16 = (a.M + 15) / 16, wh = swiglu ? a.nwave / 2 : a.nwave, slabs = (a.kr + wh - 1) / wh;
+  const int start = 70, slab[5] = {0, 14, 19, 26, 33}, slab6 = 31;
+  GemmPlan p{};
+  long best = 0;
+  auto take = [&](int RG, int U, int G, int blocks, int cost) {
+    const long t = ((long)a.ks * blocks * G + 255) / 256 * (start + slabs * cost);
+    if (!best || t < best) { best = t; p = GemmPlan{RG, U, G, blocks}; }
+  };
+  for (int G = 1; G <= 4 && G <= n16; G *= 2) {
+    const int U = (n16 + G - 1) / G;
+    if (G > 1 && (long)a.ks * a.ntiles * G > 512) break;
+    if (a.seg[0].m.type == T_Q6_K) best = 0;  // the most groups
+    take(4, U, G, a.ntiles, slab[U]);
+  }
   if (!gemm_has6(a.seg[0].m.type) || n16 < 2) return p;
   int b6 = 0;
   for (int i = 0; i < (swiglu ? 1 : a.nseg); i++) b6 += gemm_blocks6(a.seg[i].rows);
-  const int g6 = (n16 + 1) / 2, cost[5] = {0, 7, 10, 14, 18};
-  auto rounds = [](long n) { return (n + 255) / 256; };
+  const int g6 = (n16 + 1) / 2;
   // (the work spaces hold its K parts, and a quantised output's rows up to the next multiple of 64 are all in a block)
   const bool fits = a.ks == 1 || ((long)b6 * g6 <= GEMV_CNT_TILES && (long)b6 * a.ks * g6 * 2 * 32 * 96 <= GEMV_PART_DOUBLES);
-  if (!fits || (swiglu && b6 * 96 < (a.seg[0].rows + 63) / 64 * 64)) return p;
-  if (15 * rounds((long)a.ks * b6 * g6) < cost[p.U] * rounds((long)blocks * p.G)) p = GemmPlan{6, 2, g6, b6};
+  if (fits && (!swiglu || b6 * 96 >= (a.seg[0].rows + 63) / 64 * 64)) take(6, 2, g6, b6, slab6);
   return p;
 }
 
