@@ -119,9 +119,10 @@ __device__ __forceinline__ void gm_unpack(const GmRaw<FMT, J> &o, int g, gm_i32x
 }
 
 // RG: 16-row groups per workgroup. 4: a tile. 6: 96 rows, taken three groups at a time against the same staged tokens,
-// for launches whose workgroups of 64 rows would fill the last of their rounds of 256 (one per CU) badly: see gemm_plan.
+// for launches whose workgroups of 64 rows would fill the last of their rounds of 256 (one per CU) badly; 2: half a tile,
+// for launches of few tiles (two of 8 waves fit a CU): see gemm_plan.
 template <int FMT, int EPI, int W, int U, int RG>
-__global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
+__global__ __launch_bounds__(W * 64, RG == 2 ? 4 : 1) void k_gemm(const GemvArgs a) {
   extern __shared__ __align__(16) uint8_t xl[];
   constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1;
   constexpr int WH = NR == 2 ? W / 2 : W;                 // waves per matrix
@@ -144,7 +145,8 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
   const int wl = wave - grp * WH;
   const int ks = a.ks, M = Ml;  // this group's tokens
   // first row blocks of the second and third segment
-  const int blk1 = RG == 4 ? a.seg[1].tile0 : gemm_blocks6(a.seg[0].rows), blk2 = RG == 4 ? a.seg[2].tile0 : blk1 + gemm_blocks6(a.seg[1].rows);
+  const int blk1 = RG == 6 ? gemm_blocks6(a.seg[0].rows) : a.seg[1].tile0 * 4 / RG;
+  const int blk2 = RG == 6 ? blk1 + gemm_blocks6(a.seg[1].rows) : a.seg[2].tile0 * 4 / RG;
   const int si = __builtin_amdgcn_readfirstlane(EPI == EPI_SWIGLU ? 0 : (a.nseg > 2 && blk >= blk2) ? 2 : (a.nseg > 1 && blk >= blk1) ? 1 : 0);
 #define ZL_SEG(f) (si == 0 ? a.seg[0].f : si == 1 ? a.seg[1].f : a.seg[2].f)
   const int lb = blk - (si == 0 ? 0 : si == 1 ? blk1 : blk2), rows = ZL_SEG(rows), nq = (rows + 15) >> 4;
@@ -315,14 +317,14 @@ __global__ __launch_bounds__(W * 64) void k_gemm(const GemvArgs a) {
   // ---- every wave parks its sums, then each wave adds its share of the (row, token) sums over the waves of each matrix
   // in the order of a halving tree (as k_gemv_tiles) and runs the epilogue (or stores a K part). Its NU units of 64 sums
   // go through each step together, so their loads and chains overlap: one by one the hand-off's loads alone were NU
-  // round trips. Unit k: 64-row tiles, token wave + W k and row `lane`; 96-row blocks, 32 rows (a whole block of the
+  // round trips. Unit k: 64-row tiles, token wave + W k and row `lane`; 96- and 32-row blocks, 32 rows (a whole block of the
   // quantised output) of two tokens.
-  constexpr int UPG = RG / (W / 4);  // units per wave and token group
+  constexpr int UPG = RG / (W / 4), RU = RG / 2;  // units per wave and token group; 32-row units per block
   constexpr int NU = U * UPG;
   auto unit_t = [&](int k) {
-    return RG == 4 ? wave + W * k : 16 * (k / UPG) + 2 * (wave + W * ((k % UPG) / 3)) + (lane >> 5);
+    return RG == 4 ? wave + W * k : 16 * (k / UPG) + 2 * (wave + W * ((k % UPG) / RU)) + (lane >> 5);
   };
-  auto unit_r = [&](int k) { return RG == 4 ? lane : 32 * ((k % UPG) % 3) + (lane & 31); };
+  auto unit_r = [&](int k) { return RG == 4 ? lane : 32 * ((k % UPG) % RU) + (lane & 31); };
   double *red = (double *)xl;  // [token group of a batch][W][RG j][4 v][64 lanes]
   const int PW = NR * MP * BR;  // doubles per K part
   double *pp = a.part + (((long)blk * G + zg) * ks + kp) * PW;
@@ -451,6 +453,7 @@ inline void launch_gemm_w(const GemvArgs &a, hipStream_t st) {
   if constexpr (gemm_has6(FMT)) {
     if (p.RG == 6) return launch_gemm_k<FMT, EPI, W, 2, 6>(a, p, st);
   }
+  if (p.RG == 2) return launch_gemm_k<FMT, EPI, W, 1, 2>(a, p, st);
   switch (p.U) {
     case 1: launch_gemm_k<FMT, EPI, W, 1>(a, p, st); break;
     case 2: launch_gemm_k<FMT, EPI, W, 2>(a, p, st); break;

@@ -217,14 +217,16 @@ bool gemm_takes(const GemvArgs &a);
 long gemv_part_need(const GemvArgs &a);
 // Split of a GEMM launch of a.M <= 64 tokens: workgroups of RG 16-row groups and 16 U tokens, `blocks` of them along the
 // rows and G along the tokens per K part, each token group re-reading the matrix (no group is empty): 64-row tiles
-// (RG 4) in 1, 2 or 4 token groups, or 96-row blocks of 32 tokens (RG 6, U 2).
+// (RG 4) in 1, 2 or 4 token groups, 96-row blocks of 32 tokens (RG 6, U 2) or 32-row blocks of 16 (RG 2, U 1).
 // The registers leave room for one workgroup per CU, so a launch takes whole rounds of 256, and a round costs a
 // workgroup's start, reduction and hand-off (about 7 us) and its slabs' compute. The plan takes the split of the lowest
 // rounds x cost, the slabs' costs as measured with Q4_K at 64 tokens (in 0.1 us per slab and wave: 19 for 32 tokens, 31 in
 // 96-row blocks; 16, 48 and 64 tokens after their instruction counts). At 64 tokens (8B and 4B shapes), two token groups
 // against the split taken: Q4_K gate/up 12288 x 4096 (384 workgroups, the second round half empty; 96-row blocks: 256)
 // 72 -> 55 us, 9216 x 2560 50 -> 38, q+k 5120 x 4096 30.6 -> 22.0; Q5_K 8192 x 2560 (one group) 31.6 -> 27.1, Q4_K
-// 4096 x 2560 (two, of four) 20.0 -> 15.8, attn_output 4096 x 4096 (one) 23.8 -> 22.3. Q6_K takes the most token groups
+// 4096 x 2560 (two, of four) 20.0 -> 15.8, attn_output 4096 x 4096 (one) 23.8 -> 22.0. 32-row blocks (8 after their
+// instruction count; where the launch is small): Q8_0 1024 x 3072 at 64 tokens 10.0 -> 6.9 us, matvec calls of Q8_0 1024 x
+// 1024 at 11 tokens 8.9 -> 7.4, Q4_K 1024 x 2560 at 11 14.4 -> 10.9, Q6_K 1024 x 4096 at 16 12.7 -> 10.3. Q6_K takes the most token groups
 // within 512 workgroups: the operands of its four dots leave no registers for more tokens (4096 x 12288 in two groups 45 us,
 // in one 72).
 struct GemmPlan { int RG, U, G, blocks; };
@@ -232,7 +234,7 @@ __host__ __device__ constexpr bool gemm_has6(int fmt) { return fmt == T_Q4_K || 
 __host__ __device__ inline int gemm_blocks6(int rows) { return (rows + 95) / 96; }
 inline GemmPlan gemm_plan(const GemvArgs &a, bool swiglu) {
   const int n16 = (a.M + 15) / 16, wh = swiglu ? a.nwave / 2 : a.nwave, slabs = (a.kr + wh - 1) / wh;
-  const int start = 70, slab[5] = {0, 14, 19, 26, 33}, slab6 = 31;
+  const int start = 70, slab[5] = {0, 14, 19, 26, 33}, slab6 = 31, slab2 = 8;
   GemmPlan p{};
   long best = 0;
   auto take = [&](int RG, int U, int G, int blocks, int cost) {
@@ -244,6 +246,13 @@ inline GemmPlan gemm_plan(const GemvArgs &a, bool swiglu) {
     if (G > 1 && (long)a.ks * a.ntiles * G > 512) break;
     if (a.seg[0].m.type == T_Q6_K) best = 0;  // the most groups
     take(4, U, G, a.ntiles, slab[U]);
+  }
+  if (n16 != 3) {  // 32-row blocks of 16 tokens, two to a CU
+    const long n = (long)a.ks * 2 * a.ntiles * n16, t = start + (n + 255) / 256 * slabs * slab2;
+    if (n <= 512 && n16 <= p.U * p.G && (a.ks == 1 || 2L * a.ntiles * n16 <= GEMV_CNT_TILES) && t < best) {
+      best = t;
+      p = GemmPlan{2, 1, n16, 2 * a.ntiles};
+    }
   }
   if (!gemm_has6(a.seg[0].m.type) || n16 < 2) return p;
   int b6 = 0;
