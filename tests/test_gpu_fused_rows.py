@@ -41,3 +41,21 @@ def test_fused_rows_equal_a_launch_before(gpu, type_, rows, cols):
         assert (y[:M].cpu().numpy().view(np.uint32) == want.view(np.uint32)).all(), M
         assert bool((y[M:] == 7.0).all())
     m.free()
+
+
+@pytest.mark.parametrize("type_", [G.Q8_0, G.Q4_K, G.Q6_K, G.F16])
+def test_result_over_the_rows(gpu, type_):
+    n = 256
+    raw = (float_raw(type_, n, n, 3) if type_ == G.F16
+           else synth.tensor_bytes(synth.TensorSpec("w", type_, n, n, seed=3), use_device=True))
+    m = Mat(type_, raw, n, n)
+    X = np.random.default_rng(3).standard_normal((3, n)).astype(np.float32)
+    st = torch.cuda.Stream()
+    for M in (2, 3):
+        print(f"case type {type_} tokens {M} in place", flush=True)
+        x = torch.from_numpy(X).cuda()
+        torch.cuda.synchronize()
+        call("zl_mat_gemv_noalloc", m.h, C.c_void_p(x.data_ptr()), M, C.c_void_p(x.data_ptr()), C.c_void_p(st.cuda_stream))
+        st.synchronize()
+        assert (x[:M].cpu().numpy().view(np.uint32) == m.gemv(X[:M]).view(np.uint32)).all()
+    m.free()

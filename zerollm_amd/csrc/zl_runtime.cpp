@@ -1723,15 +1723,20 @@ static void mat_gemv_noalloc(zl_mat *m, const float *x, int M, float *y, hipStre
     launch_gemv_rg(a, EPI_STORE, st);
     return;
   }
-  if (!is_quant(mm.type)) {  // float weights read the f32 rows as they are
-    launch_gemv(a, EPI_STORE, x, mm.cols, st);
-    return;
-  }
-  GemvArgs f = a;  // short rows: quantised by the GEMV itself, no launch before it
-  f.xf = x; f.ldxf = mm.cols; f.xrow0 = 0; f.n = mm.cols; f.nw = nullptr; f.eps = 0.0;
-  if (gemv_xq_ok(f, EPI_STORE)) {
-    launch_gemv(f, EPI_STORE, act.f, act.ld, st);
-    return;
+  // rows that the result overwrites are quantised (copied) before; others are read by the GEMV itself: float weights take
+  // them as they are, quantised ones quantise short rows, with no launch before
+  const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
+  if (x0 + (uintptr_t)M * mm.cols * 4 <= y0 || y0 + (uintptr_t)M * mm.rows * 4 <= x0) {
+    if (!is_quant(mm.type)) {
+      launch_gemv(a, EPI_STORE, x, mm.cols, st);
+      return;
+    }
+    GemvArgs f = a;
+    f.xf = x; f.ldxf = mm.cols; f.xrow0 = 0; f.n = mm.cols; f.nw = nullptr; f.eps = 0.0;
+    if (gemv_xq_ok(f, EPI_STORE)) {
+      launch_gemv(f, EPI_STORE, act.f, act.ld, st);
+      return;
+    }
   }
   launch_norm_quant(x, mm.cols, 0, M, nullptr, 0.0, mm.cols, ld, act, st);
   launch_gemv(a, EPI_STORE, act.f, act.ld, st);
