@@ -7,9 +7,9 @@
 // halving tree over the waves and the same K parts. A token therefore gets the same bits whatever the size of
 // the pass it is in (1..9 tokens through the GEMV kernels, 10..64 here).
 //
-// Mapping (tiles; in 96-row blocks a wave takes six row groups, three at a time). The workgroup is the GEMV's (K part,
-// 64-row tile) with its W waves (gate/up pairs: W / 2 per matrix); wave
-// wl of a matrix walks slabs s0 + wl + WH i as in k_gemv_tiles, but for every token of the launch at once. One
+// Mapping (64-row tiles; blocks of 96 and 32 rows are six and two row groups of 16 in place of four). The workgroup is the
+// GEMV's (K part, 64-row tile) with its W waves (gate/up pairs: W / 2 per matrix); wave wl of a matrix walks
+// slabs s0 + wl + WH i as in k_gemv_tiles, but for every token of the launch at once. One
 // v_mfma_i32_16x16x64_i8 multiplies A (16 tokens: lane l supplies token l mod 16's values of the slab's value quarter
 // g = l / 16) by B (16 rows of the tile: lane l supplies row l mod 16's values of quarter g) into D[token][row]; lane l
 // receives tokens 4 g + v (v = 0..3) of row l mod 16. To keep one 32-value block (Q6_K: one 16-value group) per dot, A
@@ -217,93 +217,94 @@ __global__ __launch_bounds__(W * 64, RG == 2 ? 4 : 1) void k_gemm(const GemvArgs
   auto round = [&](int r, GmRaw<FMT, JH> *slots) {
     #pragma unroll
     for (int h = 0; h < NH; h++) {
-    u32x4 sg[SPH];
-    gm_i32x4 B[JH];
-    double f[JH][gm_nf<FMT>];
-    uint32_t gs[JH];
-    gm_unpack<FMT, JH>(slots[h], g, B, f, gs);
-    // the operands are formed here, before the slot is reloaded (not sunk to their uses below), so the reload can
-    // land in the slot's own registers
-    #pragma unroll
-    for (int j = 0; j < JH; j++) {
-      asm volatile("" : "+v"(B[j]));
+      u32x4 sg[SPH];
+      gm_i32x4 B[JH];
+      double f[JH][gm_nf<FMT>];
+      uint32_t gs[JH];
+      gm_unpack<FMT, JH>(slots[h], g, B, f, gs);
+      // the operands are formed here, before the slot is reloaded (not sunk to their uses below), so the reload can
+      // land in the slot's own registers
       #pragma unroll
-      for (int k = 0; k < gm_nf<FMT>; k++) asm volatile("" : "+v"(f[j][k]));
-      if constexpr (FMT == T_Q6_K) asm volatile("" : "+v"(gs[j]));
-    }
-    __builtin_amdgcn_sched_barrier(0);  // issue order: the staging loads, then the weights (the stores below wait for
-    stage_load(r + 1, h * SPH, sg);     // the former only)
-    __builtin_amdgcn_sched_barrier(0);
-    load(r + DEPTH, h, slots[h]);  // past the wave's last slab: no memory access
-    __builtin_amdgcn_sched_barrier(0);
-    if (r < n) {
-      const uint8_t *buf = xl + (r & 1) * RB;
-      const uint8_t *vals = buf + wl * MP * 64, *recs = buf + WH * MP * 64 + wl * MP * 32;
-      #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const uint4 av = *(const uint4 *)(vals + (16 * u + n16) * 64 + 16 * g);
-        if constexpr (FMT == T_Q6_K) {
-          // the two groups of a block join in integers, the slab's two blocks in one product with d: 9 VALU instructions
-          // per (row, token) and slab where a term per group took 16 (4096 x 12288 at 64 tokens 73.8 -> 48.9 us, bound by
-          // their issue). One slab ahead in flight: two (40 registers each) spilled. Row group j's sums are formed while the matrix cores run j + 1's dots (the
-          // barriers keep the scheduler from holding all four row groups' dots in registers at once)
-          gm_i32x4 A[4], D[2][4];
-          double xd[2][4];
-          #pragma unroll
-          for (int b = 0; b < 4; b++) A[b] = g == b ? gm_i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w} : gm_i32x4{0, 0, 0, 0};
-          #pragma unroll
-          for (int v = 0; v < 4; v++)
+      for (int j = 0; j < JH; j++) {
+        asm volatile("" : "+v"(B[j]));
+        #pragma unroll
+        for (int k = 0; k < gm_nf<FMT>; k++) asm volatile("" : "+v"(f[j][k]));
+        if constexpr (FMT == T_Q6_K) asm volatile("" : "+v"(gs[j]));
+      }
+      __builtin_amdgcn_sched_barrier(0);  // issue order: the staging loads, then the weights (the stores below wait for
+      stage_load(r + 1, h * SPH, sg);     // the former only)
+      __builtin_amdgcn_sched_barrier(0);
+      load(r + DEPTH, h, slots[h]);  // past the wave's last slab: no memory access
+      __builtin_amdgcn_sched_barrier(0);
+      if (r < n) {
+        const uint8_t *buf = xl + (r & 1) * RB;
+        const uint8_t *vals = buf + wl * MP * 64, *recs = buf + WH * MP * 64 + wl * MP * 32;
+        #pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint4 av = *(const uint4 *)(vals + (16 * u + n16) * 64 + 16 * g);
+          if constexpr (FMT == T_Q6_K) {
+            // the two groups of a block join in integers, the slab's two blocks in one product with d: 9 VALU instructions
+            // per (row, token) and slab where a term per group took 16 (4096 x 12288 at 64 tokens 73.8 -> 48.9 us, bound by
+            // their issue). One slab ahead in flight: two (40 registers each) spilled. Row group j's sums are formed while
+            // the matrix cores run j + 1's dots (the barriers keep the scheduler from holding all four row groups' dots in
+            // registers at once)
+            gm_i32x4 A[4], D[2][4];
+            double xd[2][4];
             #pragma unroll
-            for (int blk = 0; blk < 2; blk++) xd[blk][v] = *(const double *)(recs + (16 * u + 4 * g + v) * 32 + blk * 16);
-          auto dots = [&](int j) {
+            for (int b = 0; b < 4; b++) A[b] = g == b ? gm_i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w} : gm_i32x4{0, 0, 0, 0};
             #pragma unroll
-            for (int b = 0; b < 4; b++) D[j & 1][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[b], B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
-          };
-          dots(0);
-          #pragma unroll
-          for (int j = 0; j < JH; j++) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (j < JH - 1) dots(j + 1);
-            const gm_i32x4 (&d)[4] = D[j & 1];
-            int sc[4];
-            #pragma unroll
-            for (int k = 0; k < 4; k++) sc[k] = (int)(int8_t)(gs[j] >> (8 * k));
-            #pragma unroll
-            for (int v = 0; v < 4; v++) {
-              const int e0 = __mul24(d[0][v], sc[0]) + __mul24(d[1][v], sc[1]);
-              const int e1 = __mul24(d[2][v], sc[2]) + __mul24(d[3][v], sc[3]);
-              double &s = acc[h * JH + j][u][v];
-              s = fma(f[j][0], fma(xd[1][v], (double)e1, xd[0][v] * (double)e0), s);
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        } else {
-          #pragma unroll
-          for (int b = 0; b < 2; b++) {
-            const bool on = (g >> 1) == b;  // this lane's quarter lies in block b
-            const gm_i32x4 A = on ? gm_i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w} : gm_i32x4{0, 0, 0, 0};
-            gm_i32x4 D[JH];
-            #pragma unroll
-            for (int j = 0; j < JH; j++) D[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
-            #pragma unroll
-            for (int v = 0; v < 4; v++) {
-              const uint4 rc = *(const uint4 *)(recs + (16 * u + 4 * g + v) * 32 + b * 16);
-              const double xd = dbl(rc.x, rc.y);
+            for (int v = 0; v < 4; v++)
               #pragma unroll
-              for (int j = 0; j < JH; j++) {
+              for (int blk = 0; blk < 2; blk++) xd[blk][v] = *(const double *)(recs + (16 * u + 4 * g + v) * 32 + blk * 16);
+            auto dots = [&](int j) {
+              #pragma unroll
+              for (int b = 0; b < 4; b++) D[j & 1][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[b], B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
+            };
+            dots(0);
+            #pragma unroll
+            for (int j = 0; j < JH; j++) {
+              __builtin_amdgcn_sched_barrier(0);
+              if (j < JH - 1) dots(j + 1);
+              const gm_i32x4 (&d)[4] = D[j & 1];
+              int sc[4];
+              #pragma unroll
+              for (int k = 0; k < 4; k++) sc[k] = (int)(int8_t)(gs[j] >> (8 * k));
+              #pragma unroll
+              for (int v = 0; v < 4; v++) {
+                const int e0 = __mul24(d[0][v], sc[0]) + __mul24(d[1][v], sc[1]);
+                const int e1 = __mul24(d[2][v], sc[2]) + __mul24(d[3][v], sc[3]);
                 double &s = acc[h * JH + j][u][v];
-                if constexpr (FMT == T_Q8_0) {
-                  s = fma((double)D[j][v] * f[j][b], xd, s);
-                } else {
-                  s = fma(xd, fma(f[j][b], (double)D[j][v], -(f[j][2 + b] * dbl(rc.z, rc.w))), s);
+                s = fma(f[j][0], fma(xd[1][v], (double)e1, xd[0][v] * (double)e0), s);
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          } else {
+            #pragma unroll
+            for (int b = 0; b < 2; b++) {
+              const bool on = (g >> 1) == b;  // this lane's quarter lies in block b
+              const gm_i32x4 A = on ? gm_i32x4{(int)av.x, (int)av.y, (int)av.z, (int)av.w} : gm_i32x4{0, 0, 0, 0};
+              gm_i32x4 D[JH];
+              #pragma unroll
+              for (int j = 0; j < JH; j++) D[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B[j], gm_i32x4{0, 0, 0, 0}, 0, 0, 0);
+              #pragma unroll
+              for (int v = 0; v < 4; v++) {
+                const uint4 rc = *(const uint4 *)(recs + (16 * u + 4 * g + v) * 32 + b * 16);
+                const double xd = dbl(rc.x, rc.y);
+                #pragma unroll
+                for (int j = 0; j < JH; j++) {
+                  double &s = acc[h * JH + j][u][v];
+                  if constexpr (FMT == T_Q8_0) {
+                    s = fma((double)D[j][v] * f[j][b], xd, s);
+                  } else {
+                    s = fma(xd, fma(f[j][b], (double)D[j][v], -(f[j][2 + b] * dbl(rc.z, rc.w))), s);
+                  }
                 }
               }
             }
           }
         }
       }
-    }
-    stage_store(r + 1, h * SPH, sg);  // buffer (r + 1) & 1 was last read in round r - 1, before the previous barrier
+      stage_store(r + 1, h * SPH, sg);  // buffer (r + 1) & 1 was last read in round r - 1, before the previous barrier
     }
     __syncthreads();
   };

@@ -225,10 +225,10 @@ long gemv_part_need(const GemvArgs &a);
 // against the split taken: Q4_K gate/up 12288 x 4096 (384 workgroups, the second round half empty; 96-row blocks: 256)
 // 72 -> 55 us, 9216 x 2560 50 -> 38, q+k 5120 x 4096 30.6 -> 22.0; Q5_K 8192 x 2560 (one group) 31.6 -> 27.1, Q4_K
 // 4096 x 2560 (two, of four) 20.0 -> 15.8, attn_output 4096 x 4096 (one) 23.8 -> 22.0. 32-row blocks (8 after their
-// instruction count; where the launch is small): Q8_0 1024 x 3072 at 64 tokens 10.0 -> 6.9 us, matvec calls of Q8_0 1024 x
-// 1024 at 11 tokens 8.9 -> 7.4, Q4_K 1024 x 2560 at 11 14.4 -> 10.9, Q6_K 1024 x 4096 at 16 12.7 -> 10.3. Q6_K takes the most token groups
-// within 512 workgroups: the operands of its four dots leave no registers for more tokens (4096 x 12288 in two groups 45 us,
-// in one 72).
+// instruction count; for launches of few tiles): Q8_0 1024 x 3072 at 64 tokens 10.0 -> 6.9 us, matvec calls of Q8_0 1024 x
+// 1024 at 11 tokens 8.9 -> 7.4, Q4_K 1024 x 2560 at 11 14.4 -> 10.9, Q6_K 1024 x 4096 at 16 12.7 -> 10.3. Q6_K's tiles take
+// the most token groups within 512 workgroups: the operands of its four dots leave no registers for more tokens (4096 x
+// 12288 in two groups 45 us, in one 72).
 struct GemmPlan { int RG, U, G, blocks; };
 __host__ __device__ constexpr bool gemm_has6(int fmt) { return fmt == T_Q4_K || fmt == T_Q5_K || fmt == T_Q8_0; }
 __host__ __device__ inline int gemm_blocks6(int rows) { return (rows + 95) / 96; }
