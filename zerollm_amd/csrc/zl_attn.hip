@@ -544,11 +544,14 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
   constexpr int PPR = AV_ROW / 16;       // loads per row
   constexpr int LPT = AV_DIMS * PPR / 256;   // 16-byte loads per thread per staged piece
   constexpr int NP = 256 * NSC;          // positions per block at most
-  const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  // grid (slices, heads, chunks x tokens), chunks slowest: a row's short last chunk would otherwise take a place on a CU ahead
+  // of a whole chunk of another row
+  const int nB = gridDim.z / a.nchunk;
+  const int h = blockIdx.y, chunk = blockIdx.z / nB, b = blockIdx.z - chunk * nB, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int stB = a.step->B, stPos0 = a.step->pos0;  // the pass's step record (scalar loads, read before the pins)
   pin_args(a.hd, a.nHead, a.nHeadKv, a.layer, a.vstride, a.vcache, a.scores, a.sld, a.ctx);
   const int hd = a.hd, kvh = h / (a.nHead / a.nHeadKv), NS = hd / AV_DIMS;
-  const int slice = blockIdx.x % NS, chunk = blockIdx.x / NS;
+  const int slice = blockIdx.x;
   const int t00 = chunk * ATTN_CHUNK, ctxc = a.ctx - t00;  // the chunk's first position, cache positions from there on
   float *p = (float *)lds;               // [NP] probabilities
   uint8_t *vbuf = lds + NP * 4;          // [2][AV_DIMS][AV_PITCH] staged V rows
@@ -1164,7 +1167,7 @@ static void launch_scores_k(const AttnArgs &a, dim3 grid, int B, hipStream_t st)
 
 template <bool F16KV>
 static void launch_av_k(const AttnArgs &a, int B, hipStream_t st) {
-  const dim3 grid(a.hd / AV_DIMS * a.nchunk, a.nHead, B);
+  const dim3 grid(a.hd / AV_DIMS, a.nHead, a.nchunk * B);
   if (a.ctx <= 1024) hipLaunchKernelGGL((k_attn_av<F16KV, 4>), grid, dim3(256), attention_lds(4), st, a);
   else hipLaunchKernelGGL((k_attn_av<F16KV, 8>), grid, dim3(256), attention_lds(8), st, a);
 }
