@@ -1232,11 +1232,15 @@ void launch_attention(const AttnArgs &a0, int B, hipStream_t st) {
     // the probabilities of every row part, then the weighted sums on the matrix cores
     hipLaunchKernelGGL(k_attn_softmax_rows, dim3(a.nchunk, a.nHead, B), dim3(64), 0, st, a);
     const int nrows = group * B;
+    // blocks of 64 dimensions where the CUs hold one each (a block's chain waves share its LDS): a 509-token prompt of the 8B
+    // shapes 3446 -> 3408 us, 16 tokens of 256-dimension heads at 2K positions 21.1 -> 17.6 us; with 432 of them (9 rows at
+    // 16K positions) two layers took 480 us, in 216 of 128 dimensions 454
+    const bool narrow = a.hd == 64 || (long)a.hd / 128 * a.nHeadKv * ((nrows + MMV_RB - 1) / MMV_RB) * a.nchunk <= 128;
     if (a.kvF16) {
-      if (a.hd == 64) launch_av_mm_k<true, 2>(a, nrows, st);
+      if (narrow) launch_av_mm_k<true, 2>(a, nrows, st);
       else launch_av_mm_k<true, 4>(a, nrows, st);
     } else {
-      if (a.hd == 64) launch_av_mm_k<false, 2>(a, nrows, st);
+      if (narrow) launch_av_mm_k<false, 2>(a, nrows, st);
       else launch_av_mm_k<false, 4>(a, nrows, st);
     }
     ZL_HIP(hipGetLastError());
