@@ -861,8 +861,11 @@ __global__ __launch_bounds__(NDG * 192, NDG * 6 / 4) void k_attn_av_mm(const Att
     const int pt = tid - NDG * 64;                  // producer thread 0 .. NPT - 1
     const int pr = pt * PN / CT, pq = pt * PN % CT; // its row and first position of its PN probabilities in a piece
     const int np = rnp[pr];
-    // both by buffer loads: the thread's offset in registers, the piece's in a scalar, and no branch around a load (past
-    // the V rows and the pass's scores zeros, without an access), so that the waits count exactly the piece they are for
+    // both by buffer loads and no branch around a load, so that the waits count exactly the piece they are for. Up to D
+    // pieces past the block's last one are requested (and never staged), so a load's whole offset, the piece's part
+    // included, is its vector offset: that is what the range check compares with the resource's size (the end of the V
+    // rows and of the pass's scores), and past it a load returns zeros without an access. A scalar offset may be left
+    // out of that comparison, or be larger than the resource.
     const uint32_t vrow = (uint32_t)a.vstride * VB;
     const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc((void *)vbase, (short)0, (int)(DB * vrow - t00 * VB), 0x00020000);
     const long pend = (long)Bd * a.nHead * a.sld - r00;  // floats from the block's first row on
@@ -876,15 +879,16 @@ __global__ __launch_bounds__(NDG * 192, NDG * 6 / 4) void k_attn_av_mm(const Att
     };
     // piece c's V and scores (what lies past a row's or the pass's last position is zeroed when the piece is staged)
     auto fetch = [&](int c, Pre &s) {
+      const uint32_t t0 = (uint32_t)c * CT;
       #pragma unroll
       for (int k = 0; k < VU; k++) {
         const int u = k * NPT + pt, dim = u / UPR;
+        const uint32_t vo = dim * vrow + (t0 + (u % UPR) * 16) * VB;
         #pragma unroll
-        for (int l = 0; l < UL; l++)
-          s.v[k][l] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(vr, dim * vrow + ((u % UPR) * 16 + l * EPP) * VB, c * CT * VB, 0));
+        for (int l = 0; l < UL; l++) s.v[k][l] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(vr, vo + l * 16, 0, 0));
       }
       #pragma unroll
-      for (int j = 0; j < PN; j++) s.p[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(pr_, poff + 4 * j, c * CT * 4, 0));
+      for (int j = 0; j < PN; j++) s.p[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(pr_, poff + t0 * 4 + 4 * j, 0, 0));
     };
     auto stage_f = [&](auto whole, int c, const Pre &s) {
       constexpr bool W = decltype(whole)::value;
