@@ -1,0 +1,68 @@
+"""Rows of several 2048-position chunks against the softmax over the whole row in float64 (attention_tables), in passes of
+one token (lane chains), 16 and 64 tokens (matrix cores)."""
+import numpy as np
+import pytest
+
+from attention_tables import IDS, Tables
+
+pytestmark = pytest.mark.gpu
+
+ORDINARY = IDS - 8  # ids below it have the tables' random rows; those from it on are set by the tests
+
+
+def rows_of(m, ids, first, n):
+    """Logits of positions `first`.. in passes of n tokens."""
+    m.truncate(0)
+    for i in range(0, first, 64):
+        m.forward_batch(ids[i:min(i + 64, first)], logits="none")
+    return np.concatenate([m.forward_batch(ids[i:i + n], logits="all").copy() for i in range(first, len(ids), n)])
+
+
+def special(case, t, ids):
+    """Sets the tables' special ids and places them; the rows whose outputs must not be finite."""
+    a, b = ORDINARY, ORDINARY + 1
+    t.k[:ORDINARY, -2:] = 0.25
+    t.q[:, :, -2:] = 1.0
+    if case == "a chunk of NaN":
+        # the last key overflows the f16 cache in two dimensions of opposite signs: inf - inf, alone in its chunk
+        t.k[a, -2:] = 1e5, -1e5
+        ids[2048] = a
+    elif case == "first chunk -inf":
+        t.k[a, -1] = -1e5
+        ids[:2048] = a
+    elif case == "middle chunk -inf":
+        t.k[a, -1] = -1e5
+        ids[2048:4096] = a
+    elif case == "every chunk -inf":
+        t.k[a, -1] = -1e5
+        ids[:] = a
+    elif case == "inf at weight 0":
+        # one value overflows in a chunk whose scores lie 1000 below the others': 0 times inf
+        t.q[:, :, -1] = 100.0
+        t.k[:ORDINARY, -1] = 0.0
+        t.k[a], t.k[b] = t.k[0], t.k[1]
+        t.k[[a, b], -1] = -10.0 * np.sqrt(t.hd)
+        t.v[b, 3] = 1e5
+        ids[:2048] = a
+        ids[1000] = b
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("case,length", [("a chunk of NaN", 2049), ("a chunk of NaN", 2064), ("first chunk -inf", 2700),
+                                         ("middle chunk -inf", 4200), ("every chunk -inf", 2060), ("inf at weight 0", 2700)])
+def test_infinities_and_nan_are_those_of_the_whole_row(gpu, monkeypatch, tmp_path, case, length, head_dim):
+    t = Tables(head_dim, 3)
+    ids = np.random.default_rng(4).integers(0, ORDINARY, length)
+    special(case, t, ids)
+    first = max(length - 16, 2048)
+    m = t.load(monkeypatch, str(tmp_path / "t.gguf"), ctx=length + 3, kv="f16")
+    want = t.exact(ids, range(first, length))
+    for n in (1, 16, 64):
+        print(f"case {case} head {head_dim} passes of {n}", flush=True)
+        got = rows_of(m, ids.tolist(), first, n)
+        bad = ~np.isfinite(want).all(1)
+        assert bad.all() == (case in ("a chunk of NaN", "every chunk -inf", "inf at weight 0")) and bad.all() == bad.any()
+        assert (np.isfinite(got).all(1) == ~bad).all(), n
+        if not bad.any():
+            assert np.abs(t.outputs(got, ids[first:]) - want).max() <= 1e-5 * np.abs(want).max()
+    m.close()

@@ -460,6 +460,11 @@ __device__ __forceinline__ double exp_neg(double x) {
 // position alone and a token gets the same bits in a pass of any size. Against float64 the joined chunks are closer than
 // the single f32 chain, whose rounding errors grow with its length.
 //
+// Infinities and NaN come out as in a softmax over the whole row. A chunk of a longer row without a score above -inf is
+// taken against 0 in place of its maximum (chunk_max), so l_c and the probabilities are 0 where every score is -inf
+// (which counts for nothing beside a finite score elsewhere, except that 0 times a V of inf or NaN is NaN) and NaN where
+// one is NaN. No chunk is left out for a weight of 0.
+//
 // A chunk of a longer row leaves a record [m_c, l_c (lane chains), o_c of 32 dimensions] in a.rec ([token][head][32-dimension slice]
 // [chunk]); the block that arrives last at the counter of its (token, head, slice) or row block joins them. The hand-off
 // is that of the GEMV's K parts: device-coherent stores, complete (vmcnt(0)) before the relaxed arrival, device-coherent
@@ -473,9 +478,11 @@ __device__ __forceinline__ void chunk_store(double *r, int lane, double m, doubl
   __hip_atomic_store((float *)(r + 2) + lane, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (lane < 2) __hip_atomic_store(r + lane, lane == 0 ? m : l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// what a chunk's exponentials are taken against, and 1 / sum of them
+__device__ __forceinline__ double chunk_max(double m, int nrow) { return nrow > ATTN_CHUNK && m == -INFINITY ? 0.0 : m; }
+__device__ __forceinline__ double chunk_inv(double l) { return l == 0.0 ? 0.0 : 1.0 / l; }
 // The joined outputs of dimension `lane` (32 consecutive lanes) of NS neighbouring slices of n chunks' records at r
-// (slices lds apart); ml(c) gives chunk c's (m, l). A chunk whose scores are all -inf counts for nothing beside one that
-// has a finite score (the reference's e of such a position is 0).
+// (slices lds apart); ml(c) gives chunk c's (m, l).
 template <int NS, typename ML>
 __device__ __forceinline__ void chunk_join(const double *r, long lds, int n, int lane, const ML &ml, float (&out)[NS]) {
   constexpr int NJ = NS > 1 ? 4 : 8;  // chunks whose loads are issued together
@@ -488,7 +495,7 @@ __device__ __forceinline__ void chunk_join(const double *r, long lds, int n, int
   for (int c0 = 0; c0 < n; c0 += 32) {
     const int nc = min(32, n - c0);
     const double2 v = ml(min(c0 + lane, n - 1));
-    const double w = v.x == -INFINITY && M != -INFINITY ? 0.0 : exp(v.x - (double)M) * v.y;
+    const double w = v.x == -INFINITY && M != -INFINITY ? v.y : exp(v.x - (double)M) * v.y;  // (l = 0 or NaN there)
     for (int j0 = 0; j0 < nc; j0 += NJ) {
       float o[NS][NJ];
       #pragma unroll
@@ -500,7 +507,7 @@ __device__ __forceinline__ void chunk_join(const double *r, long lds, int n, int
       #pragma unroll
       for (int j = 0; j < NJ; j++) {
         const double wj = __shfl(w, min(j0 + j, nc - 1), 32);
-        if (j0 + j < nc && wj != 0.0) {
+        if (j0 + j < nc) {
           L += wj;
           #pragma unroll
           for (int i = 0; i < NS; i++) O[i] = fma(wj, (double)o[i][j], O[i]);
@@ -602,14 +609,14 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
   mx = group_fmax(mx, 64);
   if (lane == 0) redf[wave] = mx;
   __syncthreads();
-  const double m = (double)fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
+  const double m = (double)fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3])), mz = chunk_max(m, nrow);
   double sum = 0.0;
   #pragma unroll
   for (int k0 = 0; k0 < NSC; k0 += 4) {
     if (k0 * 256 < npos) {  // (uniform)
       double e[4];  // four independent chains
       #pragma unroll
-      for (int k = 0; k < 4; k++) e[k] = exp_neg((double)v[k0 + k] - m);
+      for (int k = 0; k < 4; k++) e[k] = exp_neg((double)v[k0 + k] - mz);
       #pragma unroll
       for (int k = 0; k < 4; k++) {
         const bool on = (k0 + k) * 256 + tid < npos;
@@ -621,7 +628,7 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
   sum = wave_sum_xor(sum, 64);
   if (lane == 0) redd[wave] = sum;
   __syncthreads();
-  const double l = (redd[0] + redd[1]) + (redd[2] + redd[3]), inv = 1.0 / l;
+  const double l = (redd[0] + redd[1]) + (redd[2] + redd[3]), inv = chunk_inv(l);
   #pragma unroll
   for (int k = 0; k < NSC; k++) {  // (zeros from the last position to the end of its unit, at least)
     const int t = k * 256 + tid;
@@ -732,7 +739,7 @@ __global__ __launch_bounds__(64) void k_attn_softmax_rows(const AttnArgs a) {
   constexpr int NK = ATTN_CHUNK / 64;
   const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
   const Step *st = a.step;
-  const int t00 = chunk * ATTN_CHUNK, npos = min(st->pos0 + b + 1 - t00, ATTN_CHUNK);
+  const int t00 = chunk * ATTN_CHUNK, nrow = st->pos0 + b + 1, npos = min(nrow - t00, ATTN_CHUNK);
   if (b >= st->B || npos <= 0) return;
   float *srow = a.scores + ((long)b * a.nHead + h) * a.sld + t00;
   float v[NK], mx = -INFINITY;
@@ -749,14 +756,14 @@ __global__ __launch_bounds__(64) void k_attn_softmax_rows(const AttnArgs a) {
       for (int j = k; j < k + 8; j++) mx = fmaxf(mx, v[j]);
     }
   mx = group_fmax(mx, 64);
-  const double m = (double)mx;
+  const double m = (double)mx, mz = chunk_max(m, nrow);
   double sum[4] = {0.0, 0.0, 0.0, 0.0};
   #pragma unroll
   for (int k = 0; k < NK; k += 4)
     if (k * 64 < npos) {  // positions 256 (k / 4) + 64 w + lane of the four waves w
       double e[4];
       #pragma unroll
-      for (int w = 0; w < 4; w++) e[w] = exp_neg((double)v[k + w] - m);
+      for (int w = 0; w < 4; w++) e[w] = exp_neg((double)v[k + w] - mz);
       #pragma unroll
       for (int w = 0; w < 4; w++) {
         if ((k + w) * 64 + lane < npos) sum[w] += e[w];
@@ -765,7 +772,7 @@ __global__ __launch_bounds__(64) void k_attn_softmax_rows(const AttnArgs a) {
     }
   #pragma unroll
   for (int w = 0; w < 4; w++) sum[w] = wave_sum_xor(sum[w], 64);
-  const double l = (sum[0] + sum[1]) + (sum[2] + sum[3]), inv = 1.0 / l;
+  const double l = (sum[0] + sum[1]) + (sum[2] + sum[3]), inv = chunk_inv(l);
   #pragma unroll
   for (int k = 0; k < NK; k += 4)
     if (k * 64 < npos) {
