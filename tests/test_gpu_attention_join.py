@@ -66,3 +66,25 @@ def test_infinities_and_nan_are_those_of_the_whole_row(gpu, monkeypatch, tmp_pat
         if not bad.any():
             assert np.abs(t.outputs(got, ids[first:]) - want).max() <= 1e-5 * np.abs(want).max()
     m.close()
+
+
+@pytest.mark.parametrize("kv", ["f16", "f32"])
+@pytest.mark.parametrize("ctx,at", [(1024, 300), (4224, 300), (4224, 2050), (4224, 2500)])
+def test_values_of_discarded_tokens_stay_out(gpu, monkeypatch, tmp_path, ctx, at, kv):
+    """Values of tokens that were dropped again lie in the cache past a row's last position, in the same 16 bytes as its own:
+    infinite ones there change nothing (the row has `at` + 1 positions)."""
+    t = Tables(64, 5)
+    t.v[ORDINARY, ::3] = 1e5 if kv == "f16" else 4e39  # (4e39: the product overflows float32, its weight does not)
+    ids = np.random.default_rng(6).integers(0, ORDINARY, at + 2)
+    m = t.load(monkeypatch, str(tmp_path / "t.gguf"), ctx=ctx, kv=kv)
+    want = t.exact(ids, [at, at + 1])
+    for n in (1, 2):
+        print(f"case discarded values after {at} of {ctx} kv {kv} passes of {n}", flush=True)
+        m.truncate(0)
+        for i in range(0, at, 64):
+            m.forward_batch(ids[i:min(i + 64, at)].tolist(), logits="none")
+        m.forward_batch([ORDINARY] * 9, logits="none")
+        m.truncate(at)
+        got = np.concatenate([m.forward_batch(ids[i:i + n].tolist(), logits="all").copy() for i in range(at, at + 2, n)])
+        assert np.abs(t.outputs(got, ids[at:]) - want).max() <= 1e-5 * np.abs(want).max(), n
+    m.close()

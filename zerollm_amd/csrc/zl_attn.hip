@@ -634,21 +634,19 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
     const int t = k * 256 + tid;
     if (k * 256 < npos) p[t] = t < npos ? (float)((double)v[k] * inv) : 0.f;
   }
-  #pragma unroll
-  for (int k = 0; k < LPT; k++) {  // the first piece from the last position on: zeros, as in later ones
-    const int t = ((k * 256 + tid) % PPR) * EPP;
-    if (t >= npos) pre[k] = make_uint4(0, 0, 0, 0);
-    else if (t + EPP > npos) {
-      uint32_t w[4] = {pre[k].x, pre[k].y, pre[k].z, pre[k].w};
-      #pragma unroll
-      for (int e = 0; e < EPP; e++)
-        if (t + e >= npos) {
-          if (F16KV) w[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
-          else w[e] = 0u;
-        }
-      pre[k] = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-  }
+  // the last piece from the last position on: zeros (the cache may hold anything there, inf and NaN of a discarded token
+  // included, and a probability of 0 does not take those out of the sum); a thread's loads are of the same positions of
+  // different dimensions
+  auto trim = [&](int c) {
+    static_assert(256 % PPR == 0, "one set of positions per thread");
+    const int r = npos - c * CT - (tid % PPR) * EPP;  // how many of them lie below the last position
+    uint32_t w[4];
+    #pragma unroll
+    for (int e = 0; e < 4; e++) w[e] = !F16KV ? (r > e ? ~0u : 0u) : r > 2 * e + 1 ? ~0u : r > 2 * e ? 0xffffu : 0u;
+    #pragma unroll
+    for (int k = 0; k < LPT; k++) pre[k] = make_uint4(pre[k].x & w[0], pre[k].y & w[1], pre[k].z & w[2], pre[k].w & w[3]);
+  };
+  if (nch == 1) trim(0);
   store(0);
   __syncthreads();
   // ---- weighted sum of V: f32 fma chain in position order, one output dimension per lane (lanes 0-31 of wave 0)
@@ -659,8 +657,8 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
     if (chainLane) {
       // units of UNIT positions, software pipelined: the LDS reads of unit u + 1 are issued before the fma steps of
       // unit u, so the chain (one dependent fma per position, ~2.2 ns each) does not wait out an LDS latency per unit.
-      // p is zero past the last position, so a unit may run past `cnt`: fmaf(0, v, o) == o for the finite cached
-      // values read there. The read-ahead index is clamped to the chunk's last unit (a re-read, never past it).
+      // p and V are zero past the last position, so a unit may run past `cnt`: fmaf(0, 0, o) == o. The read-ahead index
+      // is clamped to the chunk's last unit (a re-read, never past it).
       const int t0 = c * CT, cnt = min(CT, npos - t0), nu = (cnt + AV_UNIT - 1) / AV_UNIT;
       const uint8_t *row = vbuf + (c & 1) * AV_STAGE + lane * AV_PITCH;
       const float *pc = p + t0;
@@ -703,7 +701,10 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
       if (u < nu) steps(pa, va);
     }
     __syncthreads();
-    if (c + 1 < nch) store((c + 1) & 1);
+    if (c + 1 < nch) {
+      if (c + 2 == nch) trim(c + 1);
+      store((c + 1) & 1);
+    }
     __syncthreads();
   }
   if (!chainLane) return;
