@@ -24,7 +24,7 @@ class Tables:
 
     def load(self, monkeypatch, path, **kw):
         hd, d = self.hd, IDS + HEADS * self.hd
-        spec = synth.build_spec("llama", d, 1, HEADS, 1, hd, 32, d, 32768, synth.all_type(gguf.F32), 1)
+        spec = synth.build_spec("llama", d, 1, HEADS, 1, hd, 32, d, 1 << 18, synth.all_type(gguf.F32), 1)
         spec.rope_base = 1e30
         x = 1.0 / np.sqrt(1.0 / d + spec.rms_eps)  # the normed embedding's one value
         w = {t.name: np.zeros((t.rows, t.cols), np.float32) for t in spec.tensors}

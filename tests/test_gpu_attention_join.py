@@ -88,3 +88,26 @@ def test_values_of_discarded_tokens_stay_out(gpu, monkeypatch, tmp_path, ctx, at
         got = np.concatenate([m.forward_batch(ids[i:i + n].tolist(), logits="all").copy() for i in range(at, at + 2, n)])
         assert np.abs(t.outputs(got, ids[at:]) - want).max() <= 1e-5 * np.abs(want).max(), n
     m.close()
+
+
+@pytest.mark.parametrize("head_dim,kv", [(64, "f16"), (128, "f16"), (128, "f32")])
+def test_rows_of_more_chunks_than_have_blocks_of_their_own(gpu, monkeypatch, tmp_path, head_dim, kv):
+    """Rows on both sides of 16, 17 and 18 chunks (blocks then walk two of them), and short rows of the same large cache."""
+    t = Tables(head_dim, 8)
+    ids = np.random.default_rng(9).integers(0, IDS, 36870)
+    m = t.load(monkeypatch, str(tmp_path / "t.gguf"), ctx=36900, kv=kv)
+    spans = [(700, 716), (4090, 4106), (32760, 32776), (34810, 34826), (36854, 36870)]
+    got = {}
+    for n in (1, 5, 16):
+        print(f"case more chunks than blocks head {head_dim} kv {kv} passes of {n}", flush=True)
+        m.truncate(0)
+        at = 0
+        for a, b in spans:
+            for i in range(at, a, 64):
+                m.forward_batch(ids[i:min(i + 64, a)].tolist(), logits="none")
+            rows = np.concatenate([m.forward_batch(ids[i:min(i + n, b)].tolist(), logits="all").copy() for i in range(a, b, n)])
+            at = b
+            want = t.exact(ids, range(a, b))
+            assert np.abs(t.outputs(rows, ids[a:b]) - want).max() <= 1e-5 * np.abs(want).max(), (n, a)
+            assert (rows.view(np.uint32) == got.setdefault(a, rows).view(np.uint32)).all(), (n, a)
+    m.close()

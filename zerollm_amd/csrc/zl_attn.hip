@@ -470,6 +470,19 @@ __device__ __forceinline__ double exp_neg(double x) {
 // is that of the GEMV's K parts: device-coherent stores, complete (vmcnt(0)) before the relaxed arrival, device-coherent
 // loads by the last.
 constexpr int REC_D = ATTN_REC_DOUBLES;
+// Chunks of a row that have blocks of their own. The blocks of caches of more chunks walk several (WALK: chunks z, z + 16,
+// ...), so a launch stops growing with the cache's capacity: with a block per chunk a token at position 700 of a cache of
+// 262,144 cost 4 layers of the 0.6B shapes 299 us where one of 1024 costs 176. The kernels below that have no loop over
+// chunks, whose registers (constants kept across the chunks) would cost occupancy: k_attn_av 143 -> 175.
+constexpr int ATTN_ZMAX = 16;
+// The thread's index, in a walk as a value of its own in every chunk, so that what follows from it is formed there and not
+// kept in registers across the chunks.
+template <bool WALK>
+__device__ __forceinline__ int thread_index() {
+  int t = threadIdx.x;
+  if constexpr (WALK) __asm__ volatile("" : "+v"(t));
+  return t;
+}
 __device__ __forceinline__ double *chunk_rec(const AttnArgs &a, int b, int h, int slice, int c) {
   return a.rec + ((((long)b * a.nHead + h) * (a.hd >> 5) + slice) * a.nchunk + c) * REC_D;
 }
@@ -542,21 +555,15 @@ constexpr int AV_STAGE = AV_DIMS * AV_PITCH;
 constexpr int AV_UNIT = 32;       // positions per unrolled step of the weighted sum
 
 // NSC: scores per thread (256 NSC >= the positions of a chunk), held in registers from the load to the probabilities
-template <bool F16KV, int NSC>
-__global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
-  extern __shared__ __align__(16) uint8_t lds[];
+template <bool F16KV, int NSC, bool WALK>
+__device__ __forceinline__ void av_chunk(const AttnArgs &a, int chunk, int b, int stB, int stPos0, uint8_t *lds) {
   constexpr int VB = F16KV ? 2 : 4;
   constexpr int CT = AV_ROW / VB;        // positions per staged piece
   constexpr int EPP = 16 / VB;           // positions per 16-byte load
   constexpr int PPR = AV_ROW / 16;       // loads per row
   constexpr int LPT = AV_DIMS * PPR / 256;   // 16-byte loads per thread per staged piece
   constexpr int NP = 256 * NSC;          // positions per block at most
-  // grid (slices, heads, chunks x tokens), chunks slowest: a row's short last chunk would otherwise take a place on a CU ahead
-  // of a whole chunk of another row
-  const int nB = gridDim.z / a.nchunk;
-  const int h = blockIdx.y, chunk = blockIdx.z / nB, b = blockIdx.z - chunk * nB, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int stB = a.step->B, stPos0 = a.step->pos0;  // the pass's step record (scalar loads, read before the pins)
-  pin_args(a.hd, a.nHead, a.nHeadKv, a.layer, a.vstride, a.vcache, a.scores, a.sld, a.ctx);
+  const int h = blockIdx.y, tid = thread_index<WALK>(), wave = tid >> 6, lane = tid & 63;
   const int hd = a.hd, kvh = h / (a.nHead / a.nHeadKv), NS = hd / AV_DIMS;
   const int slice = blockIdx.x;
   const int t00 = chunk * ATTN_CHUNK, ctxc = a.ctx - t00;  // the chunk's first position, cache positions from there on
@@ -732,58 +739,83 @@ __global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a) {
   attn_emit(a, b, h, slice * AV_DIMS + lane, out[0]);
 }
 
+// Grid (slices, heads, nz x tokens), chunks slowest (a row's short last chunk would otherwise take a place on a CU ahead of
+// a whole chunk of another row). Chunk 0's first loads go out before the pass's step record arrives; a block of a later
+// chunk waits for the record, as in a cache longer than the row it has nothing to load.
+template <bool F16KV, int NSC, bool WALK>
+__global__ __launch_bounds__(256) void k_attn_av(const AttnArgs a, int nB, int nz) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int z = blockIdx.z / nB, b = blockIdx.z - z * nB;
+  const int stB = a.step->B, stPos0 = a.step->pos0;  // the pass's step record (scalar loads, read before the pins)
+  pin_args(a.hd, a.nHead, a.nHeadKv, a.layer, a.vstride, a.vcache, a.scores, a.sld, a.ctx);
+  for (int chunk = z;; chunk += nz) {
+    if (chunk > 0) {
+      __asm__ volatile("");  // (keeps the test of the record a branch of its own: chunk 0 does not wait for it)
+      if (b >= stB || chunk * ATTN_CHUNK > stPos0 + b) return;
+    }
+    av_chunk<F16KV, NSC, WALK>(a, chunk, b, stB, stPos0, lds);
+    if (!WALK) return;
+  }
+}
+
 // The probabilities of every (chunk, query head, token) part of a pass of several tokens, in place of its scores, and its
 // (m_c, l_c). One wave per part: lane i takes k_attn_av's threads i, i + 64, i + 128 and i + 192 (their positions in their
 // order, then the same four 64-lane sums and (w0 + w1) + (w2 + w3)), so a part has one maximum and no barrier. Bound by
 // the f64 exponentials (~30 VALU instructions a position); with four waves per part their reductions cost as much again.
+template <bool WALK>
 __global__ __launch_bounds__(64) void k_attn_softmax_rows(const AttnArgs a) {
   constexpr int NK = ATTN_CHUNK / 64;
-  const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
+  const int h = blockIdx.y, b = blockIdx.z;
   const Step *st = a.step;
-  const int t00 = chunk * ATTN_CHUNK, nrow = st->pos0 + b + 1, npos = min(nrow - t00, ATTN_CHUNK);
-  if (b >= st->B || npos <= 0) return;
-  float *srow = a.scores + ((long)b * a.nHead + h) * a.sld + t00;
-  float v[NK], mx = -INFINITY;
-  #pragma unroll
-  for (int k = 0; k < NK; k += 8)
-    if (k * 64 < npos) {  // (uniform; a position past the last repeats the first)
-      #pragma unroll
-      for (int j = k; j < k + 8; j++) { const int t = j * 64 + lane; v[j] = srow[t < npos ? t : 0]; }
-    }
-  #pragma unroll
-  for (int k = 0; k < NK; k += 8)
-    if (k * 64 < npos) {
-      #pragma unroll
-      for (int j = k; j < k + 8; j++) mx = fmaxf(mx, v[j]);
-    }
-  mx = group_fmax(mx, 64);
-  const double m = (double)mx, mz = chunk_max(m, nrow);
-  double sum[4] = {0.0, 0.0, 0.0, 0.0};
-  #pragma unroll
-  for (int k = 0; k < NK; k += 4)
-    if (k * 64 < npos) {  // positions 256 (k / 4) + 64 w + lane of the four waves w
-      double e[4];
-      #pragma unroll
-      for (int w = 0; w < 4; w++) e[w] = exp_neg((double)v[k + w] - mz);
-      #pragma unroll
-      for (int w = 0; w < 4; w++) {
-        if ((k + w) * 64 + lane < npos) sum[w] += e[w];
-        v[k + w] = (float)e[w];
+  const int nrow = st->pos0 + b + 1;
+  if (b >= st->B) return;
+  for (int chunk = blockIdx.x; chunk * ATTN_CHUNK < nrow; chunk += gridDim.x) {
+    const int lane = thread_index<WALK>();
+    const int t00 = chunk * ATTN_CHUNK, npos = min(nrow - t00, ATTN_CHUNK);
+    float *srow = a.scores + ((long)b * a.nHead + h) * a.sld + t00;
+    float v[NK], mx = -INFINITY;
+    #pragma unroll
+    for (int k = 0; k < NK; k += 8)
+      if (k * 64 < npos) {  // (uniform; a position past the last repeats the first)
+        #pragma unroll
+        for (int j = k; j < k + 8; j++) { const int t = j * 64 + lane; v[j] = srow[t < npos ? t : 0]; }
       }
-    }
-  #pragma unroll
-  for (int w = 0; w < 4; w++) sum[w] = wave_sum_xor(sum[w], 64);
-  const double l = (sum[0] + sum[1]) + (sum[2] + sum[3]), inv = chunk_inv(l);
-  #pragma unroll
-  for (int k = 0; k < NK; k += 4)
-    if (k * 64 < npos) {
-      #pragma unroll
-      for (int j = k; j < k + 4; j++) {
-        const int t = j * 64 + lane;
-        if (t < npos) srow[t] = (float)((double)v[j] * inv);
+    #pragma unroll
+    for (int k = 0; k < NK; k += 8)
+      if (k * 64 < npos) {
+        #pragma unroll
+        for (int j = k; j < k + 8; j++) mx = fmaxf(mx, v[j]);
       }
-    }
-  if (lane == 0) a.cml[((long)b * a.nHead + h) * a.nchunk + chunk] = make_double2(m, l);
+    mx = group_fmax(mx, 64);
+    const double m = (double)mx, mz = chunk_max(m, nrow);
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    #pragma unroll
+    for (int k = 0; k < NK; k += 4)
+      if (k * 64 < npos) {  // positions 256 (k / 4) + 64 w + lane of the four waves w
+        double e[4];
+        #pragma unroll
+        for (int w = 0; w < 4; w++) e[w] = exp_neg((double)v[k + w] - mz);
+        #pragma unroll
+        for (int w = 0; w < 4; w++) {
+          if ((k + w) * 64 + lane < npos) sum[w] += e[w];
+          v[k + w] = (float)e[w];
+        }
+      }
+    #pragma unroll
+    for (int w = 0; w < 4; w++) sum[w] = wave_sum_xor(sum[w], 64);
+    const double l = (sum[0] + sum[1]) + (sum[2] + sum[3]), inv = chunk_inv(l);
+    #pragma unroll
+    for (int k = 0; k < NK; k += 4)
+      if (k * 64 < npos) {
+        #pragma unroll
+        for (int j = k; j < k + 4; j++) {
+          const int t = j * 64 + lane;
+          if (t < npos) srow[t] = (float)((double)v[j] * inv);
+        }
+      }
+    if (lane == 0) a.cml[((long)b * a.nHead + h) * a.nchunk + chunk] = make_double2(m, l);
+    if (!WALK) return;
+  }
 }
 
 // ---- weighted sum of passes of several tokens on the matrix cores. v_mfma_f32_16x16x4_f32 adds its four products to
@@ -805,9 +837,8 @@ constexpr int MMV_RB = 16;                  // rows per block
 constexpr int MMV_CT = 64;                  // positions per staged piece
 constexpr int MMV_SF = MMV_CT / 4;          // floats of one position section
 constexpr int MMV_RS = 4 * MMV_SF + 4;      // floats of one dimension or row (4 x an odd number: conflict-free chain reads)
-template <bool F16KV, int NDG>
-__global__ __launch_bounds__(NDG * 192, NDG * 6 / 4) void k_attn_av_mm(const AttnArgs a, int nrows) {
-  extern __shared__ __align__(16) uint8_t lds[];
+template <bool F16KV, int NDG, bool WALK>
+__device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int chunk, int L, uint8_t *lds) {
   typedef float f4 __attribute__((ext_vector_type(4)));
   constexpr int VB = F16KV ? 2 : 4, DB = 32 * NDG, RB = MMV_RB;
   constexpr int CT = MMV_CT, SF = MMV_SF, RS = MMV_RS, NPT = NDG * 128;
@@ -823,20 +854,14 @@ __global__ __launch_bounds__(NDG * 192, NDG * 6 / 4) void k_attn_av_mm(const Att
   __shared__ long roff[RB];
   __shared__ int rnp[RB], rfull[RB];                // the row's positions in the chunk, and in all
   __shared__ uint32_t arrived;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n16 = lane & 15, g = lane >> 4;
-  // XCD-aware block order: workgroup i of a chunk's blocks (a multiple of 8) goes to XCD i mod 8, and logical block
-  // L = (i mod 8) (blocks / 8) + i / 8 gives each XCD a contiguous run of L, ordered dimension block fastest, then row
-  // block, then KV head, so the blocks that read the same V share one L2
+  const int tid = thread_index<WALK>(), lane = tid & 63, wave = tid >> 6, n16 = lane & 15, g = lane >> 4;
   const int ND = a.hd / DB, NZ = (nrows + RB - 1) / RB;
-  const int L = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  if (L >= ND * NZ * a.nHeadKv) return;
   const int kvh = L / (ND * NZ), rbk = (L / ND) % NZ, d0 = (L % ND) * DB;
   const int G = a.nHead / a.nHeadKv;
   const Step *st = a.step;
   // positions below are relative to the chunk's first one, t00
-  const int chunk = blockIdx.y, t00 = chunk * ATTN_CHUNK;
+  const int t00 = chunk * ATTN_CHUNK;
   const int Bd = st->B, pos0 = st->pos0, nmax = pos0 + Bd - t00;
-  if (nmax <= 0) return;
   // the block's rows: scores row offsets, positions (0: no row; such a row reads the block's first one)
   const long r0h = ((long)(rbk * RB / G) * a.nHead + kvh * G) * a.sld, r00 = r0h + t00;
   if (tid < RB) {
@@ -1017,6 +1042,23 @@ __global__ __launch_bounds__(NDG * 192, NDG * 6 / 4) void k_attn_av_mm(const Att
   }
 }
 
+// Grid (blocks of a chunk, nz chunks).
+// XCD-aware block order: workgroup i of a chunk's blocks (a multiple of 8) goes to XCD i mod 8, and logical block
+// L = (i mod 8) (blocks / 8) + i / 8 gives each XCD a contiguous run of L, ordered dimension block fastest, then row block,
+// then KV head, so the blocks that read the same V share one L2
+template <bool F16KV, int NDG, bool WALK>
+__global__ __launch_bounds__(NDG * 192, NDG * 6 / 4) void k_attn_av_mm(const AttnArgs a, int nrows) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int L = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (L >= a.hd / (32 * NDG) * ((nrows + MMV_RB - 1) / MMV_RB) * a.nHeadKv) return;
+  const int nmax = a.step->pos0 + a.step->B;
+  for (int chunk = blockIdx.y; chunk * ATTN_CHUNK < nmax; chunk += gridDim.y) {
+    av_mm_chunk<F16KV, NDG, WALK>(a, nrows, chunk, L, lds);
+    if (!WALK) return;
+    __syncthreads();  // the chunk's LDS has been read
+  }
+}
+
 static size_t attention_av_mm_lds(int ndg) { return (size_t)2 * (32 * ndg + MMV_RB) * MMV_RS * 4; }
 
 // ---- position-split weighted sum (long contexts). The exact chain above runs one dependent f32 step per position, so
@@ -1131,16 +1173,22 @@ AttnForm attention_form(int ctx) {
   return f;
 }
 
-template <bool F16KV, int NDG>
-static void launch_av_mm_k(const AttnArgs &a, int nrows, hipStream_t st) {
+template <bool F16KV, int NDG, bool WALK>
+static void launch_av_mm_w(const AttnArgs &a, int nrows, hipStream_t st) {
   static bool attr = false;  // dynamic LDS above 64 KB must be requested per kernel
+  const size_t lds = attention_av_mm_lds(NDG);
   if (!attr) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_mm<F16KV, NDG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)attention_av_mm_lds(NDG)));
+    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_mm<F16KV, NDG, WALK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr = true;
   }
   const int nb = a.hd / (32 * NDG) * a.nHeadKv * ((nrows + MMV_RB - 1) / MMV_RB);  // (dimensions, KV head, rows) blocks
-  const dim3 grid((nb + 7) / 8 * 8, a.nchunk);
-  hipLaunchKernelGGL((k_attn_av_mm<F16KV, NDG>), grid, dim3(NDG * 192), attention_av_mm_lds(NDG), st, a, nrows);
+  const dim3 grid((nb + 7) / 8 * 8, std::min(a.nchunk, ATTN_ZMAX));
+  hipLaunchKernelGGL((k_attn_av_mm<F16KV, NDG, WALK>), grid, dim3(NDG * 192), lds, st, a, nrows);
+}
+template <bool F16KV, int NDG>
+static void launch_av_mm_k(const AttnArgs &a, int nrows, hipStream_t st) {
+  if (a.nchunk > ATTN_ZMAX) launch_av_mm_w<F16KV, NDG, true>(a, nrows, st);
+  else launch_av_mm_w<F16KV, NDG, false>(a, nrows, st);
 }
 
 template <int HD, bool F16KV>
@@ -1179,9 +1227,11 @@ static void launch_scores_k(const AttnArgs &a, dim3 grid, int B, hipStream_t st)
 
 template <bool F16KV>
 static void launch_av_k(const AttnArgs &a, int B, hipStream_t st) {
-  const dim3 grid(a.hd / AV_DIMS, a.nHead, a.nchunk * B);
-  if (a.ctx <= 1024) hipLaunchKernelGGL((k_attn_av<F16KV, 4>), grid, dim3(256), attention_lds(4), st, a);
-  else hipLaunchKernelGGL((k_attn_av<F16KV, 8>), grid, dim3(256), attention_lds(8), st, a);
+  const int nz = std::min(a.nchunk, ATTN_ZMAX);
+  const dim3 grid(a.hd / AV_DIMS, a.nHead, nz * B);
+  if (a.ctx <= 1024) hipLaunchKernelGGL((k_attn_av<F16KV, 4, false>), grid, dim3(256), attention_lds(4), st, a, B, nz);
+  else if (a.nchunk <= ATTN_ZMAX) hipLaunchKernelGGL((k_attn_av<F16KV, 8, false>), grid, dim3(256), attention_lds(8), st, a, B, nz);
+  else hipLaunchKernelGGL((k_attn_av<F16KV, 8, true>), grid, dim3(256), attention_lds(8), st, a, B, nz);
 }
 
 template <bool F16KV>
@@ -1242,7 +1292,10 @@ void launch_attention(const AttnArgs &a0, int B, hipStream_t st) {
   }
   if (avmm) {
     // the probabilities of every row part, then the weighted sums on the matrix cores
-    hipLaunchKernelGGL(k_attn_softmax_rows, dim3(a.nchunk, a.nHead, B), dim3(64), 0, st, a);
+    const bool walk = a.nchunk > ATTN_ZMAX;
+    const dim3 gr(std::min(a.nchunk, ATTN_ZMAX), a.nHead, B);
+    if (walk) hipLaunchKernelGGL(k_attn_softmax_rows<true>, gr, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL(k_attn_softmax_rows<false>, gr, dim3(64), 0, st, a);
     const int nrows = group * B;
     // blocks of 64 dimensions where the CUs hold one each (a block's chain waves share its LDS): a 509-token prompt of the 8B
     // shapes 3446 -> 3408 us, 16 tokens of 256-dimension heads at 2K positions 21.1 -> 17.6 us; with 432 of them (9 rows at
