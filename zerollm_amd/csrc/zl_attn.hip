@@ -825,33 +825,39 @@ __global__ __launch_bounds__(64) void k_attn_softmax_rows(const AttnArgs a) {
 // the accumulator as four fused multiply-adds in k order (measured on gfx950, every element of random wide-range
 // operands), so a chain of them over positions t, t + 1, ... in order is the reference's f32 chain out += p_t v_t
 // (one rounding per position, src/model/forward.js:131-134) for 16 rows x 16 dimensions at once: the bits of k_attn_av.
-// Block: one chunk of 16 rows r = b G + g (token b, query head kvh G + g) and 32 NDG dimensions of a KV head. Chain wave w
-// < NDG runs dimensions 32 w .. + 31 as two chains that share the A operand (lane l supplies A = p[row l mod 16][position
-// 4 m + l / 16], B = V[dimension l mod 16 (+ 16)][4 m + l / 16] and holds (row 4 (l / 16) + v, dimension l mod 16));
-// 2 NDG producer waves stage piece c + 1 meanwhile: V as f32 (zero past the pass's last position) and the probabilities
-// (already normalised by k_attn_softmax_rows, zero past a row's last position), with up to four pieces more on their way
-// in registers (a piece takes ~0.5 us, a load from memory 2-3); one barrier per piece. Operands lie in LDS by position mod 4 (section k holds positions 4 m + k), so a 16-byte
-// read gives four MFMAs' operands and the chain waves issue nothing but MFMAs and reads.
-// Bound by the MFMAs (32 cycles each) with the producers' instructions close behind (a wave alone on a SIMD issues one
-// every ~7 cycles, two one every ~5, so two producer waves share the staging of a SIMD's chain wave); a chain wave reads
-// 384 bytes of LDS per MFMA, 512 with one chain per wave. Pieces of 64 positions, so two blocks fit a CU.
+// Block: one chunk of 16 rows r = b G + g (token b, query head kvh G + g) and 32 NDG dimensions of a KV head. A chain wave runs
+// 16 CPW dimensions: one chain, or two that share the A operand (lane l supplies A = p[row l mod 16][position 4 m + l / 16],
+// B = V[dimension l mod 16 (+ 16)][4 m + l / 16] and holds (row 4 (l / 16) + v, dimension l mod 16)); the producer waves stage
+// piece c + 1 meanwhile: V as f32 (zero past the pass's last position) and the probabilities (already normalised by
+// k_attn_softmax_rows, zero past a row's last position), with up to four pieces more on their way in registers (a piece takes
+// ~0.5 us, a load from memory 2-3); one barrier per piece. Operands lie in LDS by position mod 4 (section k holds positions
+// 4 m + k), so a 16-byte read gives four MFMAs' operands and the chain waves issue nothing but MFMAs and reads.
+// Bound by the MFMAs (32 cycles each) and, per piece, the barrier and the first reads behind it, with the producers'
+// instructions close behind (a wave alone on a SIMD issues one every ~7 cycles, two one every ~5). A wave of two chains reads
+// 384 bytes of LDS per MFMA, of one chain 512, but two chains on one SIMD take twice the time of one: they are for launches
+// that fill the chip anyway. Pieces of 64 positions for 128 dimensions (two blocks fit a CU), of 128 for 32 dimensions (16
+// tokens of 128-dimension heads at 2K positions 16.5 -> 15.3 us against pieces of 64).
 template <bool B> struct Whole { static constexpr bool value = B; };  // a piece below every row's last position
 constexpr int MMV_RB = 16;                  // rows per block
-constexpr int MMV_CT = 64;                  // positions per staged piece
-constexpr int MMV_SF = MMV_CT / 4;          // floats of one position section
-constexpr int MMV_RS = 4 * MMV_SF + 4;      // floats of one dimension or row (4 x an odd number: conflict-free chain reads)
-template <bool F16KV, int NDG, bool WALK>
+constexpr int mmv_ct(int cpw) { return cpw == 2 ? 64 : 128; }  // positions per staged piece
+constexpr int mmv_rs(int cpw) { return mmv_ct(cpw) + 4; }  // floats of one dimension or row (4 x an odd number: conflict-free chain reads)
+// NDG x CPW: 4 x 2 (128 dimensions, two chains per wave) or 1 x 1 (32, one chain per wave)
+constexpr int mmv_producers(int cpw) { return cpw == 2 ? 8 : 4; }
+constexpr int mmv_waves(int ndg, int cpw) { return 2 * ndg / cpw + mmv_producers(cpw); }
+template <bool F16KV, int NDG, int CPW, bool WALK>
 __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int chunk, int L, uint8_t *lds) {
   typedef float f4 __attribute__((ext_vector_type(4)));
   constexpr int VB = F16KV ? 2 : 4, DB = 32 * NDG, RB = MMV_RB;
-  constexpr int CT = MMV_CT, SF = MMV_SF, RS = MMV_RS, NPT = NDG * 128;
+  constexpr int CT = mmv_ct(CPW), SF = CT / 4, RS = mmv_rs(CPW), NPT = mmv_producers(CPW) * 64;
   constexpr int EPP = 16 / VB;                      // positions per 16-byte V load
-  constexpr int UL = 16 / EPP;                      // V loads per unit of 16 positions (2 f16, 4 f32)
-  constexpr int UPR = CT / 16;                      // units per dimension of a piece
+  constexpr int UP = DB * CT / NPT >= 16 ? 16 : 8;  // positions of a unit, 16 or as many as there are for a thread
+  constexpr int UL = UP / EPP;                      // V loads per unit
+  constexpr int UPR = CT / UP;                      // units per dimension of a piece
   constexpr int D = F16KV ? 4 : 2;                  // pieces in flight (as many as the registers hold)
   constexpr int VU = DB * UPR / NPT;                // V units per producer thread per piece
-  constexpr int PN = RB * CT / NPT;                 // probabilities per producer thread per piece (2 or 4)
-  static_assert(VU * NPT == DB * UPR && (PN == 2 || PN == 4), "producer units");
+  constexpr int PN = RB * CT / NPT;                 // probabilities per producer thread per piece
+  constexpr int NCW = 2 * NDG / CPW;                // chain waves
+  static_assert(VU * NPT == DB * UPR && (PN == 2 || PN == 4 || PN == 8 || PN == 16) && (CPW == 1 || CPW == 2), "producer units");
   float *vk = (float *)lds;                         // [2][DB][RS]: V of position 4 m + k, dimension j at j RS + k SF + m
   float *pk = vk + 2 * DB * RS;                     // [2][RB][RS]: p of row i, position 4 m + k at i RS + k SF + m
   __shared__ long roff[RB];
@@ -889,12 +895,12 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
   const int nch = (nrmax + CT - 1) / CT;
   const int nend = (nrmax + AV_UNIT - 1) / AV_UNIT * AV_UNIT;  // positions the chains run
   const uint8_t *vbase = (const uint8_t *)a.vcache + ((((long)a.layer * a.nHeadKv + kvh) * a.hd + d0) * a.vstride + t00) * VB;
-  const bool producer = wave >= NDG;
+  const bool producer = wave >= NCW;
   f4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
   // the producers and the chain waves run loops of their own with one barrier per piece each (the same count), so the
   // chains' accumulators stay in their registers from piece to piece
   if (producer) {
-    const int pt = tid - NDG * 64;                  // producer thread 0 .. NPT - 1
+    const int pt = tid - NCW * 64;                  // producer thread 0 .. NPT - 1
     const int pr = pt * PN / CT, pq = pt * PN % CT; // its row and first position of its PN probabilities in a piece
     const int np = rnp[pr];
     // both by buffer loads and no branch around a load, so that the waits count exactly the piece they are for. Up to D
@@ -919,7 +925,7 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
       #pragma unroll
       for (int k = 0; k < VU; k++) {
         const int u = k * NPT + pt, dim = u / UPR;
-        const uint32_t vo = dim * vrow + (t0 + (u % UPR) * 16) * VB;
+        const uint32_t vo = dim * vrow + (t0 + (u % UPR) * UP) * VB;
         #pragma unroll
         for (int l = 0; l < UL; l++) s.v[k][l] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(vr, vo + l * 16, 0, 0));
       }
@@ -931,22 +937,25 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
       float *vs = vk + (c & 1) * DB * RS;
       #pragma unroll
       for (int k = 0; k < VU; k++) {
-        const int u = k * NPT + pt, dim = u / UPR, uu = u % UPR, t0 = c * CT + uu * 16;
-        float f[16];
+        const int u = k * NPT + pt, dim = u / UPR, uu = u % UPR, t0 = c * CT + uu * UP;
+        float f[UP];
         #pragma unroll
-        for (int e = 0; e < 16; e++) {
+        for (int e = 0; e < UP; e++) {
           const int w = e % EPP;
           const uint32_t wd = s.v[k][e / EPP][F16KV ? w >> 1 : w];
           const float x = F16KV ? h2f((uint16_t)((w & 1) ? (wd >> 16) : (wd & 0xffff))) : __uint_as_float(wd);
           f[e] = W || t0 + e < nmax ? x : 0.f;
         }
-        float *drow = vs + dim * RS + uu * 4;
+        float *drow = vs + dim * RS + uu * (UP / 4);
         #pragma unroll
-        for (int q = 0; q < 4; q++) *(f4 *)(drow + q * SF) = (f4){f[q], f[q + 4], f[q + 8], f[q + 12]};
+        for (int q = 0; q < 4; q++) {
+          if constexpr (UP == 16) *(f4 *)(drow + q * SF) = (f4){f[q], f[q + 4], f[q + 8], f[q + 12]};
+          else *(float2 *)(drow + q * SF) = make_float2(f[q], f[q + 4]);
+        }
       }
       float *prow = pk + (c & 1) * RB * RS + pr * RS + (pq >> 2);
       #pragma unroll
-      for (int j = 0; j < PN; j++) prow[((pq + j) & 3) * SF] = W || c * CT + pq + j < np ? s.p[j] : 0.f;
+      for (int j = 0; j < PN; j++) prow[((pq + j) & 3) * SF + (PN > 4 ? j >> 2 : 0)] = W || c * CT + pq + j < np ? s.p[j] : 0.f;
     };
     auto stage = [&](int c, const Pre &s) {
       if ((c + 1) * CT <= nrmin) stage_f(Whole<true>{}, c, s);
@@ -971,8 +980,9 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
     }
   } else {
     __syncthreads();
+    constexpr int Y = CPW == 2 ? 16 * RS : 0;       // the second chain's dimensions (none: the same reads)
     auto ld = [&](const float *q) { return *(const f4 *)q; };
-    const float *vr0 = vk + (wave * 32 + n16) * RS + g * SF, *pr0 = pk + n16 * RS + g * SF;
+    const float *vr0 = vk + (wave * 16 * CPW + n16) * RS + g * SF, *pr0 = pk + n16 * RS + g * SF;
     for (int c = 0; c < nch; c++) {
       // 16 positions per step (4 MFMAs per chain; lane group g: positions 4 m + g, m = 4 u .. 4 u + 3), the next step's
       // reads ahead of the current one's MFMAs; two steps per unit of 32 positions
@@ -981,22 +991,24 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
         #pragma unroll
         for (int i = 0; i < 4; i++) {
           acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i], v0[i], acc0, 0, 0, 0);
-          acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i], v1[i], acc1, 0, 0, 0);
+          if constexpr (CPW == 2) acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i], v1[i], acc1, 0, 0, 0);
         }
       };
-      const int nu = min(CT, nend - c * CT) / 16;  // 2 or 4 steps
-      f4 p0 = ld(pr), x0 = ld(vr), y0 = ld(vr + 16 * RS);
-      f4 p1 = ld(pr + 4), x1 = ld(vr + 4), y1 = ld(vr + 16 * RS + 4);
+      const int nu = min(CT, nend - c * CT) / 16;  // an even number of steps
+      f4 p0 = ld(pr), x0 = ld(vr), y0 = ld(vr + Y);
+      f4 p1 = ld(pr + 4), x1 = ld(vr + 4), y1 = ld(vr + Y + 4);
       __builtin_amdgcn_sched_barrier(0);
       step(p0, x0, y0);
-      if (nu > 2) {
-        p0 = ld(pr + 8); x0 = ld(vr + 8); y0 = ld(vr + 16 * RS + 8);
-        __builtin_amdgcn_sched_barrier(0);
-        step(p1, x1, y1);
-        p1 = ld(pr + 12); x1 = ld(vr + 12); y1 = ld(vr + 16 * RS + 12);
-        __builtin_amdgcn_sched_barrier(0);
-        step(p0, x0, y0);
-      }
+      #pragma unroll
+      for (int u = 2; u < CT / 16; u += 2)
+        if (nu > u) {
+          p0 = ld(pr + 4 * u); x0 = ld(vr + 4 * u); y0 = ld(vr + Y + 4 * u);
+          __builtin_amdgcn_sched_barrier(0);
+          step(p1, x1, y1);
+          p1 = ld(pr + 4 * u + 4); x1 = ld(vr + 4 * u + 4); y1 = ld(vr + Y + 4 * u + 4);
+          __builtin_amdgcn_sched_barrier(0);
+          step(p0, x0, y0);
+        }
       step(p1, x1, y1);
       __syncthreads();
     }
@@ -1008,12 +1020,12 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
   if (!producer) {
     #pragma unroll
     for (int v = 0; v < 4; v++) {
-      ot[(4 * g + v) * OP + 32 * wave + n16] = acc0[v];
-      ot[(4 * g + v) * OP + 32 * wave + 16 + n16] = acc1[v];
+      ot[(4 * g + v) * OP + 16 * CPW * wave + n16] = acc0[v];
+      if constexpr (CPW == 2) ot[(4 * g + v) * OP + 32 * wave + 16 + n16] = acc1[v];
     }
   }
   __syncthreads();
-  constexpr int NH = 6 * NDG;                       // half-waves
+  constexpr int NH = 2 * mmv_waves(NDG, CPW);       // half-waves
   const int hw = tid >> 5, l32 = tid & 31;
   for (int e = hw; e < RB * NDG; e += NH) {
     const int i = e / NDG, sl = e % NDG;
@@ -1049,20 +1061,20 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
 // XCD-aware block order: workgroup i of a chunk's blocks (a multiple of 8) goes to XCD i mod 8, and logical block
 // L = (i mod 8) (blocks / 8) + i / 8 gives each XCD a contiguous run of L, ordered dimension block fastest, then row block,
 // then KV head, so the blocks that read the same V share one L2
-template <bool F16KV, int NDG, bool WALK>
-__global__ __launch_bounds__(NDG * 192, NDG * 6 / 4) void k_attn_av_mm(const AttnArgs a, int nrows) {
+template <bool F16KV, int NDG, int CPW, bool WALK>
+__global__ __launch_bounds__(mmv_waves(NDG, CPW) * 64, CPW == 1 ? 4 : NDG * 6 / 4) void k_attn_av_mm(const AttnArgs a, int nrows) {
   extern __shared__ __align__(16) uint8_t lds[];
   const int L = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (L >= a.hd / (32 * NDG) * ((nrows + MMV_RB - 1) / MMV_RB) * a.nHeadKv) return;
   const int nmax = a.step->pos0 + a.step->B;
   for (int chunk = blockIdx.y; chunk * ATTN_CHUNK < nmax; chunk += gridDim.y) {
-    av_mm_chunk<F16KV, NDG, WALK>(a, nrows, chunk, L, lds);
+    av_mm_chunk<F16KV, NDG, CPW, WALK>(a, nrows, chunk, L, lds);
     if (!WALK) return;
     __syncthreads();  // the chunk's LDS has been read
   }
 }
 
-static size_t attention_av_mm_lds(int ndg) { return (size_t)2 * (32 * ndg + MMV_RB) * MMV_RS * 4; }
+static size_t attention_av_mm_lds(int ndg, int cpw) { return (size_t)2 * (32 * ndg + MMV_RB) * mmv_rs(cpw) * 4; }
 
 // ---- position-split weighted sum (long contexts). The exact chain above runs one dependent f32 step per position, so
 // at 16K positions it is ~40 us per output element. Here one block per (256-position chunk, query head, token) takes
@@ -1176,22 +1188,36 @@ AttnForm attention_form(int ctx) {
   return f;
 }
 
-template <bool F16KV, int NDG, bool WALK>
+template <bool F16KV, int NDG, int CPW, bool WALK>
 static void launch_av_mm_w(const AttnArgs &a, int nrows, hipStream_t st) {
   static bool attr = false;  // dynamic LDS above 64 KB must be requested per kernel
-  const size_t lds = attention_av_mm_lds(NDG);
+  const size_t lds = attention_av_mm_lds(NDG, CPW);
   if (!attr) {
-    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_mm<F16KV, NDG, WALK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_mm<F16KV, NDG, CPW, WALK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr = true;
   }
   const int nb = a.hd / (32 * NDG) * a.nHeadKv * ((nrows + MMV_RB - 1) / MMV_RB);  // (dimensions, KV head, rows) blocks
   const dim3 grid((nb + 7) / 8 * 8, std::min(a.nchunk, ATTN_ZMAX));
-  hipLaunchKernelGGL((k_attn_av_mm<F16KV, NDG, WALK>), grid, dim3(NDG * 192), lds, st, a, nrows);
+  hipLaunchKernelGGL((k_attn_av_mm<F16KV, NDG, CPW, WALK>), grid, dim3(mmv_waves(NDG, CPW) * 64), lds, st, a, nrows);
 }
-template <bool F16KV, int NDG>
+template <bool F16KV, int NDG, int CPW>
 static void launch_av_mm_k(const AttnArgs &a, int nrows, hipStream_t st) {
-  if (a.nchunk > ATTN_ZMAX) launch_av_mm_w<F16KV, NDG, true>(a, nrows, st);
-  else launch_av_mm_w<F16KV, NDG, false>(a, nrows, st);
+  if (a.nchunk > ATTN_ZMAX) launch_av_mm_w<F16KV, NDG, CPW, true>(a, nrows, st);
+  else launch_av_mm_w<F16KV, NDG, CPW, false>(a, nrows, st);
+}
+// One chain per wave and 32 dimensions per block, where each chain wave then has a SIMD's matrix pipe to itself or nearly so
+// (a CU holds three blocks), two chains per wave and 128 dimensions, which read V and p less often per MFMA, where the launch
+// fills the chip several times over. Only the cache's capacity is known here, so the line is drawn for rows of a quarter to all
+// of it. Whole passes in 32- against 128-dimension blocks: verify 8B, 9 tokens (96 blocks a chunk, 16 chunks) after 3000
+// positions 327 and 346 us, after 15000 420 and 419, after 28000 531 and 529; prompt 8B in 16 tokens (128 blocks) after 7000
+// 1478 and 1519, after 28000 2243 and 2146; in 64 tokens (512) after 700 537 and 545, after 7000 841 and 815. 64-dimension
+// blocks of two chains per wave were slower than the one-chain form in every one of 54 passes.
+constexpr long MMV_ONE_CHAIN_BLOCKS = 1536;
+template <bool F16KV>
+static void launch_av_mm(const AttnArgs &a, int nrows, hipStream_t st) {
+  const long blocks = (long)a.hd / 32 * a.nHeadKv * ((nrows + MMV_RB - 1) / MMV_RB) * std::min(a.nchunk, ATTN_ZMAX);
+  if (a.hd == 64 || blocks <= MMV_ONE_CHAIN_BLOCKS) launch_av_mm_k<F16KV, 1, 1>(a, nrows, st);
+  else launch_av_mm_k<F16KV, 4, 2>(a, nrows, st);
 }
 
 template <int HD, bool F16KV>
@@ -1300,17 +1326,8 @@ void launch_attention(const AttnArgs &a0, int B, hipStream_t st) {
     if (walk) hipLaunchKernelGGL(k_attn_softmax_rows<true>, gr, dim3(64), 0, st, a);
     else hipLaunchKernelGGL(k_attn_softmax_rows<false>, gr, dim3(64), 0, st, a);
     const int nrows = group * B;
-    // blocks of 64 dimensions where the CUs hold one each (a block's chain waves share its LDS): a 509-token prompt of the 8B
-    // shapes 3446 -> 3408 us, 16 tokens of 256-dimension heads at 2K positions 21.1 -> 17.6 us; with 432 of them (9 rows at
-    // 16K positions) two layers took 480 us, in 216 of 128 dimensions 454
-    const bool narrow = a.hd == 64 || (long)a.hd / 128 * a.nHeadKv * ((nrows + MMV_RB - 1) / MMV_RB) * a.nchunk <= 128;
-    if (a.kvF16) {
-      if (narrow) launch_av_mm_k<true, 2>(a, nrows, st);
-      else launch_av_mm_k<true, 4>(a, nrows, st);
-    } else {
-      if (narrow) launch_av_mm_k<false, 2>(a, nrows, st);
-      else launch_av_mm_k<false, 4>(a, nrows, st);
-    }
+    if (a.kvF16) launch_av_mm<true>(a, nrows, st);
+    else launch_av_mm<false>(a, nrows, st);
     ZL_HIP(hipGetLastError());
     return;
   }
