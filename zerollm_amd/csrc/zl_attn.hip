@@ -835,35 +835,38 @@ __global__ __launch_bounds__(64) void k_attn_softmax_rows(const AttnArgs a) {
 // Bound by the MFMAs (32 cycles each) and, per piece, the barrier and the first reads behind it, with the producers'
 // instructions close behind (a wave alone on a SIMD issues one every ~7 cycles, two one every ~5). A wave of two chains reads
 // 384 bytes of LDS per MFMA, of one chain 512, but two chains on one SIMD take twice the time of one: they are for launches
-// that fill the chip anyway. Pieces of 64 positions for 128 dimensions (two blocks fit a CU), of 128 for 32 dimensions (16
-// tokens of 128-dimension heads at 2K positions 16.5 -> 15.3 us against pieces of 64).
+// that fill the chip anyway. Pieces of 64 positions, so two blocks of 128 dimensions fit a CU, or four of 32 (with pieces of 128
+// or four producer waves fewer: 9 tokens of 32 heads after 16384 positions, 864 blocks, 451 us a pass of two layers, 453 and 474).
 template <bool B> struct Whole { static constexpr bool value = B; };  // a piece below every row's last position
 constexpr int MMV_RB = 16;                  // rows per block
-constexpr int mmv_ct(int cpw) { return cpw == 2 ? 64 : 128; }  // positions per staged piece
-constexpr int mmv_rs(int cpw) { return mmv_ct(cpw) + 4; }  // floats of one dimension or row (4 x an odd number: conflict-free chain reads)
+constexpr int MMV_CT = 64;                  // positions per staged piece
+constexpr int MMV_SF = MMV_CT / 4;          // floats of one position section
+constexpr int MMV_RS = 4 * MMV_SF + 4;      // floats of one dimension or row (4 x an odd number: conflict-free chain reads)
 // NDG x CPW: 4 x 2 (128 dimensions, two chains per wave) or 1 x 1 (32, one chain per wave)
-constexpr int mmv_producers(int cpw) { return cpw == 2 ? 8 : 4; }
+constexpr int mmv_producers(int cpw) { return cpw == 2 ? 8 : 2; }
 constexpr int mmv_waves(int ndg, int cpw) { return 2 * ndg / cpw + mmv_producers(cpw); }
 template <bool F16KV, int NDG, int CPW, bool WALK>
 __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int chunk, int L, uint8_t *lds) {
   typedef float f4 __attribute__((ext_vector_type(4)));
   constexpr int VB = F16KV ? 2 : 4, DB = 32 * NDG, RB = MMV_RB;
-  constexpr int CT = mmv_ct(CPW), SF = CT / 4, RS = mmv_rs(CPW), NPT = mmv_producers(CPW) * 64;
+  constexpr int CT = MMV_CT, SF = MMV_SF, RS = MMV_RS, NPT = mmv_producers(CPW) * 64;
   constexpr int EPP = 16 / VB;                      // positions per 16-byte V load
-  constexpr int UP = DB * CT / NPT >= 16 ? 16 : 8;  // positions of a unit, 16 or as many as there are for a thread
-  constexpr int UL = UP / EPP;                      // V loads per unit
-  constexpr int UPR = CT / UP;                      // units per dimension of a piece
+  constexpr int UL = 16 / EPP;                      // V loads per unit of 16 positions (2 f16, 4 f32)
+  constexpr int UPR = CT / 16;                      // units per dimension of a piece
   constexpr int D = F16KV ? 4 : 2;                  // pieces in flight (as many as the registers hold)
   constexpr int VU = DB * UPR / NPT;                // V units per producer thread per piece
   constexpr int PN = RB * CT / NPT;                 // probabilities per producer thread per piece
   constexpr int NCW = 2 * NDG / CPW;                // chain waves
-  static_assert(VU * NPT == DB * UPR && (PN == 2 || PN == 4 || PN == 8 || PN == 16) && (CPW == 1 || CPW == 2), "producer units");
+  static_assert(VU * NPT == DB * UPR && (PN == 2 || PN == 8) && (CPW == 1 || CPW == 2), "producer units");
   float *vk = (float *)lds;                         // [2][DB][RS]: V of position 4 m + k, dimension j at j RS + k SF + m
   float *pk = vk + 2 * DB * RS;                     // [2][RB][RS]: p of row i, position 4 m + k at i RS + k SF + m
   __shared__ long roff[RB];
   __shared__ int rnp[RB], rfull[RB];                // the row's positions in the chunk, and in all
   __shared__ uint32_t arrived;
-  const int tid = thread_index<WALK>(), lane = tid & 63, wave = tid >> 6, n16 = lane & 15, g = lane >> 4;
+  const int tid = thread_index<WALK>(), lane = tid & 63, n16 = lane & 15, g = lane >> 4;
+  // wave w of a block runs on SIMD w mod 4: every other four-wave block takes its last two for the chains, so that two blocks
+  // on a CU use the matrix pipes of all four (1 % of a pass)
+  const int wave = CPW == 1 ? (tid >> 6) ^ (L & 1) * 2 : tid >> 6;
   const int ND = a.hd / DB, NZ = (nrows + RB - 1) / RB;
   const int kvh = L / (ND * NZ), rbk = (L / ND) % NZ, d0 = (L % ND) * DB;
   const int G = a.nHead / a.nHeadKv;
@@ -900,7 +903,7 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
   // the producers and the chain waves run loops of their own with one barrier per piece each (the same count), so the
   // chains' accumulators stay in their registers from piece to piece
   if (producer) {
-    const int pt = tid - NCW * 64;                  // producer thread 0 .. NPT - 1
+    const int pt = (wave - NCW) * 64 + lane;                  // producer thread 0 .. NPT - 1
     const int pr = pt * PN / CT, pq = pt * PN % CT; // its row and first position of its PN probabilities in a piece
     const int np = rnp[pr];
     // both by buffer loads and no branch around a load, so that the waits count exactly the piece they are for. Up to D
@@ -925,7 +928,7 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
       #pragma unroll
       for (int k = 0; k < VU; k++) {
         const int u = k * NPT + pt, dim = u / UPR;
-        const uint32_t vo = dim * vrow + (t0 + (u % UPR) * UP) * VB;
+        const uint32_t vo = dim * vrow + (t0 + (u % UPR) * 16) * VB;
         #pragma unroll
         for (int l = 0; l < UL; l++) s.v[k][l] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(vr, vo + l * 16, 0, 0));
       }
@@ -937,21 +940,18 @@ __device__ __forceinline__ void av_mm_chunk(const AttnArgs &a, int nrows, int ch
       float *vs = vk + (c & 1) * DB * RS;
       #pragma unroll
       for (int k = 0; k < VU; k++) {
-        const int u = k * NPT + pt, dim = u / UPR, uu = u % UPR, t0 = c * CT + uu * UP;
-        float f[UP];
+        const int u = k * NPT + pt, dim = u / UPR, uu = u % UPR, t0 = c * CT + uu * 16;
+        float f[16];
         #pragma unroll
-        for (int e = 0; e < UP; e++) {
+        for (int e = 0; e < 16; e++) {
           const int w = e % EPP;
           const uint32_t wd = s.v[k][e / EPP][F16KV ? w >> 1 : w];
           const float x = F16KV ? h2f((uint16_t)((w & 1) ? (wd >> 16) : (wd & 0xffff))) : __uint_as_float(wd);
           f[e] = W || t0 + e < nmax ? x : 0.f;
         }
-        float *drow = vs + dim * RS + uu * (UP / 4);
+        float *drow = vs + dim * RS + uu * 4;
         #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          if constexpr (UP == 16) *(f4 *)(drow + q * SF) = (f4){f[q], f[q + 4], f[q + 8], f[q + 12]};
-          else *(float2 *)(drow + q * SF) = make_float2(f[q], f[q + 4]);
-        }
+        for (int q = 0; q < 4; q++) *(f4 *)(drow + q * SF) = (f4){f[q], f[q + 4], f[q + 8], f[q + 12]};
       }
       float *prow = pk + (c & 1) * RB * RS + pr * RS + (pq >> 2);
       #pragma unroll
@@ -1074,7 +1074,7 @@ __global__ __launch_bounds__(mmv_waves(NDG, CPW) * 64, CPW == 1 ? 4 : NDG * 6 / 
   }
 }
 
-static size_t attention_av_mm_lds(int ndg, int cpw) { return (size_t)2 * (32 * ndg + MMV_RB) * mmv_rs(cpw) * 4; }
+static size_t attention_av_mm_lds(int ndg) { return (size_t)2 * (32 * ndg + MMV_RB) * MMV_RS * 4; }
 
 // ---- position-split weighted sum (long contexts). The exact chain above runs one dependent f32 step per position, so
 // at 16K positions it is ~40 us per output element. Here one block per (256-position chunk, query head, token) takes
@@ -1191,7 +1191,7 @@ AttnForm attention_form(int ctx) {
 template <bool F16KV, int NDG, int CPW, bool WALK>
 static void launch_av_mm_w(const AttnArgs &a, int nrows, hipStream_t st) {
   static bool attr = false;  // dynamic LDS above 64 KB must be requested per kernel
-  const size_t lds = attention_av_mm_lds(NDG, CPW);
+  const size_t lds = attention_av_mm_lds(NDG);
   if (!attr) {
     ZL_HIP(hipFuncSetAttribute((const void *)k_attn_av_mm<F16KV, NDG, CPW, WALK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr = true;
@@ -1206,12 +1206,12 @@ static void launch_av_mm_k(const AttnArgs &a, int nrows, hipStream_t st) {
   else launch_av_mm_w<F16KV, NDG, CPW, false>(a, nrows, st);
 }
 // One chain per wave and 32 dimensions per block, where each chain wave then has a SIMD's matrix pipe to itself or nearly so
-// (a CU holds three blocks), two chains per wave and 128 dimensions, which read V and p less often per MFMA, where the launch
-// fills the chip several times over. Only the cache's capacity is known here, so the line is drawn for rows of a quarter to all
-// of it. Whole passes in 32- against 128-dimension blocks: verify 8B, 9 tokens (96 blocks a chunk, 16 chunks) after 3000
-// positions 327 and 346 us, after 15000 420 and 419, after 28000 531 and 529; prompt 8B in 16 tokens (128 blocks) after 7000
-// 1478 and 1519, after 28000 2243 and 2146; in 64 tokens (512) after 700 537 and 545, after 7000 841 and 815. 64-dimension
-// blocks of two chains per wave were slower than the one-chain form in every one of 54 passes.
+// (a CU holds four blocks), two chains per wave and 128 dimensions, which read V and p less often per MFMA, where the launch
+// fills the chip several times over. Only the cache's capacity is known here, so the line is drawn between rows of a quarter
+// and of all of it. Whole passes in 32- against 128-dimension blocks: verify 8B, 9 tokens (96 blocks a chunk, 16 chunks) after
+// 3000 positions 305 and 346 us, after 15000 403 and 418, after 28000 521 and 526; 5 tokens (64) after 5000 of 8K 292 and 308,
+// after 28000 of 32K 456 and 444; prompt 8B in 16 tokens (128) after 7000 1478 and 1519, after 28000 2243 and 2146; in 64 tokens
+// (512) after 700 537 and 545, after 7000 841 and 815.
 constexpr long MMV_ONE_CHAIN_BLOCKS = 1536;
 template <bool F16KV>
 static void launch_av_mm(const AttnArgs &a, int nrows, hipStream_t st) {
