@@ -59,3 +59,23 @@ def test_result_over_the_rows(gpu, type_):
         st.synchronize()
         assert (x[:M].cpu().numpy().view(np.uint32) == m.gemv(X[:M]).view(np.uint32)).all()
     m.free()
+
+
+@pytest.mark.parametrize("type_,rows,cols", [(G.Q8_0, 2048, 2048), (G.Q8_0, 4096, 512), (G.Q8_0, 70, 96), (G.Q4_K, 2048, 2048),
+                                             (G.Q6_K, 2048, 512)])
+def test_single_token_result_over_the_row(gpu, type_, rows, cols):
+    """One token whose result overwrites its row, all of it or from its middle on."""
+    raw = synth.tensor_bytes(synth.TensorSpec("w", type_, rows, cols, seed=9), use_device=True)
+    m = Mat(type_, raw, rows, cols)
+    X = np.random.default_rng(9).standard_normal((1, cols)).astype(np.float32)
+    want = m.gemv(X)[0]
+    st = torch.cuda.Stream()
+    for shift in (0, cols // 2):
+        print(f"case type {type_} {rows} x {cols} one token, result from value {shift} on", flush=True)
+        buf = torch.zeros(shift + max(rows, cols), device="cuda")
+        buf[:cols] = torch.from_numpy(X[0]).cuda()
+        torch.cuda.synchronize()
+        call("zl_mat_gemv_noalloc", m.h, C.c_void_p(buf.data_ptr()), 1, C.c_void_p(buf.data_ptr() + 4 * shift), C.c_void_p(st.cuda_stream))
+        st.synchronize()
+        assert (buf[shift:shift + rows].cpu().numpy().view(np.uint32) == want.view(np.uint32)).all(), shift
+    m.free()

@@ -1692,8 +1692,9 @@ static unsigned char *noalloc_scratch() {
   return g_scratch[dev];
 }
 
-// zl_mat_gemv on device rows with the static work space: the same kernels (activation quantisation, then the GEMV
-// dispatch of launch_gemv) as zl_mat_gemv, so the results are the same bits.
+// zl_mat_gemv on device rows with the static work space, the same bits as zl_mat_gemv: the activation quantisation and the
+// GEMV dispatch of launch_gemv, or where the rows and the result lie apart a GEMV that reads the f32 rows itself (single
+// Q8_0 tokens, short rows, float weights).
 static void mat_gemv_noalloc(zl_mat *m, const float *x, int M, float *y, hipStream_t st) {
   const DevMat &mm = m->copies[0];
   ZL_REQUIRE(M >= 1 && M <= NOALLOC_MAX_M && mm.cols <= NOALLOC_MAX_K, ZL_ERR_ARG,
@@ -1718,15 +1719,18 @@ static void mat_gemv_noalloc(zl_mat *m, const float *x, int M, float *y, hipStre
   GemvArgs a = gemv_args(&seg, 1, M, EPI_STORE, act, gw);
   ZL_REQUIRE(a.ks == 1 || (a.ntiles <= GEMV_CNT_TILES && (size_t)gemv_part_need(a) <= NOALLOC_PART_DOUBLES),
              ZL_ERR_ARG, "zl_mat_gemv_noalloc: this matrix's split-K partial sums exceed the static work space");
-  if (use_rg() && M == 1 && mm.type == T_Q8_0 && mm.nslab <= 48) {  // the probe's single-token path (no quantisation pass)
-    a.xf = x; a.ldxf = mm.cols; a.xrow0 = 0; a.n = mm.cols; a.nw = nullptr; a.eps = 0.0;
+  // rows that the result overwrites are quantised (copied) before, as no workgroup may store while another one still reads
+  // them; others are read by the GEMV itself: float weights take them as they are, quantised ones quantise short rows, with
+  // no launch before
+  const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
+  const bool apart = x0 + (uintptr_t)M * mm.cols * 4 <= y0 || y0 + (uintptr_t)M * mm.rows * 4 <= x0;
+  if (use_rg() && M == 1 && mm.type == T_Q8_0 && mm.nslab <= 48) {  // the probe's single-token path
+    if (!apart) launch_norm_quant(x, mm.cols, 0, 1, nullptr, 0.0, mm.cols, ld, act, st);
+    a.xf = apart ? x : act.f; a.ldxf = mm.cols; a.xrow0 = 0; a.n = mm.cols; a.nw = nullptr; a.eps = 0.0;
     launch_gemv_rg(a, EPI_STORE, st);
     return;
   }
-  // rows that the result overwrites are quantised (copied) before; others are read by the GEMV itself: float weights take
-  // them as they are, quantised ones quantise short rows, with no launch before
-  const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
-  if (x0 + (uintptr_t)M * mm.cols * 4 <= y0 || y0 + (uintptr_t)M * mm.rows * 4 <= x0) {
+  if (apart) {
     if (!is_quant(mm.type)) {
       launch_gemv(a, EPI_STORE, x, mm.cols, st);
       return;
