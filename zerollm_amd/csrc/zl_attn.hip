@@ -8,6 +8,7 @@
 // Scores live in a [token][head][ctx] f32 buffer between the two. The weighted sum keeps the reference's f32 rounding
 // after every position: a random-weight network turns a 1e-7 change there into a visible logit difference.
 #include "zl_kernels.h"
+#include "zl_exp.h"
 #include <algorithm>
 #include <climits>
 
@@ -419,35 +420,6 @@ __global__ __launch_bounds__(NWV * 64) void k_attn_scores_mm(const AttnArgs a, i
 
 size_t attention_mm_lds(int hd) { return (size_t)MM_PT * (hd + 2) * 8; }
 
-
-constexpr double LN2_HI = 2977044472.0 / 4294967296.0;     // ln 2 to 32 fractional bits (n LN2_HI is exact)
-constexpr double LN2_LO = -4.2009150726810846e-11;          // ln 2 - LN2_HI
-
-// exp of x <= 0 in f64 (NaN and -inf included): x = n ln 2 + r with |r| <= ln 2 / 2 (ln 2 in two parts, n exact), the
-// Taylor polynomial of degree 13 in Horner form (remainder r^14 / 14! < 5e-18), scaled by 2^n. Within an ulp of the
-// exact value. 21 VALU instructions where the device library's exp, which serves every argument, takes about 45: the
-// softmax of a 12K-position prefill row is bound by them.
-__device__ __forceinline__ double exp_neg(double x) {
-  const double y = x < -1000.0 ? -1000.0 : x;  // (2^n underflows to 0 long before; a NaN stays one)
-  const double n = rint(y * 1.4426950408889634);
-  double r = fma(n, -LN2_HI, y);
-  r = fma(n, -LN2_LO, r);
-  double p = 1.0 / 6227020800.0;
-  p = fma(p, r, 1.0 / 479001600.0);
-  p = fma(p, r, 1.0 / 39916800.0);
-  p = fma(p, r, 1.0 / 3628800.0);
-  p = fma(p, r, 1.0 / 362880.0);
-  p = fma(p, r, 1.0 / 40320.0);
-  p = fma(p, r, 1.0 / 5040.0);
-  p = fma(p, r, 1.0 / 720.0);
-  p = fma(p, r, 1.0 / 120.0);
-  p = fma(p, r, 1.0 / 24.0);
-  p = fma(p, r, 1.0 / 6.0);
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
-  return ldexp(p, (int)n);
-}
 
 // ---- chunks of a row. A row of positions 0 .. pos is cut into chunks of ATTN_CHUNK positions. Each chunk is a softmax
 // and a weighted sum of its own, with the reference's arithmetic (src/compute/ref-kernels.js:313-320,
