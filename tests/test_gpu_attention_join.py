@@ -47,6 +47,35 @@ def special(case, t, ids):
         ids[1000] = b
 
 
+@pytest.mark.parametrize("head_dim,kv", [(64, "f16"), (128, "f16"), (256, "f16"), (128, "f32")])
+def test_chunks_of_uneven_weight_join_to_the_softmax_of_the_row(gpu, monkeypatch, tmp_path, head_dim, kv):
+    """Three chunks whose scores differ by a few units, the last one of about 1000 positions, each with a share of the sum
+    that counts: the outputs against float64, and an answer with one chunk lost or given a neighbour's weight is far off."""
+    t = Tables(head_dim, 12)
+    third = IDS // 3
+    t.q[:, :, -1] = 1.0
+    for c, score in enumerate((0.0, 1.5, -0.75)):  # of the ids of chunk c
+        t.k[c * third:(c + 1) * third, -1] = np.float16(score * np.sqrt(head_dim))
+    rng = np.random.default_rng(13)
+    ids = np.concatenate([rng.integers(c * third, (c + 1) * third, n) for c, n in enumerate((2048, 2048, 1016))])
+    first = len(ids) - 16
+    want = t.exact(ids, range(first, len(ids)))
+    # float32 scores of at most 8 in all (2^-22 absolute), probabilities rounded twice, and the chain's one rounding of the
+    # running sum a position, which add up like sqrt(2048) 2^-24 of sum p |v| (0.8 of a value's standard deviation)
+    bound = 2.0 ** -22 + 2.0 ** -23 + 4 * np.sqrt(2048) * 2.0 ** -24
+    for lost in range(3):
+        keep = np.r_[:lost * 2048, min((lost + 1) * 2048, len(ids)):len(ids)]
+        if lost < 2:
+            assert np.abs(t.exact(ids[keep], range(len(keep) - 16, len(keep))) - want).max() > 100 * bound
+    m = t.load(monkeypatch, str(tmp_path / "t.gguf"), ctx=len(ids) + 8, kv=kv)
+    for n in (1, 5, 16):
+        print(f"case uneven chunks head {head_dim} kv {kv} passes of {n}", flush=True)
+        err = np.abs(t.outputs(rows_of(m, ids.tolist(), first, n), ids[first:]) - want).max()
+        print(f"largest error {err:.2e}, bound {bound:.2e}", flush=True)
+        assert err <= bound, n
+    m.close()
+
+
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("case,length", [("a chunk of NaN", 2049), ("a chunk of NaN", 2064), ("first chunk -inf", 2700),
                                          ("middle chunk -inf", 4200), ("every chunk -inf", 2060), ("inf at weight 0", 2700)])

@@ -345,25 +345,19 @@ def test_long_context_attention_matches_oracle(gpu, tiny_files):
 
 
 @pytest.mark.parametrize("kv", ["f16", "f32"])
-def test_per_head_weighted_sum_equals_slice_form_and_oracle(gpu, tiny_files, monkeypatch, kv):
-    """The long-context weighted sums forced at a 1300-position context, each against the slice form (k_attn_av) and
-    the oracle:
-    - "grouped": ZEROLLM_ATTN_HEAD_CTX=1024 sends passes of several tokens to k_attn_softmax_rows + k_attn_av_group
-      (single-token passes keep k_attn_av);
-    - "head": ZEROLLM_ATTN_HEAD1_CTX=1024 in addition sends single-token passes to the per-head kernel k_attn_av_head
-      (what single-token passes take beyond ~29,900 positions).
-    In every form the batched rows equal the single-token passes bit for bit, and the rows equal the slice form's."""
+def test_weighted_sum_forms_equal_each_other_and_oracle(gpu, tiny_files, monkeypatch, kv):
+    """Both weighted sums forced for every pass at a 1300-position context (ZEROLLM_ATTN_MMAV_B): the lane chains
+    (k_attn_av, also for the 16-token prompt chunks) and the matrix cores (k_attn_softmax_rows + k_attn_av_mm, also for single
+    tokens). In each form the batched rows equal the single-token passes bit for bit, and the rows equal the other form's
+    and match the oracle."""
     toks = prompt(1210, seed=19)
     ref = O.OracleModel(tiny_files[0], ctx=1300, kv=kv)
     for t in toks[:-6]:
         ref.forward(t, logits=False)
     want = np.stack([ref.forward(t) for t in toks[-6:]])
     rows = {}
-    for form in ("slice", "grouped", "head"):
-        if form == "grouped":
-            monkeypatch.setenv("ZEROLLM_ATTN_HEAD_CTX", "1024")
-        if form == "head":
-            monkeypatch.setenv("ZEROLLM_ATTN_HEAD1_CTX", "1024")
+    for form, least in (("lanes", "1000"), ("matrix cores", "1")):
+        monkeypatch.setenv("ZEROLLM_ATTN_MMAV_B", least)
         print(f"case weighted sum {form} kv {kv}", flush=True)
         m = Mdl.HipModel.load(tiny_files[0], ctx=1300, kv=kv)
         for i in range(0, 1200, 16):
@@ -375,28 +369,29 @@ def test_per_head_weighted_sum_equals_slice_form_and_oracle(gpu, tiny_files, mon
         m.close()
         assert (single.view(np.uint32) == batched.view(np.uint32)).all(), form
         rows[form] = single
-    for form in ("grouped", "head"):
-        assert (rows[form].view(np.uint32) == rows["slice"].view(np.uint32)).all(), form
-    exact = np.mean(rows["head"].view(np.uint32) == want.view(np.uint32))
-    assert exact >= 0.999 and np.abs(rows["head"] - want).max() <= 1e-6 * np.abs(want).max(), exact
+    assert (rows["lanes"].view(np.uint32) == rows["matrix cores"].view(np.uint32)).all()
+    exact = np.mean(rows["lanes"].view(np.uint32) == want.view(np.uint32))
+    assert exact >= 0.999 and np.abs(rows["lanes"] - want).max() <= 1e-6 * np.abs(want).max(), exact
 
 
 @pytest.mark.parametrize("kv", ["f16", "f32"])
-def test_matrix_core_slice_form_equals_lane_chains_and_oracle(gpu, tiny_files, monkeypatch, kv):
-    """The slice form's weighted sums with the chains on the matrix cores (k_attn_av_mfma: the default from 4096
-    positions, forced here by ZEROLLM_ATTN_AVMF=1) and on the lanes (k_attn_av, ZEROLLM_ATTN_AVMF=0) give the same rows
-    bit for bit, for single-token passes and a 6-token pass at a 1300-position context (three staged chunks), and match
-    the oracle."""
+def test_caches_of_every_size_give_the_same_rows(gpu, tiny_files, kv):
+    """The cache's capacity chooses the kernels (one chunk, several, more than have blocks of their own; matrix cores from 2
+    tokens on in large ones): single-token and 6-token passes after 1204 positions give the same bits in all, those of the
+    oracle."""
+    from zerollm_amd import synth
+
     toks = prompt(1210, seed=29)
     ref = O.OracleModel(tiny_files[0], ctx=1300, kv=kv)
     for t in toks[:-6]:
         ref.forward(t, logits=False)
     want = np.stack([ref.forward(t) for t in toks[-6:]])
-    rows = {}
-    for form in ("mfma", "lanes"):
-        monkeypatch.setenv("ZEROLLM_ATTN_AVMF", "1" if form == "mfma" else "0")
-        print(f"case slice form {form} kv {kv}", flush=True)
-        m = Mdl.HipModel.load(tiny_files[0], ctx=1300, kv=kv)
+    spec, _ = synth.tiny_pair()
+    spec.ctx_train = 65536  # the tiny target with a trained context that admits the larger caches
+    first = None
+    for ctx in (1300, 4096, 9000, 40000):
+        print(f"case cache of {ctx} kv {kv}", flush=True)
+        m = synth.build_on_device(spec, ctx=ctx, kv=kv)
         for i in range(0, 1200, 16):
             m.forward_batch(toks[i:i + 16], logits="none")
         m.forward_batch(toks[1200:1204], logits="none")
@@ -404,11 +399,10 @@ def test_matrix_core_slice_form_equals_lane_chains_and_oracle(gpu, tiny_files, m
         m.truncate(1204)
         batched = m.forward_batch(toks[-6:], logits="all").copy()
         m.close()
-        assert (single.view(np.uint32) == batched.view(np.uint32)).all(), form
-        rows[form] = single
-    assert (rows["mfma"].view(np.uint32) == rows["lanes"].view(np.uint32)).all()
-    exact = np.mean(rows["mfma"].view(np.uint32) == want.view(np.uint32))
-    assert exact >= 0.999 and np.abs(rows["mfma"] - want).max() <= 1e-6 * np.abs(want).max(), exact
+        first = single if first is None else first
+        assert (single.view(np.uint32) == first.view(np.uint32)).all() and (batched.view(np.uint32) == first.view(np.uint32)).all(), ctx
+    exact = np.mean(first.view(np.uint32) == want.view(np.uint32))
+    assert exact >= 0.999 and np.abs(first - want).max() <= 1e-6 * np.abs(want).max(), exact
 
 
 def test_16k_context_verify_width_9_equals_sequential_and_rolls_back(gpu, tiny_files):
@@ -477,10 +471,10 @@ def test_split_weighted_sum_matches_oracle_at_1200_positions(gpu, tiny_files, mo
     _check_simd_tolerance(got, want, "split vs oracle")
 
 
-def test_split_weighted_sum_matches_exact_chain_at_16k(gpu, monkeypatch):
-    """At 16384 positions (the long-context configuration's length) the split weighted sum against the exact f32
-    chain (bit-exact with the oracle at shorter contexts) on the same model and tokens: the deviation the split path
-    has at that length."""
+def test_split_weighted_sum_matches_joined_chunks_at_16k(gpu, monkeypatch):
+    """At 16384 positions (the long-context configuration's length) the position-split weighted sum (float64 sums of 256
+    positions) against the default one (float32 chains of 2048 positions, joined in float64) on the same model and tokens:
+    how far two correct orders of the sum move this model's logits at that length."""
     from zerollm_amd import synth
 
     ctx = 16384 + 32
@@ -488,7 +482,7 @@ def test_split_weighted_sum_matches_exact_chain_at_16k(gpu, monkeypatch):
     spec, _ = synth.tiny_pair()
     spec.ctx_train = 32768
     rows = {}
-    for mode, thr in (("exact", "100000"), ("split", "1024")):
+    for mode, thr in (("chunks", "100000"), ("split", "1024")):
         monkeypatch.setenv("ZEROLLM_ATTN_EXACT_CTX", thr)
         print(f"case 16k {mode}", flush=True)
         m = synth.build_on_device(spec, ctx=ctx, kv="f16")
@@ -496,7 +490,5 @@ def test_split_weighted_sum_matches_exact_chain_at_16k(gpu, monkeypatch):
             m.forward_batch(toks[i:i + 16], logits="none")
         rows[mode] = m.forward_batch(toks[16384:], logits="all").copy()
         m.close()
-    # observed: max-abs 0.031, mean-abs 0.0054, min cosine 0.99985, below the reference's 0.9999: at 16K positions
-    # the path does not meet the reference's SIMD bounds on this random model, which is why contexts the exact chain
-    # can hold (up to ~29900 positions) use the exact chain
-    _check_simd_tolerance(rows["split"], rows["exact"], "16k split vs exact", min_cos=0.9995)
+    # (a 1e-6 change of an attention output flips int8 activation codes of this random model)
+    _check_simd_tolerance(rows["split"], rows["chunks"], "16k split vs joined chunks", min_cos=0.9995)

@@ -63,18 +63,17 @@ def test_logits_and_state_match_oracle(gpu, quant, kv):
     ref.close()
 
 
-@pytest.mark.parametrize("form", ["matrix-core", "per-head"])
+@pytest.mark.parametrize("form", ["matrix-core", "large-cache"])
 def test_gated_attention_forms_give_the_same_bits(gpu, monkeypatch, form):
     """The gated attention's weighted sum on the matrix cores for every pass, single tokens included
-    (ZEROLLM_ATTN_MMAV_B=1: the form 256-dimension heads take beyond ~29,900 positions, where the slice form's softmax
-    row leaves LDS), and the per-head and grouped forms of long contexts (ZEROLLM_ATTN_HEAD_CTX=0,
-    ZEROLLM_ATTN_HEAD1_CTX=0) give the default forms' logits bit for bit (the slice form of single-token passes, the
-    lane chains of several-token passes), over single-token and 5-token passes."""
+    (ZEROLLM_ATTN_MMAV_B=1), and the forms of a cache of 40,000 positions (blocks that walk its chunks; matrix cores from 2
+    tokens on) give the default forms' logits bit for bit (the lane chains), over single-token and 5-token passes."""
     spec = synth.tiny_qwen35(seed=21, quant="q8_0")
     toks = prompt(40, seed=6)
 
-    def run():
-        m = synth.build_on_device(spec, ctx=128, kv="f16")
+    def run(ctx=128):
+        m = synth.build_on_device(spec, ctx=ctx, kv="f16")
+        assert m.ctx == ctx
         a = np.stack([m.forward(t).copy() for t in toks[:30]])
         b = m.forward_batch(toks[30:35], logits="all").copy()
         c = np.stack([m.forward(t).copy() for t in toks[35:]])
@@ -85,10 +84,10 @@ def test_gated_attention_forms_give_the_same_bits(gpu, monkeypatch, form):
     want = run()
     if form == "matrix-core":
         monkeypatch.setenv("ZEROLLM_ATTN_MMAV_B", "1")
+        got = run()
     else:
-        monkeypatch.setenv("ZEROLLM_ATTN_HEAD_CTX", "0")
-        monkeypatch.setenv("ZEROLLM_ATTN_HEAD1_CTX", "0")
-    got = run()
+        spec.ctx_train = max(spec.ctx_train, 65536)
+        got = run(40000)
     assert (got.view(np.uint32) == want.view(np.uint32)).all()
 
 
