@@ -5,8 +5,9 @@
 //   k_attn_av      softmax over the scores (e = exp(s - max) in f64, stored f32; p = f32(e * (1/sum e))), then
 //                  out_i = sum_t p_t V_t,i accumulated in f32 in position order, one block per (32-dim slice, query
 //                  head, token, chunk of 2048 positions); the head output is also quantised for the output projection.
-// Scores live in a [token][head][ctx] f32 buffer between the two. The weighted sum keeps the reference's f32 rounding
-// after every position: a random-weight network turns a 1e-7 change there into a visible logit difference.
+// Scores live in a [token][head][ctx] f32 buffer between the two. The weighted sum of a chunk keeps the reference's f32
+// rounding after every position, so rows of up to 2048 positions are the reference's bits (a random-weight network turns a
+// 1e-7 change there into a visible logit difference); the chunks of longer rows are joined in f64.
 #include "zl_kernels.h"
 #include "zl_exp.h"
 #include <algorithm>
@@ -635,7 +636,7 @@ __device__ __forceinline__ void av_chunk(const AttnArgs &a, int chunk, int b, in
     if (c + 1 < nch) fetch(c + 1, npos);
     if (chainLane) {
       // units of UNIT positions, software pipelined: the LDS reads of unit u + 1 are issued before the fma steps of
-      // unit u, so the chain (one dependent fma per position, ~2.2 ns each) does not wait out an LDS latency per unit.
+      // unit u, so the chain (one dependent fma per position, ~4 ns each) does not wait out an LDS latency per unit.
       // p and V are zero past the last position, so a unit may run past `cnt`: fmaf(0, 0, o) == o. The read-ahead index
       // is clamped to the chunk's last unit (a re-read, never past it).
       const int t0 = c * CT, cnt = min(CT, npos - t0), nu = (cnt + AV_UNIT - 1) / AV_UNIT;
@@ -1048,13 +1049,13 @@ __global__ __launch_bounds__(mmv_waves(NDG, CPW) * 64, CPW == 1 ? 4 : NDG * 6 / 
 
 static size_t attention_av_mm_lds(int ndg) { return (size_t)2 * (32 * ndg + MMV_RB) * MMV_RS * 4; }
 
-// ---- position-split weighted sum (long contexts). The exact chain above runs one dependent f32 step per position, so
-// at 16K positions it is ~40 us per output element. Here one block per (256-position chunk, query head, token) takes
+// ---- position-split weighted sum (only where it is asked for). Here one block per (256-position chunk, query head, token) takes
 // the chunk's scores, its max m_c, e_t = exp(s_t - m_c) and l_c = sum e_t in f64, and o_c[i] = sum e_t V_t,i in f64
 // (V staged through LDS with coalesced loads); k_attn_merge then forms out_i = f32(sum_c w_c o_c[i] / sum_c w_c l_c),
 // w_c = exp(m_c - max_c m_c), adding the chunks in chunk order. Every order is a function of the position count only,
 // so batched and single-token passes agree bit for bit. The result is the softmax-weighted sum in f64, rounded once:
-// it differs from the reference's f32 chain (src/model/forward.js:134-139) by that chain's own rounding error.
+// it differs from the reference's f32 chain (src/model/forward.js:134-139) by that chain's own rounding error, and from the
+// joined chunks above by the rounding errors of their chains.
 template <bool F16KV>
 __global__ __launch_bounds__(256) void k_attn_av_split(const AttnArgs a) {
   extern __shared__ __align__(16) uint8_t lds[];
@@ -1153,8 +1154,7 @@ AttnForm attention_form(int ctx) {
   // (verify passes at long contexts); ZEROLLM_ATTN_MM_B overrides the token count (tests)
   const char *em = getenv("ZEROLLM_ATTN_MM_B");
   f.mmMinB = em ? atoi(em) : ctx >= LONG_CTX ? 2 : 16;
-  // their weighted sums on the matrix cores likewise: from 16 tokens on (32-row blocks), and from 2 where the context
-  // is long (16-row blocks)
+  // their weighted sums on the matrix cores likewise: from 16 tokens on, and from 2 where the context is long
   const char *ea = getenv("ZEROLLM_ATTN_MMAV_B");
   f.mmAvMinB = ea ? atoi(ea) : em ? f.mmMinB : ctx >= LONG_CTX ? 2 : 16;
   return f;
