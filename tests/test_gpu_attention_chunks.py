@@ -76,3 +76,24 @@ def test_passes_that_end_at_the_last_position_of_the_cache(gpu, ctx):
         rows = np.concatenate([m.forward_batch(ids[i:i + n], logits="all").copy() for i in range(ctx - 32, ctx, n)])
         assert (rows.view(np.uint32) == one.view(np.uint32)).all(), n
     m.close()
+
+
+@pytest.mark.parametrize("head_dim,kv,ctx", [(128, "f16", 36900), (128, "f32", 36900), (256, "f16", 36900), (128, "f16", 9000)])
+def test_passes_of_many_blocks_equal_single_tokens(gpu, head_dim, kv, ctx):
+    """64-token passes of 8 KV heads, whose weighted sums take 128-dimension blocks (in caches of more than 16 chunks blocks
+    that walk them), across chunk borders and at short rows: the bits of single-token passes."""
+    spec = synth.build_spec(n_layer=1, arch="qwen3", n_embd=256, n_head=16, n_head_kv=8, head_dim=head_dim, n_ff=512, vocab=2048,
+                            ctx_train=65536, types=synth.all_type(synth.gguf.Q8_0), seed=7)
+    ids = synth.seeded_ids(ctx, 24, spec.vocab)
+    m = synth.build_on_device(spec, ctx=ctx, kv=kv, max_batch=64, logits_batch=64)
+    at = 0
+    for a in [a for a in (600, 2020, 4064, 32740, 34790, 36830) if a + 64 <= ctx]:
+        print(f"case many blocks head {head_dim} kv {kv} cache {ctx} rows from {a}", flush=True)
+        for i in range(at, a, 64):
+            m.forward_batch(ids[i:min(i + 64, a)], logits="none")
+        one = np.stack([m.forward(t).copy() for t in ids[a:a + 64]])
+        m.truncate(a)
+        rows = m.forward_batch(ids[a:a + 64], logits="all").copy()
+        assert (rows.view(np.uint32) == one.view(np.uint32)).all(), a
+        at = a + 64
+    m.close()
